@@ -69,6 +69,13 @@ int kvax_mask_build(const int32_t* q_pos, const int32_t* q_seg, const int32_t* k
                     int skip_pad_tokens, const kvax_mask_desc* masks, int num_masks,
                     void* workspace, size_t workspace_bytes, kvax_stream_t stream);
 
+/* Reorders the sequence axis for balanced causal work under context parallelism (reference
+ * kvax/utils/permutation.py:9-116): src and dst are contiguous [batch, num_chunks, chunk_bytes]
+ * arrays; chunk j of dst is chunk 0, n-1, 1, n-2, ... of src (`reverse`: the inverse).  num_chunks is
+ * even; chunk_bytes and both pointers are multiples of 4; src and dst do not overlap. */
+int kvax_permute_chunks(const void* src, void* dst, int64_t batch, int num_chunks, int64_t chunk_bytes,
+                        int reverse, kvax_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------
  * Flash attention, forward and backward.
  * kvax_fa_fwd replaces the `jt.triton_call` of flash_attention_forward_kernel
@@ -139,7 +146,11 @@ typedef struct kvax_fa_args {
   int32_t dtype;                         /* KVAX_BF16 or KVAX_F16 */
   int32_t flags;                         /* KVAX_FA_* bits */
   float scale;
-  int32_t reserved;
+  /* Backward under context parallelism, all shards in one call: the query axis is `dkdv_shards`
+   * contiguous shards (of whole query blocks) and dkdv_mask is [batch, dkdv_shards, kv blocks] with
+   * shard-local bounds, as kvax_mask_build(num_q_shards) writes it.  0 and 1: unsharded. */
+  int16_t dkdv_shards;
+  int16_t reserved;
 } kvax_fa_args;
 
 /* Workspaces (16-byte aligned device memory, contents undefined on entry, reusable right after the

@@ -53,7 +53,7 @@ class FaArgs(C.Structure):
         ("fwd_query_block", C.c_int32), ("fwd_kv_block", C.c_int32),
         ("bwd_query_block", C.c_int32), ("bwd_kv_block", C.c_int32),
         ("dtype", C.c_int32), ("flags", C.c_int32),
-        ("scale", C.c_float), ("reserved", C.c_int32),
+        ("scale", C.c_float), ("dkdv_shards", C.c_int16), ("reserved", C.c_int16),
     ]
 
 
@@ -86,6 +86,10 @@ def lib() -> C.CDLL:
     l.kvax_mask_build.argtypes = [
         C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int,
         C.POINTER(MaskDesc), C.c_int, C.c_void_p, C.c_size_t, C.c_void_p,
+    ]
+    l.kvax_permute_chunks.restype = C.c_int
+    l.kvax_permute_chunks.argtypes = [
+        C.c_void_p, C.c_void_p, C.c_int64, C.c_int, C.c_int64, C.c_int, C.c_void_p,
     ]
     for name in ("kvax_fa_fwd", "kvax_fa_bwd"):
         if hasattr(l, name):

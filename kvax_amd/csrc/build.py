@@ -17,7 +17,7 @@ ROOT = PKG.parent
 LIB = PKG / "libkvax_amd.so"
 OBJ = CSRC / "build"
 
-SOURCES = ["abi.cpp", "mask_builder.hip", "fa_tiles.hip", "fa_fwd.hip", "fa_bwd.hip"]
+SOURCES = ["abi.cpp", "mask_builder.hip", "fa_tiles.hip", "permute.hip", "fa_fwd.hip", "fa_bwd.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

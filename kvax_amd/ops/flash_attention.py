@@ -10,8 +10,8 @@ of the reference's ``jax.custom_vjp``, :1882-1944).  The device work is two call
 
 Context parallelism: when the attention specs name a mesh axis for the query sequence, the query
 axis is treated as ``cp`` contiguous shards, exactly what ``shard_map`` hands to each device in
-the reference.  This build has one GPU, so the shards are evaluated one after another on it and
-dK/dV are summed over shards (the reference's psum of the replicated operands' cotangents).
+the reference.  This build has one GPU, so the shards share one call on it, in which the dK/dV kernel
+sums over them (the reference's psum of the replicated operands' cotangents).
 """
 from __future__ import annotations
 
@@ -147,9 +147,10 @@ def backward_workspace_bytes(query, key) -> int:
 
 def flash_attention_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, dq_mask, dkdv_mask,
                              out, lse, dout, scale, fwd_params, bwd_params, dkdv_fp32=False,
-                             flags=0, buffers=None):
+                             flags=0, buffers=None, dkdv_shards=1):
     """One device's backward: returns (dq, dk, dv); dq in the dtype of query, dk / dv too unless
-    ``dkdv_fp32`` asks for the kernels' fp32 accumulators (used to sum context shards)."""
+    ``dkdv_fp32`` asks for the kernels' fp32 accumulators (to sum them over devices).  ``dkdv_shards``:
+    the query axis holds that many context shards and ``dkdv_mask`` a row of bounds for each."""
     kv_dtype = torch.float32 if dkdv_fp32 else key.dtype
     if buffers is not None:  # (dq, dk, dv, workspace) reused across calls, e.g. by the benchmark
         dq, dk, dv, ws = buffers
@@ -166,6 +167,7 @@ def flash_attention_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, dq
     a.dq_strides, a.dk_strides, a.dv_strides = _strides3(dq), _strides3(dk), _strides3(dv)
     a.dq_mask, a.dkdv_mask = _mask_ptrs(dq_mask), _mask_ptrs(dkdv_mask)
     a.flags = (_native.KVAX_FA_DKDV_F32 if dkdv_fp32 else 0) | flags
+    a.dkdv_shards = dkdv_shards
     lib = _native.lib()
     if not hasattr(lib, "kvax_fa_bwd"):
         raise _native.KvaxNativeError("libkvax_amd.so was built without kvax_fa_bwd")
@@ -178,20 +180,13 @@ def flash_attention_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, dq
     return dq, dk, dv
 
 
-def _slice_mask(mask, shard: int, cp: int, kv_outer: bool):
-    """The part of a global mask that ``shard_map`` would hand to one context shard."""
-    arrays = mask.flatten() if isinstance(mask, AttentionMask) else tuple(mask)
-    if cp == 1:
-        return tuple(a.contiguous() for a in arrays)
-    if kv_outer:  # [batch, cp, n_kv_blocks] -> [batch, 1, n_kv_blocks]
-        return tuple(a[:, shard:shard + 1].contiguous() for a in arrays)
-    n = arrays[0].shape[-1] // cp  # [batch, 1, n_q_blocks] split along the last axis
-    return tuple(a[..., shard * n:(shard + 1) * n].contiguous() for a in arrays)
+def _contiguous(mask):
+    return tuple(a.contiguous() for a in (mask.flatten() if isinstance(mask, AttentionMask) else mask))
 
 
 class _FlashAttentionFn(torch.autograd.Function):
-    """Counterpart of flash_attention_triton_single_device + defvjp (:1882-1944), applied to
-    every context shard in turn."""
+    """Counterpart of flash_attention_triton_single_device + defvjp (:1882-1944), for all context
+    shards at once."""
 
     @staticmethod
     def forward(ctx, query, key, value, q_pos, q_seg, kv_pos, kv_seg, masks, scale, fwd_params,
@@ -202,19 +197,12 @@ class _FlashAttentionFn(torch.autograd.Function):
         kv_pos, kv_seg = _ids(kv_pos, "kv_positions", (b, sk)), _ids(kv_seg, "kv_segment_ids", (b, sk))
         if sq % cp:
             raise ValueError(f"query length {sq} does not split into {cp} context shards")
-        n = sq // cp
-        if cp > 1 and n % fwd_params.query_block_size:
+        if cp > 1 and sq // cp % fwd_params.query_block_size:
             raise ValueError("context shards must hold whole query blocks")
-        outs, lses = [], []
-        for r in range(cp):
-            sl = slice(r * n, (r + 1) * n)
-            o, l = flash_attention_forward(
-                query[:, sl], key, value, q_pos[:, sl].contiguous(), q_seg[:, sl].contiguous(),
-                kv_pos, kv_seg, _slice_mask(masks[0], r, cp, False), scale, fwd_params, bwd_params)
-            outs.append(o)
-            lses.append(l)
-        out = outs[0] if cp == 1 else torch.cat(outs, dim=1)
-        lse = lses[0] if cp == 1 else torch.cat(lses, dim=2)
+        # A query-outer mask has one entry per query block whatever the sharding: every shard's
+        # queries are in one call.
+        out, lse = flash_attention_forward(query, key, value, q_pos, q_seg, kv_pos, kv_seg,
+                                           _contiguous(masks[0]), scale, fwd_params, bwd_params)
         ctx.save_for_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, out, lse)
         ctx.masks, ctx.scale, ctx.cp = masks, scale, cp
         ctx.fwd_params, ctx.bwd_params = fwd_params, bwd_params
@@ -231,23 +219,10 @@ class _FlashAttentionFn(torch.autograd.Function):
                 or key.shape[1] % bwd.kv_block_size:
             raise ValueError(
                 "backward needs sequence lengths divisible by the backward block sizes")
-        n = query.shape[1] // cp
-        dqs, dk, dv = [], None, None
-        for r in range(cp):
-            sl = slice(r * n, (r + 1) * n)
-            dq_r, dk_r, dv_r = flash_attention_backward(
-                query[:, sl], key, value, q_pos[:, sl].contiguous(), q_seg[:, sl].contiguous(),
-                kv_pos, kv_seg, _slice_mask(masks[1], r, cp, False),
-                _slice_mask(masks[2], r, cp, True), out[:, sl], lse[:, :, sl].contiguous(),
-                dout[:, sl], ctx.scale, ctx.fwd_params, bwd, dkdv_fp32=cp > 1)
-            dqs.append(dq_r)
-            if dk is None:
-                dk, dv = dk_r, dv_r
-            else:
-                dk += dk_r
-                dv += dv_r
-        dq = dqs[0] if cp == 1 else torch.cat(dqs, dim=1)
-        return (dq, dk.to(key.dtype), dv.to(value.dtype)) + (None,) * 9
+        dq, dk, dv = flash_attention_backward(
+            query, key, value, q_pos, q_seg, kv_pos, kv_seg, _contiguous(masks[1]), _contiguous(masks[2]),
+            out, lse, dout, ctx.scale, ctx.fwd_params, bwd, dkdv_shards=cp)
+        return (dq, dk, dv) + (None,) * 9
 
 
 def flash_attention(

@@ -11,6 +11,7 @@ from typing import Sequence
 
 import torch
 
+from kvax_amd import _native
 from kvax_amd.utils.sharding import get_query_context_mesh_axis_size
 from kvax_amd.utils.typing import DeviceArray
 
@@ -28,10 +29,44 @@ def generate_shard_indices(num_shards: int, reverse: bool = False) -> list[int]:
     return inverse
 
 
+def _permute_on_device(x: torch.Tensor, num_shards: int, reverse: bool) -> torch.Tensor:
+    x = x.contiguous()
+    out = torch.empty_like(x)
+    chunk_bytes = x.numel() // (x.shape[0] * num_shards) * x.element_size()
+    with torch.cuda.device(x.device):
+        rc = _native.lib().kvax_permute_chunks(
+            x.data_ptr(), out.data_ptr(), x.shape[0], num_shards, chunk_bytes, int(reverse),
+            torch.cuda.current_stream().cuda_stream)
+    _native.check(rc, "kvax_permute_chunks")
+    return out
+
+
+class _PermuteChunks(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, num_shards, reverse):
+        ctx.num_shards, ctx.reverse = num_shards, reverse
+        return _permute_on_device(x, num_shards, reverse)
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _permute(grad, ctx.num_shards, not ctx.reverse), None, None
+
+
+def _permute(x: torch.Tensor, num_shards: int, reverse: bool) -> torch.Tensor:
+    """One tensor, permuted by the copy kernel; tensors it does not take (on the host, or in pieces that
+    are not a multiple of 4 bytes) by an index."""
+    if x.is_cuda and x.numel() and x.shape[0] <= 65535 and \
+            x.numel() // (x.shape[0] * num_shards) * x.element_size() % 4 == 0:
+        return _PermuteChunks.apply(x, num_shards, reverse)
+    order = generate_shard_indices(num_shards, reverse=reverse)
+    idx = torch.as_tensor(order, device=x.device, dtype=torch.long)
+    chunks = x.reshape(x.shape[0], num_shards, x.shape[1] // num_shards, *x.shape[2:])
+    return chunks.index_select(1, idx).reshape(x.shape)
+
+
 def apply_permutation(
     inputs: Sequence[DeviceArray], num_shards: int, reverse_permutation: bool
 ) -> list[DeviceArray]:
-    order = generate_shard_indices(num_shards, reverse=reverse_permutation)
     outputs = []
     for x in inputs:
         seq = x.shape[1]
@@ -39,9 +74,7 @@ def apply_permutation(
             raise ValueError(
                 f"sequence length {seq} is not divisible by the number of chunks {num_shards}"
             )
-        idx = torch.as_tensor(order, device=x.device, dtype=torch.long)
-        chunks = x.reshape(x.shape[0], num_shards, seq // num_shards, *x.shape[2:])
-        outputs.append(chunks.index_select(1, idx).reshape(x.shape))
+        outputs.append(_permute(x, num_shards, reverse_permutation))
     return outputs
 
 

@@ -4,7 +4,7 @@ The reference wraps every op in ``jax.experimental.shard_map`` over a jax ``Mesh
 (kvax/utils/sharding.py:37-67) and reads the context-parallel axis name and size from the global
 attention specs (sharding.py:70-86).  This build runs on one GPU, so a mesh is only a mapping
 ``axis name -> size`` that tells the host code how many query shards a context-parallel call is
-split into; the shards are then evaluated one after another on the same device.
+split into; the shards then share the device and each call.
 
 Any object with a ``shape`` mapping (a jax ``Mesh`` included) is accepted wherever a mesh is.
 """

@@ -1,0 +1,69 @@
+"""All context shards in one call: the dK/dV kernel's walk over shard-local masks, and the chunk
+permutation kernel."""
+import pytest
+import torch
+
+from kvax_amd import FlashAttentionParamsConfig, Mesh, attention_specs, create_attention_mask
+from kvax_amd.ops.flash_attention import flash_attention_backward, flash_attention_forward
+from kvax_amd.utils.benchmarking import generate_random_segments_lengths, make_random_attention_inputs
+from kvax_amd.utils.permutation import apply_permutation, generate_shard_indices
+
+pytestmark = pytest.mark.gpu
+CP_SPECS = (("data", "context", None, None), ("data", None, None, None))
+
+
+@pytest.mark.parametrize("sq, sk, cp, block, heads, kv_heads, dim, pad, docs", [
+    (96, 128, 3, 32, 2, 2, 64, 0, 1),         # shards of half a query tile: tiles straddle two shards
+    (320, 320, 2, 32, 4, 1, 128, 40, 3),      # a shard that starts inside a tile, padding, several documents
+    (1024, 1024, 8, 64, 4, 2, 128, 700, 2),   # shards that are padding only
+    (512, 700, 4, 128, 2, 1, 256, 0, 4),      # ragged keys, head_dim 256
+])
+def test_shards_in_one_call_equal_shard_by_shard(device, sq, sk, cp, block, heads, kv_heads, dim, pad, docs):
+    data, scale = make_random_attention_inputs(
+        2, sq, sk, heads, kv_heads, dim, dim, seed=sq + cp, num_pad_tokens=pad,
+        list_of_segment_lengths=generate_random_segments_lengths(min(sq, sk), docs), device=device)
+    q, k, v, q_pos, q_seg, kv_pos, kv_seg = data
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(1)).to(q.dtype).to(device)
+    p = FlashAttentionParamsConfig(block, block)
+    mesh = Mesh({"data": 1, "context": cp, "model": 1})
+    with attention_specs(*CP_SPECS):
+        masks = create_attention_mask(q_pos, q_seg, kv_pos, kv_seg, fwd_params=p, bwd_params=p, calc_bwd_mask=True,
+                                      mesh=mesh)
+    out, lse = flash_attention_forward(q, k, v, q_pos, q_seg, kv_pos, kv_seg, masks[0], scale, p, p)
+    got = flash_attention_backward(q, k, v, q_pos, q_seg, kv_pos, kv_seg, masks[1], masks[2], out, lse, dout, scale, p, p,
+                                   dkdv_fp32=True, dkdv_shards=cp)
+    # shard by shard, each with its own slice of everything (what one device of the group computes)
+    n, dqs, dk, dv = sq // cp, [], 0, 0
+    for r in range(cp):
+        sl, nb = slice(r * n, (r + 1) * n), masks[1].lower_bounds.shape[-1] // cp
+        dq_mask = tuple(a[..., r * nb:(r + 1) * nb].contiguous() for a in masks[1].flatten())
+        kv_mask = tuple(a[:, r:r + 1].contiguous() for a in masks[2].flatten())
+        dq_r, dk_r, dv_r = flash_attention_backward(
+            q[:, sl], k, v, q_pos[:, sl].contiguous(), q_seg[:, sl].contiguous(), kv_pos, kv_seg, dq_mask, kv_mask,
+            out[:, sl], lse[:, :, sl].contiguous(), dout[:, sl], scale, p, p, dkdv_fp32=True)
+        dqs.append(dq_r)
+        dk, dv = dk + dk_r, dv + dv_r
+    # the same products in the same precision; sums of fp32 terms in another order, and exponentials
+    # of scores whose sums met other tile boundaries: far inside one unit in the last place of bf16
+    for name, a, b in zip(("dq", "dk", "dv"), got, (torch.cat(dqs, 1), dk, dv)):
+        a, b = a.float(), b.float()
+        assert (a - b).abs().max() <= 2 ** -8 * b.abs().max() and (a - b).norm() <= 1e-3 * b.norm(), name
+    if pad:
+        assert not got[1][:, sk - pad:].any() and not got[2][:, sk - pad:].any()
+
+
+@pytest.mark.parametrize("shape, chunks, dtype", [
+    ((1, 2, 1), 2, torch.int32), ((3, 12, 5), 4, torch.int32), ((2, 16, 3, 8), 16, torch.bfloat16),
+    ((2, 6, 1, 1), 2, torch.bfloat16), ((1, 4096, 2, 64), 8, torch.bfloat16), ((2, 10, 3), 10, torch.float64),
+    ((1, 2, 100003), 2, torch.int32),
+])
+def test_chunk_permutation(device, shape, chunks, dtype):
+    x = torch.arange(torch.Size(shape).numel(), device=device).reshape(shape).to(dtype)
+    order = torch.tensor(generate_shard_indices(chunks), device=device)
+    want = x.reshape(shape[0], chunks, -1)[:, order].reshape(shape)
+    assert torch.equal(apply_permutation([x], chunks, False)[0], want)
+    assert torch.equal(apply_permutation([want], chunks, True)[0], x)
+    if dtype.is_floating_point:
+        leaf, g = x.clone().requires_grad_(True), torch.randn_like(x)
+        apply_permutation([leaf], chunks, False)[0].backward(g)
+        assert torch.equal(leaf.grad, apply_permutation([g], chunks, True)[0])
