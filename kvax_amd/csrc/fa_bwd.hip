@@ -64,6 +64,9 @@ struct BwdParams {
   int32_t* order_ws;           // room for the dK/dV dispatch order and its scratch
   const int32_t* dkdv_order;   // dispatch order of the kv tiles [batch, tiles], or null
   int32_t* dkdv_queue;         // dK/dV kernel: one item counter per XCD, zero at launch
+  int dkdv_parts;              // work-groups that share the steps of a dK/dV work item (see plan_dkdv_parts)
+  int64_t dk_part, dv_part;    // bytes between the partial results of two parts
+  float* parts_ws;             // room for them
   int flags;
   float scale, scale_log2;
   float scale_log2_abs;  // |scale| * log2(e) > 0, used with K negated when the scale is negative
@@ -458,7 +461,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   // batch row and kv head) from the queues (see ItemQueue) until none is left.  The ticket for the
   // next item is drawn when the current one's step loop has ended, so that its latency hides behind
   // the final stores and an item is never held back by a long one.
-  const ItemMap items{p.batch * p.num_kv_heads, p.num_tiles, 1};
+  const ItemMap items{p.batch * p.num_kv_heads, p.num_tiles, p.dkdv_parts};
   ItemQueue work{p.dkdv_queue, p.total_items, (int)(blockIdx.x % 8)};  // thread 0's
   int* next_item = reinterpret_cast<int*>(smem + Smem::kTotal) + 1;
   if (tid == 0) *next_item = work.resolve(work.draw());
@@ -468,8 +471,10 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   int ticket = 0;
   // kv tiles in the computed dispatch order (without one: early tiles first, which see the most
   // queries under a causal mask)
-  int group, rank, member;
+  int group, rank, member;  // member: which part of the item's steps
   if (items.decode(item, group, rank, member)) {
+  char* const dk_out = p.dk + member * p.dk_part;
+  char* const dv_out = p.dv + member * p.dv_part;
   const int kv_head = group % p.num_kv_heads;
   const int b = group / p.num_kv_heads;
   const int entry = p.dkdv_order ? p.dkdv_order[(int64_t)b * p.num_tiles + rank] : rank;
@@ -483,8 +488,8 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     for (int i = tid; i < rows * chunks; i += NW * 64) {
       const int64_t row = k0 + i / chunks;
       const int at = (i % chunks) * 16;
-      *reinterpret_cast<uint4*>(p.dk + ((int64_t)b * p.dk_sb + (int64_t)kv_head * p.dk_sh + row * p.dk_ss) * (row_bytes / D) + at) = make_uint4(0, 0, 0, 0);
-      *reinterpret_cast<uint4*>(p.dv + ((int64_t)b * p.dv_sb + (int64_t)kv_head * p.dv_sh + row * p.dv_ss) * (row_bytes / D) + at) = make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(dk_out + ((int64_t)b * p.dk_sb + (int64_t)kv_head * p.dk_sh + row * p.dk_ss) * (row_bytes / D) + at) = make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(dv_out + ((int64_t)b * p.dv_sb + (int64_t)kv_head * p.dv_sh + row * p.dv_ss) * (row_bytes / D) + at) = make_uint4(0, 0, 0, 0);
     }
   } else {
 
@@ -548,9 +553,13 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     compact_live_tiles<NW, true>(live_bits, words, word0, const_cast<uint32_t*>(live_list), live_count, lane);
   __syncthreads();
   const int n_live = *live_count;
-  const int steps = n_live * p.group * SUB;  // every head of the group walks the same list
+  // every head of the group walks the same list; this part's share of the (head, list entry) pairs
+  const int pairs = n_live * p.group;
+  const int pair_lo = (int)((int64_t)pairs * member / p.dkdv_parts);
+  const int steps = ((int)((int64_t)pairs * (member + 1) / p.dkdv_parts) - pair_lo) * SUB;
 
   if (steps > 0) {
+    const int first_head = pair_lo / n_live, first_li = pair_lo - first_head * n_live;
     // stationary fragments: K (negated when the scale is negative) for the P wave, V for the S wave
     vec8 frag[KSTEPS];
     {
@@ -576,11 +585,11 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
 
     const uint32_t smem_addr = (uint32_t)(uintptr_t)smem;
     const AsyncTileCopy<SR, D, NP> copy_q(p.q_ss * 2, pair, lane), copy_do(p.do_ss * 2, pair, lane);
-    // Step s = (head s / n_live of the group, list entry s % n_live); its Q tile and row data go to
+    // Steps go through the list entries of one head of the group after the other; step s: its Q tile and row data go to
     // slot s % 4 of their rings, its dO tile to slot s % 3.  The issuing side keeps its own cursor
     // (list index, per-head base pointers) and advances it by additions only: divisions and 64-bit
     // multiplies per copy are serial scalar work of the issuing wave.
-    const int head0 = kv_head * p.group;
+    const int head0 = kv_head * p.group + first_head;
     const char* is_q = p.q + ((int64_t)b * p.q_sb + (int64_t)head0 * p.q_sh) * 2;
     const char* is_do = p.dout + ((int64_t)b * p.do_sb + (int64_t)head0 * p.do_sh) * 2;
     // row-data arrays this wave copies (array w of lse, delta, seg, pos for w = pair, pair + NP, ...):
@@ -596,8 +605,8 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
                                 : (const char*)(p.q_pos + (int64_t)b * p.q_len);
       rows_per_head[r] = which < 2 ? (int64_t)p.q_len * 4 : 0;
     }
-    int is_li = 0, is_sub = 0;
-    uint32_t is_entry = live_list[0];
+    int is_li = first_li, is_sub = 0;
+    uint32_t is_entry = live_list[first_li];
     auto issue_next = [&](int q_slot, int do_slot) {
       const int qr0 = (int)(is_entry & 0xffffff) * kTile + is_sub * SR;
       copy_q(is_q, qr0, p.q_len, smem_addr + Smem::kQ + q_slot * Smem::kTileBytes);
@@ -672,8 +681,8 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
       }
     };
 
-    int li = 0, sub = 0;           // list index and sub-step of the current step
-    uint32_t e0 = live_list[0];    // its entry
+    int li = first_li, sub = 0;    // list index and sub-step of the current step
+    uint32_t e0 = live_list[li];   // its entry
     uint32_t ep = 0;               // entry of the previous step
     if (p_wave) {
       issue_next(0, 0);
@@ -813,7 +822,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   {
     // (padding keys, dead: exact zeros, see the dQ kernel's epilogue)
     const float mul = p_wave ? 1.f : p.scale;
-    char* base = p_wave ? p.dv : p.dk;
+    char* base = p_wave ? dv_out : dk_out;
     const int64_t sb = p_wave ? p.dv_sb : p.dk_sb, sh = p_wave ? p.dv_sh : p.dk_sh, ss = p_wave ? p.dv_ss : p.dk_ss;
     constexpr int PC = D < 128 ? D : 128;  // columns per pass
     constexpr int kDtPerPass = PC / 32;
@@ -867,6 +876,67 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   if (tid == 0) *next_item = work.resolve(ticket);
   __syncthreads();
   }  // items of this XCD
+}
+
+// Adds the parts' fp32 dK and dV in the order of the parts and writes them in the gradients' type and
+// strides.  A copy, bound by memory: 16 bytes per thread and part, four parts in flight.
+struct DkdvSumParams {
+  const float* parts;  // [part][dK, dV][batch, kv_len, kv heads, D]
+  char* dst[2];        // dK, dV
+  int64_t sb[2], ss[2], sh[2];
+  int64_t total;       // 4-element pieces of one tensor
+  int num_parts, kv_len, num_kv_heads;
+  int f32;
+};
+
+template <class Tr, int D>
+__global__ __launch_bounds__(256) void dkdv_sum_kernel(const DkdvSumParams p) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int which = blockIdx.y;
+  if (i >= p.total) return;
+  const float4* src = reinterpret_cast<const float4*>(p.parts) + which * p.total + i;
+  float4 sum = src[0];
+#pragma unroll 4
+  for (int part = 1; part < p.num_parts; part++) {
+    const float4 v = src[2 * p.total * part];
+    sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
+  }
+  constexpr int kPieces = D / 4;
+  int64_t row = i / kPieces;
+  const int d = (int)(i % kPieces) * 4;
+  const int head = (int)(row % p.num_kv_heads);
+  row /= p.num_kv_heads;
+  const int64_t at = row / p.kv_len * p.sb[which] + row % p.kv_len * p.ss[which] + head * p.sh[which] + d;
+  if (p.f32)
+    *reinterpret_cast<float4*>(p.dst[which] + at * 4) = sum;
+  else
+    *reinterpret_cast<uint2*>(p.dst[which] + at * 2) = make_uint2(Tr::pack2(sum.x, sum.y), Tr::pack2(sum.z, sum.w));
+}
+
+// How many work-groups share the steps of a dK/dV work item.  A launch with fewer items than compute
+// units leaves the others idle, and one with few more ends on its longest items (under a causal mask
+// the first keys see twice the mean number of queries).  An item costs about 20 us whatever its steps
+// (ids, list, first tiles, results), a step 1.2 to 1.8 us, and every part is written and read once
+// more: one round of parts on the compute units where each has at least 8 steps, two, which even out
+// the items' lengths, where it has 24, three where it has 128.  Steps are counted as if every query
+// tile were live.  dK/dV kernel and sum, us, items x steps without parts -> with (number of parts):
+//   32 x 128 (2k, heads 8/2 of 64)       126 -> 44 (8), 53 (16)
+//   64 x 64 (1k, heads 32/8 of 128)      127 -> 60 (4), 83 (8)
+//   128 x 128 (2k, heads 32/8)           178 -> 112 (2), 102 (4), 108 (6), 140 (8)
+//   192 x 192 (3k, documents of 1k)      180 -> 121 (2), 149 (4)
+//   128 x 512 (8k, heads 8/2, the same)  323 -> 184 (2), 117 (4), 139 (6), 160 (8)
+//   256 x 256 (4k, heads 32/8)           450 -> 317 (2), 348 (3)
+//   384 x 384 (6k)                       741 -> 683 (2)
+//   128 x 1024 (16k, heads 4/1)          622 -> 333 (2), 192 (4), 172 (6), 193 (8)
+//   256 x 2048 (32k, heads 4/1)          1179 -> 631 (2), 452 (3)
+// A function of the shapes, so that the workspace can be sized up front (at most 768 parts of 128 rows).
+int plan_dkdv_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int head_dim) {
+  if (batch <= 0 || q_len <= 0 || kv_len <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return 1;
+  const int64_t items = (int64_t)batch * num_kv_heads * cdiv(kv_len, head_dim > 128 ? 64 : 128);
+  const int64_t steps = (int64_t)cdiv(q_len, kTile) * (num_heads / num_kv_heads);
+  const int64_t one_round = min(kNumCus / items, steps / 8), two_rounds = min(2 * kNumCus / items, steps / 24),
+                three_rounds = min(3 * kNumCus / items, steps / 128);
+  return (int)max(min(max(max(one_round, two_rounds), three_rounds), (int64_t)16), (int64_t)1);
 }
 
 template <class K>
@@ -954,10 +1024,28 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
     const int smem = DkdvSmem<D>::kTotal + live_tiles_bytes(NW, p.list_tiles);
     if (int rc = reserve_lds(kernel, smem, kLdsLimit, &done, "the dK/dV kernel")) return rc;
     p.num_tiles = cdiv(p.kv_len, Cfg::kKvRows);
-    p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, 1}.grid();
+    p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, p.dkdv_parts}.grid();
+    DkdvSumParams sum{};
+    if (p.dkdv_parts > 1) {  // the kernel leaves fp32 parts, dkdv_sum_kernel adds them
+      sum.parts = p.parts_ws;
+      sum.dst[0] = p.dk, sum.sb[0] = p.dk_sb, sum.ss[0] = p.dk_ss, sum.sh[0] = p.dk_sh;
+      sum.dst[1] = p.dv, sum.sb[1] = p.dv_sb, sum.ss[1] = p.dv_ss, sum.sh[1] = p.dv_sh;
+      sum.total = (int64_t)p.batch * p.kv_len * p.num_kv_heads * D / 4;
+      sum.num_parts = p.dkdv_parts, sum.kv_len = p.kv_len, sum.num_kv_heads = p.num_kv_heads;
+      sum.f32 = p.dkdv_f32;
+      p.dk = (char*)p.parts_ws, p.dv = p.dk + sum.total * 16;
+      p.dk_part = p.dv_part = sum.total * 32;
+      p.dk_sh = p.dv_sh = D, p.dk_ss = p.dv_ss = (int64_t)p.num_kv_heads * D;
+      p.dk_sb = p.dv_sb = p.dk_ss * p.kv_len;
+      p.dkdv_f32 = 1;
+    }
     p.dkdv_queue = tile_order_counters(p.order_ws, p.batch, p.num_tiles) + p.batch;
     hipLaunchKernelGGL(kernel, dim3(min(p.total_items, kNumCus)), dim3(NW * 64), smem, stream, p);
     if (int rc = check_launch("fa_bwd_dkdv_kernel")) return rc;
+    if (p.dkdv_parts > 1) {
+      hipLaunchKernelGGL((dkdv_sum_kernel<Tr, D>), dim3((unsigned)((sum.total + 255) / 256), 2), dim3(256), 0, stream, sum);
+      if (int rc = check_launch("dkdv_sum_kernel")) return rc;
+    }
   }
   return KVAX_OK;
 }
@@ -971,12 +1059,23 @@ static size_t delta_bytes(const kvax_fa_args* a) {
   return ((size_t)a->batch * a->num_heads * a->q_len * sizeof(float) + 15) / 16 * 16;
 }
 
-extern "C" size_t kvax_fa_bwd_workspace_bytes(const kvax_fa_args* a) {
-  if (!a || a->batch < 0 || a->q_len < 0 || a->kv_len < 0 || a->num_heads < 0) return 0;
-  // delta [batch, heads, q_len] fp32, the tile summaries of the kv and query sequences, and the
-  // dispatch order of the dK/dV work items
+// Start of the dK/dV parts in the workspace: behind delta [batch, heads, q_len] fp32, the tile summaries
+// of the kv and query sequences, and the dispatch order of the dK/dV work items.
+static size_t parts_offset(const kvax_fa_args* a) {
   return delta_bytes(a) + tile_summary_bytes(a->batch, a->kv_len) + tile_summary_bytes(a->batch, a->q_len) +
          tile_order_bytes(a->batch, cdiv(a->kv_len, a->head_dim > 128 ? 64 : 128));
+}
+static int dkdv_parts(const kvax_fa_args* a) {
+  return plan_dkdv_parts(a->batch, a->q_len, a->kv_len, a->num_heads, a->num_kv_heads, a->head_dim);
+}
+static size_t dkdv_parts_bytes(const kvax_fa_args* a) {
+  const int parts = dkdv_parts(a);
+  return parts == 1 ? 0 : (size_t)parts * 2 * a->batch * a->kv_len * a->num_kv_heads * a->head_dim * sizeof(float);
+}
+
+extern "C" size_t kvax_fa_bwd_workspace_bytes(const kvax_fa_args* a) {
+  if (!a || a->batch < 0 || a->q_len < 0 || a->kv_len < 0 || a->num_heads < 0) return 0;
+  return parts_offset(a) + dkdv_parts_bytes(a);
 }
 
 extern "C" int kvax_fa_bwd(const kvax_fa_args* a, void* workspace, size_t workspace_bytes,
@@ -1038,6 +1137,8 @@ extern "C" int kvax_fa_bwd(const kvax_fa_args* a, void* workspace, size_t worksp
   p.bq = a->bwd_query_block, p.bk = a->bwd_kv_block;
   p.n_dq_blocks = cdiv(a->q_len, a->bwd_kv_block);
   p.n_kv_blocks = cdiv(a->kv_len, a->bwd_kv_block);
+  p.dkdv_parts = dkdv_parts(a);
+  p.parts_ws = (float*)((char*)workspace + parts_offset(a));
   p.num_shards = shards;
   p.shard_rows = a->q_len / shards;
   p.dkdv_f32 = (a->flags & KVAX_FA_DKDV_F32) != 0;

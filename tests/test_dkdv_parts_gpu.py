@@ -1,0 +1,45 @@
+"""dK/dV of launches with few work items, where several work-groups share the steps of an item and their
+fp32 results are added: against the dense CPU oracle, at uneven shares, shares without any step, ragged
+lengths, padding, strided outputs' types and at the largest number of parts."""
+import numpy as np
+import pytest
+import torch
+
+from kvax_amd import create_attention_mask
+from kvax_amd.ops.flash_attention import flash_attention_backward, flash_attention_forward
+from kvax_amd.utils import FlashAttentionParamsConfig, attention_specs
+from kvax_amd.utils.benchmarking import generate_random_segments_lengths, make_random_attention_inputs
+from oracle import attention_oracle as ao
+from tests.tolerances import OPERAND_ROUNDING, check_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b, sq, sk, hq, hkv, d, pad, docs, fp32", [
+    (1, 512, 512, 8, 1, 64, 0, 1, False),     # 8 parts of 8 steps
+    (1, 2048, 2048, 8, 1, 128, 100, 1, True),  # 16 parts, one causal document: the last keys have a few steps only
+    (2, 1000, 1000, 6, 2, 128, 77, 9, True),  # ragged; 6 parts of 48 (head, tile) pairs, documents leave most without a step
+    (1, 777, 300, 12, 4, 64, 0, 1, False),    # more queries than keys, uneven shares
+    (3, 640, 640, 4, 1, 256, 65, 3, True),
+    (1, 512, 512, 16, 16, 64, 0, 1, False),   # too few steps to share: one part
+    (1, 65, 129, 32, 1, 128, 0, 1, True),     # as few tiles as possible
+])
+def test_shared_items_match_dense_oracle(device, b, sq, sk, hq, hkv, d, pad, docs, fp32):
+    data, scale = make_random_attention_inputs(
+        b, sq, sk, hq, hkv, d, d, seed=sq + hq + d, num_pad_tokens=pad, start_query_position=max(sk - sq, 0),
+        list_of_segment_lengths=generate_random_segments_lengths(min(sq, sk), docs), device=device)
+    q, k, v, *ids = data
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(2)).to(q.dtype).to(device)
+    p = FlashAttentionParamsConfig(64, 64)
+    spec = ("data", None, "model", None)
+    with attention_specs(spec, spec):
+        masks = create_attention_mask(*ids, fwd_params=p, bwd_params=p, calc_bwd_mask=True)
+    out, lse = flash_attention_forward(q, k, v, *ids, masks[0], scale, p, p)
+    _, dk, dv = flash_attention_backward(q, k, v, *ids, masks[1], masks[2], out, lse, dout, scale, p, p, dkdv_fp32=fp32)
+    host = [x.cpu().numpy() for x in ids]
+    refs = ao.attention_backward(*(x.float().cpu().numpy() for x in (q, k, v)), *host, scale,
+                                 dout.float().cpu().numpy(), dtype=np.float64)
+    for name, got, ref in (("dk", dk, refs[1]), ("dv", dv, refs[2])):
+        # P and dS enter the sums rounded to 16 bits, whatever the number of heads that share a key
+        check_close(name, got, ref, rel=OPERAND_ROUNDING)
+        assert not got[torch.from_numpy(host[3] == -1)].any(), "padding rows must be zero"
