@@ -455,9 +455,11 @@ struct AsyncTileCopy {
     static_assert(kPerWave % 2 == 0, "a wave's copies must split over the two halves of a tile");
     part<HF * (kPerWave / 2), (HF + 1) * (kPerWave / 2)>(gbase, row0, limit, tile_addr);
   }
-  // row0 < limit
+  // row0 >= limit (a tile of which nothing is left, e.g. the second half of a query tile whose first half
+  // holds the last rows): every row is row limit - 1.
   template <int J0, int J1>
   __device__ __forceinline__ void part(const char* gbase, int row0, int limit, uint32_t tile_addr) const {
+    row0 = min(row0, limit - 1);
     const char* tile_base = gbase + (int64_t)row0 * stride;
     if (row0 + ROWS <= limit) {  // whole tile in range (uniform): scalar bases + fixed lane offsets
       const uint32_t lds = tile_addr + wave_u * 1024;

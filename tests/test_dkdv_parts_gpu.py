@@ -23,6 +23,8 @@ pytestmark = pytest.mark.gpu
     (3, 640, 640, 4, 1, 256, 65, 3, True),
     (1, 512, 512, 16, 16, 64, 0, 1, False),   # too few steps to share: one part
     (1, 65, 129, 32, 1, 128, 0, 1, True),     # as few tiles as possible
+    (1, 129, 65, 4, 4, 256, 0, 1, False),     # head_dim 256 takes half tiles: the second half of the last one holds no row
+    (2, 96, 96, 4, 2, 256, 0, 2, False),
 ])
 def test_shared_items_match_dense_oracle(device, b, sq, sk, hq, hkv, d, pad, docs, fp32):
     data, scale = make_random_attention_inputs(
