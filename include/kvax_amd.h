@@ -86,7 +86,7 @@ int kvax_permute_chunks(const void* src, void* dst, int64_t batch, int num_chunk
  * query heads of a group (:1855-1868).
  *
  * Tensors are consumed in the public [batch, seq, heads, head_dim] layout through element
- * strides {batch, seq, head}; the head_dim axis must be contiguous and head_dim is 64, 128 or 256
+ * strides {batch, seq, head}; the head_dim axis must be contiguous and head_dim is 64, 128, 192 or 256
  * (the reference's other sizes, :1397-1403, are zero-padded to these by the caller).  Sequence lengths need not
  * be multiples of the block sizes: tails are handled inside the kernels.  The reference's
  * assume_sequential_positions mode (causal test on token indices plus a per-shard offset,
@@ -150,7 +150,7 @@ typedef struct kvax_fa_args {
    * contiguous shards (of whole query blocks) and dkdv_mask is [batch, dkdv_shards, kv blocks] with
    * shard-local bounds, as kvax_mask_build(num_q_shards) writes it.  0 and 1: unsharded. */
   int16_t dkdv_shards;
-  int16_t reserved;
+  int16_t v_head_dim;  /* head_dim of v, out, dout and dv; 0: head_dim */
 } kvax_fa_args;
 
 /* Workspaces (16-byte aligned device memory, contents undefined on entry, reusable right after the

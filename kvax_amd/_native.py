@@ -53,7 +53,7 @@ class FaArgs(C.Structure):
         ("fwd_query_block", C.c_int32), ("fwd_kv_block", C.c_int32),
         ("bwd_query_block", C.c_int32), ("bwd_kv_block", C.c_int32),
         ("dtype", C.c_int32), ("flags", C.c_int32),
-        ("scale", C.c_float), ("dkdv_shards", C.c_int16), ("reserved", C.c_int16),
+        ("scale", C.c_float), ("dkdv_shards", C.c_int16), ("v_head_dim", C.c_int16),
     ]
 
 

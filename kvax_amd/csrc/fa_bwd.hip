@@ -101,22 +101,26 @@ __device__ __forceinline__ Range merged_range(const int32_t* const mask[4], int6
 // dQ: one work-group = NW wavefronts x 32 query rows of one (batch, head); streams the live K/V
 // tiles through a ring of LDS stages filled by asynchronous copies.
 // ---------------------------------------------------------------------------------------------
-template <int D, int STAGES>
+template <int D, int DV, int STAGES>
 struct DqSmem {
-  static constexpr int kTileBytes = kTile * D * 2;  // swizzled, unpadded
-  static constexpr int kStage = 2 * kTileBytes + 2 * kTile * 4;
+  static constexpr int kTileBytes = kTile * D * 2;  // K tile; swizzled, unpadded
+  static constexpr int kIds = kTileBytes + kTile * DV * 2;  // behind the V tile
+  static constexpr int kStage = kIds + 2 * kTile * 4;
   static constexpr int kTotal = STAGES * kStage;
 };
 
-template <class Tr, int D, int NW, int WPS, int STAGES>
+template <class Tr, int D, int DV, int NW, int WPS, int STAGES>
 __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams p) {
   using vec8 = typename Tr::vec8;
-  using Smem = DqSmem<D, STAGES>;
+  using Smem = DqSmem<D, DV, STAGES>;
   constexpr int TQ = NW * 32;
-  constexpr int KSTEPS = D / 16;
+  constexpr int KSTEPS = D / 16, VSTEPS = DV / 16;  // contraction steps of S^T = K Q^T and dP^T = V dO^T
   constexpr int DT = D / 32;
-  constexpr int RB = D * 2;
-  constexpr int kCopies = 2 * async_tile_copies_per_wave<kTile, D, NW>() + 1;
+  constexpr int RB = D * 2, RBV = DV * 2;
+  // operand address registers (see kNatRegs): at one wavefront per SIMD there is room for one per step
+  constexpr int kNat = WPS == 1 ? KSTEPS : kNatRegs<D>, kNatV = WPS == 1 ? VSTEPS : kNatRegs<DV>;
+  constexpr int kTr = WPS == 1 ? DT : kTrRegs<D>;
+  constexpr int kCopies = async_tile_copies_per_wave<kTile, D, NW>() + async_tile_copies_per_wave<kTile, DV, NW>() + 1;
   static_assert(STAGES == 2 || STAGES == 3, "the loop below keeps STAGES - 1 tiles in flight");
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -176,17 +180,17 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
   // step, i.e. half of its row; with the same half of O they give delta = rowsum(O * dO)
   // (reference attn_bwd_preprocess, flash_attention_triton.py:373-410), which is also written out
   // for the dK/dV kernel.
-  uint4 draw[KSTEPS];
+  uint4 draw[VSTEPS];
   // Q fragments (B operand of S^T = K Q^T), requested with dO and O so that their latency does not
   // follow that of the live-tile bookkeeping below
-  uint4 qraw[KSTEPS], oraw[KSTEPS];
+  uint4 qraw[KSTEPS], oraw[VSTEPS];
   {
     // rows beyond the sequence read row 0 and are zeroed afterwards: no load sits behind a branch
     const char* qr = p.q + ((int64_t)b * p.q_sb + (int64_t)head * p.q_sh + (int64_t)qi * p.q_ss) * 2;
     const char* dr = p.dout + ((int64_t)b * p.do_sb + (int64_t)head * p.do_sh + (int64_t)qi * p.do_ss) * 2;
     const char* orow = p.out + ((int64_t)b * p.o_sb + (int64_t)head * p.o_sh + (int64_t)qi * p.o_ss) * 2;
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) {
+    for (int ks = 0; ks < VSTEPS; ks++) {
       draw[ks] = *reinterpret_cast<const uint4*>(dr + (16 * ks + 8 * h) * 2);
       oraw[ks] = *reinterpret_cast<const uint4*>(orow + (16 * ks + 8 * h) * 2);
     }
@@ -200,8 +204,11 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
   float delta_q = 0.f;
   {
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) {
-      if (!in) draw[ks] = oraw[ks] = qraw[ks] = make_uint4(0, 0, 0, 0);
+    for (int ks = 0; ks < KSTEPS; ks++)
+      if (!in) qraw[ks] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int ks = 0; ks < VSTEPS; ks++) {
+      if (!in) draw[ks] = oraw[ks] = make_uint4(0, 0, 0, 0);
       const uint4 o4 = oraw[ks];
       const uint32_t ow[4] = {o4.x, o4.y, o4.z, o4.w}, gw[4] = {draw[ks].x, draw[ks].y, draw[ks].z, draw[ks].w};
 #pragma unroll
@@ -246,30 +253,32 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
     for (int i = 0; i < 16; i++) dq[dt][i] = 0.f;
 
   if (n_live > 0) {
-    vec8 qf[KSTEPS], dof[KSTEPS];
+    vec8 qf[KSTEPS], dof[VSTEPS];
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) {
-      qf[ks] = __builtin_bit_cast(vec8, qraw[ks]);
-      dof[ks] = __builtin_bit_cast(vec8, draw[ks]);
-    }
-    int nat_off[KSTEPS], tr_off[DT][2];
+    for (int ks = 0; ks < KSTEPS; ks++) qf[ks] = __builtin_bit_cast(vec8, qraw[ks]);
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) nat_off[ks] = nat_offset<D>(c, ks, h);
+    for (int ks = 0; ks < VSTEPS; ks++) dof[ks] = __builtin_bit_cast(vec8, draw[ks]);
+    int nat_off[kNat], nat_off_v[kNatV], tr_off[kTr][2];
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++) {
+    for (int ks = 0; ks < kNat; ks++) nat_off[ks] = nat_offset<D>(c, ks, h);
+#pragma unroll
+    for (int ks = 0; ks < kNatV; ks++) nat_off_v[ks] = nat_offset<DV>(c, ks, h);
+#pragma unroll
+    for (int dt = 0; dt < kTr; dt++) {
       tr_off[dt][0] = tr_offset<D>(lane, dt, 0);
       tr_off[dt][1] = tr_offset<D>(lane, dt, 1);
     }
 
     const uint32_t smem_addr = (uint32_t)(uintptr_t)smem;
     const int32_t* id_src = (wave & 1) ? kv_pos : kv_seg;
-    const AsyncTileCopy<kTile, D, NW> copy_k(p.k_ss * 2, wave, lane), copy_v(p.v_ss * 2, wave, lane);
+    const AsyncTileCopy<kTile, D, NW> copy_k(p.k_ss * 2, wave, lane);
+    const AsyncTileCopy<kTile, DV, NW> copy_v(p.v_ss * 2, wave, lane);
     auto issue = [&](int tile, int stage) {
       const uint32_t base = smem_addr + stage * Smem::kStage;
       copy_k(kbase, tile * kTile, p.kv_len, base);
       copy_v(vbase, tile * kTile, p.kv_len, base + Smem::kTileBytes);
       async_copy_b32(id_src + min(tile * kTile + lane, p.kv_len - 1),
-                     __builtin_amdgcn_readfirstlane(base + 2 * Smem::kTileBytes + (wave & 1) * (kTile * 4)));
+                     __builtin_amdgcn_readfirstlane(base + Smem::kIds + (wave & 1) * (kTile * 4)));
     };
 
     uint32_t e0 = live_list[0];
@@ -294,7 +303,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
         const int kv0 = t * kTile;
         const char* ktile = smem + stage * Smem::kStage;
         const char* vtile = ktile + Smem::kTileBytes;
-        const int32_t* ids = reinterpret_cast<const int32_t*>(ktile + 2 * Smem::kTileBytes);
+        const int32_t* ids = reinterpret_cast<const int32_t*>(ktile + Smem::kIds);
         const bool full = t >= tf_lo && t < tf_hi;
 
 #pragma unroll 1
@@ -305,23 +314,31 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
           for (int i2 = 0; i2 < 16; i2++) s[i2] = 0.f, dp[i2] = 0.f;
 #pragma unroll
           for (int ks = 0; ks < KSTEPS; ks++) {
-            const vec8 ka = *reinterpret_cast<const vec8*>(ktile + 32 * kt * RB + nat_off[ks]);
-            const vec8 va = *reinterpret_cast<const vec8*>(vtile + 32 * kt * RB + nat_off[ks]);
+            const vec8 ka = *reinterpret_cast<const vec8*>(ktile + 32 * kt * RB + nat_off[ks % kNat] + ks / kNat * kGroupBytes<D>);
             s = Tr::mfma(ka, qf[ks], s);
-            dp = Tr::mfma(va, dof[ks], dp);
+            if (ks < VSTEPS) {
+              const vec8 va = *reinterpret_cast<const vec8*>(vtile + 32 * kt * RBV + nat_off_v[ks % kNatV] + ks / kNatV * kGroupBytes<DV>);
+              dp = Tr::mfma(va, dof[ks], dp);
+            }
           }
           __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-          for (int i2 = 0; i2 < 2 * KSTEPS - 4; i2++) {
+          for (int i2 = 0; i2 < KSTEPS + VSTEPS - 4; i2++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
           }
           __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
           // K^T operands of this block's dQ update, requested before the element-wise work
+          // (with two wavefronts per SIMD above head_dim 128 there are no registers to do that in)
+          constexpr bool kLean = WPS == 2 && D > 128;
           vec8 ta[DT];
+          auto read_kt = [&](int dt, int row0) {
+            return tr_read_a_swz<Tr>(ktile + row0 * RB + dt / kTr * kGroupBytes<D>, tr_off[dt % kTr][0], tr_off[dt % kTr][1]);
+          };
+          if (!kLean) {
 #pragma unroll
-          for (int dt = 0; dt < DT; dt++)
-            ta[dt] = tr_read_a_swz<Tr>(ktile + 32 * kt * RB, tr_off[dt][0], tr_off[dt][1]);
+            for (int dt = 0; dt < DT; dt++) ta[dt] = read_kt(dt, 32 * kt);
+          }
 #pragma unroll
           for (int i2 = 0; i2 < 16; i2++) s[i2] = fast_exp2(__builtin_fmaf(s[i2], p.scale_log2, -lse_q));
           if (!full)
@@ -333,11 +350,16 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
           for (int st = 0; st < 2; st++) {
             const vec8 dsb = pack8<Tr>(s[8 * st + 0], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3],
                                        s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]);
+            if (kLean) {
+#pragma unroll
+              for (int dt = 0; dt < DT; dt++) dq[dt] = Tr::mfma(read_kt(dt, 32 * kt + 16 * st), dsb, dq[dt]);
+              continue;
+            }
             vec8 tb[DT];  // second half's operands, requested before the first half's MFMAs
             if (st == 0) {
 #pragma unroll
               for (int dt = 0; dt < DT; dt++)
-                tb[dt] = tr_read_a_swz<Tr>(ktile + (32 * kt + 16) * RB, tr_off[dt][0], tr_off[dt][1]);
+                tb[dt] = read_kt(dt, 32 * kt + 16);
             }
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) dq[dt] = Tr::mfma(ta[dt], dsb, dq[dt]);
@@ -362,26 +384,33 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
     // swizzled by the row index against bank conflicts.
     const bool dead = col_width == 0;
     __syncthreads();  // every wavefront has read its last tile
-    constexpr int kRowBytes = D * 2, kChunks = kRowBytes / 16, kRowsPerStore = 64 / kChunks;
+    constexpr int PC = NW * 32 * D * 2 <= Smem::kTotal ? D : 64;  // columns per pass
+    static_assert(NW * 32 * PC * 2 <= Smem::kTotal, "a wavefront's part of the tile space");
+    constexpr int kRowBytes = PC * 2, kChunks = kRowBytes / 16;
+    constexpr int kSwz = kChunks % 16 == 0 ? kChunks - 1 : 7;  // chunks are permuted within a power of two of them
     char* stage = smem + wave * (32 * kRowBytes);
     char* mine = stage + c * kRowBytes;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; g4++) {
-        uint2 u;
-        u.x = Tr::pack2(dq[dt][4 * g4 + 0] * p.scale, dq[dt][4 * g4 + 1] * p.scale);
-        u.y = Tr::pack2(dq[dt][4 * g4 + 2] * p.scale, dq[dt][4 * g4 + 3] * p.scale);
-        if (dead) u = make_uint2(0, 0);
-        *reinterpret_cast<uint2*>(mine + (((4 * dt + g4) ^ (c & (kChunks - 1))) * 16) + 8 * h) = u;
-      }
     char* dq0 = p.dq + ((int64_t)b * p.dq_sb + (int64_t)head * p.dq_sh) * 2;
 #pragma unroll
-    for (int r0 = 0; r0 < 32; r0 += kRowsPerStore) {
-      const int row = r0 + lane / kChunks, chunk = lane % kChunks;
-      const uint4 v = *reinterpret_cast<const uint4*>(stage + row * kRowBytes + ((chunk ^ (row & (kChunks - 1))) * 16));
-      const int qr = q0 + wave * 32 + row;
-      if (qr < p.q_len) *reinterpret_cast<uint4*>(dq0 + (int64_t)qr * p.dq_ss * 2 + chunk * 16) = v;
+    for (int pass = 0; pass < D / PC; pass++) {
+#pragma unroll
+      for (int dt = 0; dt < PC / 32; dt++)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4++) {
+          const f32x16& a = dq[pass * (PC / 32) + dt];
+          uint2 u;
+          u.x = Tr::pack2(a[4 * g4 + 0] * p.scale, a[4 * g4 + 1] * p.scale);
+          u.y = Tr::pack2(a[4 * g4 + 2] * p.scale, a[4 * g4 + 3] * p.scale);
+          if (dead) u = make_uint2(0, 0);
+          *reinterpret_cast<uint2*>(mine + (((4 * dt + g4) ^ (c & kSwz)) * 16) + 8 * h) = u;
+        }
+#pragma unroll
+      for (int i = 0; i < 32 * kChunks; i += 64) {
+        const int row = (i + lane) / kChunks, chunk = (i + lane) % kChunks;
+        const uint4 v = *reinterpret_cast<const uint4*>(stage + row * kRowBytes + ((chunk ^ (row & kSwz)) * 16));
+        const int qr = q0 + wave * 32 + row;
+        if (qr < p.q_len) *reinterpret_cast<uint4*>(dq0 + (int64_t)qr * p.dq_ss * 2 + pass * kRowBytes + chunk * 16) = v;
+      }
     }
   }
 }
@@ -398,32 +427,36 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
 // work while the other has MFMAs.  The work-group streams the live Q / dO tiles of every query
 // head of the group; Q tiles stay one step longer than dO tiles, hence separate rings.
 // ---------------------------------------------------------------------------------------------
-// Shape of a dK/dV work-group per head_dim.  Up to 128 it is 8 wavefronts (4 role pairs, 128 kv
-// rows) at two per SIMD, stepping through 64-row query tiles.  At 256 a wavefront's fragments and
-// accumulators need more than half a SIMD's registers, so it is 4 wavefronts (2 pairs, 64 kv rows) at
-// one per SIMD, and the Q / dO rings only fit in LDS with 32-row steps: a 64-row tile of the live
-// list is then taken as two steps.
+// Shape of a dK/dV work-group per head_dim.  Up to 192 it is 8 wavefronts (4 role pairs, 128 kv rows) at
+// two per SIMD, stepping through 64-row query tiles up to 128.  Above, the Q / dO rings and the scores of
+// a step only fit beside the accumulators with 32-row steps: a 64-row tile of the live list is then taken
+// as two steps.  At 256 a wavefront's fragments and accumulators need more than half a SIMD's registers,
+// so it is 4 wavefronts (2 pairs, 64 kv rows) at one per SIMD.  (Eight at 256 spill 8 registers in the
+// step: 16k tokens, heads 16/4 3.56 against 2.04 ms; four at 192 with 128 for the values, 2 x 4k tokens,
+// 16 heads: 380 against 244 us.)
 template <int D>
 struct DkdvCfg {
-  static constexpr int kPairs = D > 128 ? 2 : 4;
+  static constexpr int kPairs = D > 192 ? 2 : 4;
   static constexpr int kStepRows = D > 128 ? 32 : 64;  // query rows per step (and LDS stage)
-  static constexpr int kWps = D > 128 ? 1 : 2;         // wavefronts per SIMD
+  static constexpr int kWps = kPairs == 2 ? 1 : 2;     // wavefronts per SIMD
   static constexpr int kWaves = 2 * kPairs;
   static constexpr int kKvRows = 32 * kPairs;          // kv rows per work-group
   static constexpr int kUnits = kStepRows / 32;        // 32-row MFMA units per step
   static constexpr int kSub = kTile / kStepRows;       // steps per 64-row tile of the live list
 };
+inline int dkdv_kv_rows(int head_dim) { return head_dim > 192 ? 64 : 128; }
 
-template <int D>
+template <int D, int DV>
 struct DkdvSmem {
   using Cfg = DkdvCfg<D>;
-  static constexpr int kTileBytes = Cfg::kStepRows * D * 2;  // swizzled, unpadded
+  static constexpr int kQTileBytes = Cfg::kStepRows * D * 2;  // swizzled, unpadded
+  static constexpr int kDoTileBytes = Cfg::kStepRows * DV * 2;
   // lse, delta, seg, pos: 64 entries each whatever the step size (a wave-wide copy brings 64)
   static constexpr int kRowData = 4 * kTile * 4;
   static constexpr int kQStages = 4, kDoStages = 3;
   static constexpr int kQ = 0;
-  static constexpr int kDo = kQ + kQStages * kTileBytes;
-  static constexpr int kRows = kDo + kDoStages * kTileBytes;
+  static constexpr int kDo = kQ + kQStages * kQTileBytes;
+  static constexpr int kRows = kDo + kDoStages * kDoTileBytes;
   static constexpr int kExchange = kRows + kQStages * kRowData;
   // per pair two slots of P (one kStepRows x 32 tile, 16 bits per element): written for step s while
   // the slot of step s - 1 is read
@@ -431,10 +464,10 @@ struct DkdvSmem {
   static constexpr int kTotal = kExchange + Cfg::kPairs * 2 * kSlotBytes;
 };
 
-template <class Tr, int D>
+template <class Tr, int D, int DV>
 __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_bwd_dkdv_kernel(const BwdParams p) {
   using vec8 = typename Tr::vec8;
-  using Smem = DkdvSmem<D>;
+  using Smem = DkdvSmem<D, DV>;
   using Cfg = DkdvCfg<D>;
   constexpr int NW = Cfg::kWaves;
   constexpr int NP = Cfg::kPairs;
@@ -442,13 +475,14 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   constexpr int SR = Cfg::kStepRows;
   constexpr int UNITS = Cfg::kUnits;
   constexpr int SUB = Cfg::kSub;
-  constexpr int KSTEPS = D / 16;
-  constexpr int DT = D / 32;
-  constexpr int RB = D * 2;
+  static_assert(DV <= D, "the arrays below are sized by the larger head_dim");
+  constexpr int KSTEPS = D / 16, VSTEPS = DV / 16;  // contraction steps of S = Q K^T and dP = dO V^T
+  constexpr int DT = D / 32, DTV = DV / 32;         // 32-row tiles of dK^T and dV^T
+  constexpr int RB = D * 2, RBV = DV * 2;
   // only the P waves issue tile copies: they are the ones with slack before the barrier.  Each
   // also copies its share of the four row-data arrays.
   constexpr int kRowCopies = 4 / NP;
-  constexpr int kCopies = 2 * async_tile_copies_per_wave<SR, D, NP>() + kRowCopies;
+  constexpr int kCopies = async_tile_copies_per_wave<SR, D, NP>() + async_tile_copies_per_wave<SR, DV, NP>() + kRowCopies;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   const int tid = threadIdx.x;
@@ -483,14 +517,16 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   if (entry & kDeadItem) {
     // no query tile can interact with these kv rows (known from the ordering pass): zeros, no bookkeeping
     if (tid == 0) ticket = work.draw();
-    const int row_bytes = D * (p.dkdv_f32 ? 4 : 2), chunks = row_bytes / 16;
+    const int esize = p.dkdv_f32 ? 4 : 2;
     const int rows = min(TKV, p.kv_len - k0);
-    for (int i = tid; i < rows * chunks; i += NW * 64) {
-      const int64_t row = k0 + i / chunks;
-      const int at = (i % chunks) * 16;
-      *reinterpret_cast<uint4*>(dk_out + ((int64_t)b * p.dk_sb + (int64_t)kv_head * p.dk_sh + row * p.dk_ss) * (row_bytes / D) + at) = make_uint4(0, 0, 0, 0);
-      *reinterpret_cast<uint4*>(dv_out + ((int64_t)b * p.dv_sb + (int64_t)kv_head * p.dv_sh + row * p.dv_ss) * (row_bytes / D) + at) = make_uint4(0, 0, 0, 0);
-    }
+    auto zero_rows = [&](char* out, int64_t sb, int64_t sh, int64_t ss, int columns) {
+      const int chunks = columns * esize / 16;
+      for (int i = tid; i < rows * chunks; i += NW * 64)
+        *reinterpret_cast<uint4*>(out + ((int64_t)b * sb + (int64_t)kv_head * sh + (int64_t)(k0 + i / chunks) * ss) * esize +
+                                  (i % chunks) * 16) = make_uint4(0, 0, 0, 0);
+    };
+    zero_rows(dk_out, p.dk_sb, p.dk_sh, p.dk_ss, D);
+    zero_rows(dv_out, p.dv_sb, p.dv_sh, p.dv_ss, DV);
   } else {
 
   const int kbs = p.bk, qbs = p.bq;
@@ -561,6 +597,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   if (steps > 0) {
     const int first_head = pair_lo / n_live, first_li = pair_lo - first_head * n_live;
     // stationary fragments: K (negated when the scale is negative) for the P wave, V for the S wave
+    // (VSTEPS of them)
     vec8 frag[KSTEPS];
     {
       const char* base = p_wave ? p.k + ((int64_t)b * p.k_sb + (int64_t)kv_head * p.k_sh + (int64_t)(in ? kvcol : 0) * p.k_ss) * 2
@@ -569,22 +606,41 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
 #pragma unroll
       for (int ks = 0; ks < KSTEPS; ks++) {
         uint4 u = make_uint4(0, 0, 0, 0);
-        if (in) u = *reinterpret_cast<const uint4*>(base + (16 * ks + 8 * h) * 2);
+        if (in && (ks < VSTEPS || p_wave)) u = *reinterpret_cast<const uint4*>(base + (16 * ks + 8 * h) * 2);
         u.x ^= sign, u.y ^= sign, u.z ^= sign, u.w ^= sign;
         frag[ks] = __builtin_bit_cast(vec8, u);
       }
     }
-    int nat_off[KSTEPS], tr_off[DT][2];
+    // Operand addresses.  The P wave reads rows of Q and columns of dO, the S wave rows of dO and
+    // columns of Q; with value head_dim of its own each role has its own pattern in the same registers.
+    // (At one wavefront per SIMD there is room for one register per step: 16k tokens at head_dim 256 2.04
+    // against 2.32 ms with shared ones.)
+    constexpr bool kShared = Cfg::kWps == 2;
+    constexpr int kNatQ = kShared ? kNatRegs<D> : KSTEPS, kNatDo = kShared ? kNatRegs<DV> : VSTEPS;
+    constexpr int kTrQ = kShared ? kTrRegs<D> : DT, kTrDo = kShared ? kTrRegs<DV> : DTV;
+    constexpr int kNat = kNatQ > kNatDo ? kNatQ : kNatDo, kTr = kTrQ > kTrDo ? kTrQ : kTrDo;
+    int nat_off[kNat], tr_off[kTr][2];
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) nat_off[ks] = nat_offset<D>(c, ks, h);
+    for (int ks = 0; ks < kNat; ks++)
+      nat_off[ks] = D == DV || p_wave ? nat_offset<D>(c, ks, h) : nat_offset<DV>(c, ks, h);
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++) {
-      tr_off[dt][0] = tr_offset<D>(lane, dt, 0);
-      tr_off[dt][1] = tr_offset<D>(lane, dt, 1);
-    }
+    for (int dt = 0; dt < kTr; dt++)
+#pragma unroll
+      for (int half = 0; half < 2; half++)
+        tr_off[dt][half] = D == DV || !p_wave ? tr_offset<D>(lane, dt, half) : tr_offset<DV>(lane, dt, half);
+    // columns [32 dt, +32) of 16 rows of a Q tile (S wave) or a dO tile (P wave), transposed
+    auto read_q_t = [&](const char* rows16, int dt) {
+      constexpr int n = kTrQ;
+      return tr_read_a_swz<Tr>(rows16 + dt / n * kGroupBytes<D>, tr_off[dt % n][0], tr_off[dt % n][1]);
+    };
+    auto read_do_t = [&](const char* rows16, int dt) {
+      constexpr int n = kTrDo;
+      return tr_read_a_swz<Tr>(rows16 + dt / n * kGroupBytes<DV>, tr_off[dt % n][0], tr_off[dt % n][1]);
+    };
 
     const uint32_t smem_addr = (uint32_t)(uintptr_t)smem;
-    const AsyncTileCopy<SR, D, NP> copy_q(p.q_ss * 2, pair, lane), copy_do(p.do_ss * 2, pair, lane);
+    const AsyncTileCopy<SR, D, NP> copy_q(p.q_ss * 2, pair, lane);
+    const AsyncTileCopy<SR, DV, NP> copy_do(p.do_ss * 2, pair, lane);
     // Steps go through the list entries of one head of the group after the other; step s: its Q tile and row data go to
     // slot s % 4 of their rings, its dO tile to slot s % 3.  The issuing side keeps its own cursor
     // (list index, per-head base pointers) and advances it by additions only: divisions and 64-bit
@@ -609,8 +665,8 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     uint32_t is_entry = live_list[first_li];
     auto issue_next = [&](int q_slot, int do_slot) {
       const int qr0 = (int)(is_entry & 0xffffff) * kTile + is_sub * SR;
-      copy_q(is_q, qr0, p.q_len, smem_addr + Smem::kQ + q_slot * Smem::kTileBytes);
-      copy_do(is_do, qr0, p.q_len, smem_addr + Smem::kDo + do_slot * Smem::kTileBytes);
+      copy_q(is_q, qr0, p.q_len, smem_addr + Smem::kQ + q_slot * Smem::kQTileBytes);
+      copy_do(is_do, qr0, p.q_len, smem_addr + Smem::kDo + do_slot * Smem::kDoTileBytes);
 #pragma unroll
       for (int r = 0; r < kRowCopies; r++)
         async_copy_b32(is_rows[r] + (int64_t)min(qr0 + lane, p.q_len - 1) * 4,
@@ -633,15 +689,19 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     // [slot][unit mt][half st] x 64 lanes x 16 bytes, in the lane order of the C tile
     char* exchange = smem + Smem::kExchange + pair * 2 * Smem::kSlotBytes + lane * 16;
 
+    // Above head_dim 128 the accumulators and fragments leave no registers for operands requested ahead
+    // of the element-wise work.
+    constexpr bool kLean = D > 128 && Cfg::kWps == 2;
     // S wave, second part of a tile: dS = P * (dP - delta) rounded to the input dtype (masked
     // entries have P = 0), dK^T += Q^T dS.  x = dP of that tile.
     auto finish_dk = [&](const f32x16 (&x)[UNITS], const char* qtile, const float* delta_rows, const char* pslot) {
       vec8 ta[2][DT];
+      if (!kLean) {
 #pragma unroll
-      for (int st = 0; st < 2; st++)
+        for (int st = 0; st < 2; st++)
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++)
-          ta[st][dt] = tr_read_a_swz<Tr>(qtile + 16 * st * RB, tr_off[dt][0], tr_off[dt][1]);
+          for (int dt = 0; dt < DT; dt++) ta[st][dt] = read_q_t(qtile + 16 * st * RB, dt);
+      }
 #pragma unroll
       for (int mt = 0; mt < UNITS; mt++) {
         vec8 dsb[2];
@@ -660,13 +720,21 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
           }
           dsb[st] = pack8<Tr>(ds[0], ds[1], ds[2], ds[3], ds[4], ds[5], ds[6], ds[7]);
         }
+        if (kLean) {
+#pragma unroll
+          for (int st = 0; st < 2; st++)
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++)
+              acc[dt] = Tr::mfma(read_q_t(qtile + (32 * mt + 16 * st) * RB, dt), dsb[st], acc[dt]);
+          continue;
+        }
         vec8 tb[2][DT];  // operands of the next unit, requested before this unit's MFMAs
         if (mt + 1 < UNITS) {
 #pragma unroll
           for (int st = 0; st < 2; st++)
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
-              tb[st][dt] = tr_read_a_swz<Tr>(qtile + (32 * (mt + 1) + 16 * st) * RB, tr_off[dt][0], tr_off[dt][1]);
+              tb[st][dt] = read_q_t(qtile + (32 * (mt + 1) + 16 * st) * RB, dt);
         }
 #pragma unroll
         for (int st = 0; st < 2; st++)
@@ -701,14 +769,14 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
       const int t = e0 & 0xffffff;
       const bool active = (e0 >> (24 + wave)) & 1, active_prev = (ep >> (24 + wave)) & 1;
       const int qr0 = t * kTile + sub * SR;
-      const char* qtile = smem + Smem::kQ + q_slot * Smem::kTileBytes;
-      const char* dotile = smem + Smem::kDo + do_slot * Smem::kTileBytes;
+      const char* qtile = smem + Smem::kQ + q_slot * Smem::kQTileBytes;
+      const char* dotile = smem + Smem::kDo + do_slot * Smem::kDoTileBytes;
       const float* rowdata = reinterpret_cast<const float*>(smem + Smem::kRows + q_slot * Smem::kRowData);
       const int32_t* rowids = reinterpret_cast<const int32_t*>(rowdata + 2 * kTile);
       const bool full = t >= tf_lo && t < tf_hi;
 
       if (!p_wave && active_prev)
-        finish_dk(x, smem + Smem::kQ + q_prev * Smem::kTileBytes,
+        finish_dk(x, smem + Smem::kQ + q_prev * Smem::kQTileBytes,
                   reinterpret_cast<const float*>(smem + Smem::kRows + q_prev * Smem::kRowData) + kTile,
                   exchange + ((step - 1) & 1) * Smem::kSlotBytes);
 
@@ -720,28 +788,37 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
         for (int mt = 0; mt < UNITS; mt++)
 #pragma unroll
           for (int i = 0; i < 16; i++) x[mt][i] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ks++)
-#pragma unroll
-          for (int mt = 0; mt < UNITS; mt++)
-            x[mt] = Tr::mfma(*reinterpret_cast<const vec8*>(rows_a + 32 * mt * RB + nat_off[ks]), frag[ks], x[mt]);
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-        for (int i = 0; i < UNITS * KSTEPS - 4; i++) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        // (a macro: inside a lambda the scheduling barriers lost their effect)
+#define KVAX_CONTRACT(n, regs)                                                                                       \
+  _Pragma("unroll") for (int ks = 0; ks < (n) / 16; ks++)                                                            \
+      _Pragma("unroll") for (int mt = 0; mt < UNITS; mt++)                                                           \
+          x[mt] = Tr::mfma(*reinterpret_cast<const vec8*>(rows_a + 32 * mt * ((n) * 2) + nat_off[ks % (regs)] +      \
+                                                          ks / (regs) * kGroupBytes<n>), frag[ks], x[mt]);           \
+  __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);                                                                 \
+  _Pragma("unroll") for (int i = 0; i < UNITS * ((n) / 16) - 4; i++) {                                               \
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                               \
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                                                               \
+  }                                                                                                                  \
+  __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        if constexpr (D == DV) {
+          KVAX_CONTRACT(D, kNatQ)
+        } else if (p_wave) {
+          KVAX_CONTRACT(D, kNatQ)
+        } else {
+          KVAX_CONTRACT(DV, kNatDo)
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+#undef KVAX_CONTRACT
       }
 
       if (p_wave && active) {
         // operands of dV's first unit, requested before the element-wise work
-        vec8 ta[2][DT];
+        vec8 ta[2][DTV];
+        if (!kLean) {
 #pragma unroll
-        for (int st = 0; st < 2; st++)
+          for (int st = 0; st < 2; st++)
 #pragma unroll
-          for (int dt = 0; dt < DT; dt++)
-            ta[st][dt] = tr_read_a_swz<Tr>(dotile + 16 * st * RB, tr_off[dt][0], tr_off[dt][1]);
+            for (int dt = 0; dt < DTV; dt++) ta[st][dt] = read_do_t(dotile + 16 * st * RBV, dt);
+        }
         vec8 pb[UNITS][2];
         char* pslot = exchange + (step & 1) * Smem::kSlotBytes;
 #pragma unroll
@@ -770,23 +847,31 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
         // dV^T += dO^T P
 #pragma unroll
         for (int mt = 0; mt < UNITS; mt++) {
-          vec8 tb[2][DT];
+          if (kLean) {
+#pragma unroll
+            for (int st = 0; st < 2; st++)
+#pragma unroll
+              for (int dt = 0; dt < DTV; dt++)
+                acc[dt] = Tr::mfma(read_do_t(dotile + (32 * mt + 16 * st) * RBV, dt), pb[mt][st], acc[dt]);
+            continue;
+          }
+          vec8 tb[2][DTV];
           if (mt + 1 < UNITS) {
 #pragma unroll
             for (int st = 0; st < 2; st++)
 #pragma unroll
-              for (int dt = 0; dt < DT; dt++)
-                tb[st][dt] = tr_read_a_swz<Tr>(dotile + (32 * (mt + 1) + 16 * st) * RB, tr_off[dt][0], tr_off[dt][1]);
+              for (int dt = 0; dt < DTV; dt++)
+                tb[st][dt] = read_do_t(dotile + (32 * (mt + 1) + 16 * st) * RBV, dt);
           }
 #pragma unroll
           for (int st = 0; st < 2; st++)
 #pragma unroll
-            for (int dt = 0; dt < DT; dt++) acc[dt] = Tr::mfma(ta[st][dt], pb[mt][st], acc[dt]);
+            for (int dt = 0; dt < DTV; dt++) acc[dt] = Tr::mfma(ta[st][dt], pb[mt][st], acc[dt]);
           if (mt + 1 < UNITS) {
 #pragma unroll
             for (int st = 0; st < 2; st++)
 #pragma unroll
-              for (int dt = 0; dt < DT; dt++) ta[st][dt] = tb[st][dt];
+              for (int dt = 0; dt < DTV; dt++) ta[st][dt] = tb[st][dt];
           }
         }
       }
@@ -803,7 +888,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     // the S wave still owes the last tile
     __syncthreads();
     if (!p_wave && ((ep >> (24 + wave)) & 1))
-      finish_dk(x, smem + Smem::kQ + q_prev * Smem::kTileBytes,
+      finish_dk(x, smem + Smem::kQ + q_prev * Smem::kQTileBytes,
                 reinterpret_cast<const float*>(smem + Smem::kRows + q_prev * Smem::kRowData) + kTile,
                 exchange + ((steps - 1) & 1) * Smem::kSlotBytes);
   }
@@ -824,15 +909,17 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     const float mul = p_wave ? 1.f : p.scale;
     char* base = p_wave ? dv_out : dk_out;
     const int64_t sb = p_wave ? p.dv_sb : p.dk_sb, sh = p_wave ? p.dv_sh : p.dk_sh, ss = p_wave ? p.dv_ss : p.dk_ss;
-    constexpr int PC = D < 128 ? D : 128;  // columns per pass
+    constexpr int PC = D % 128 == 0 && DV % 128 == 0 ? 128 : 64;  // columns per pass
     constexpr int kDtPerPass = PC / 32;
     const int esize = p.dkdv_f32 ? 4 : 2;
     const int row_bytes = PC * esize;             // 128, 256 or 512
     const int chunks = row_bytes / 16;            // 8, 16 or 32 per row
     char* stage = smem + wave * (32 * PC * 4);    // room for the fp32 case
+    static_assert(NW * 32 * PC * 4 <= Smem::kTotal, "a wavefront's part of the LDS");
     const int64_t tile_off = (int64_t)b * sb + (int64_t)kv_head * sh + (int64_t)(k0 + pair * 32) * ss;
 #pragma unroll
     for (int pass = 0; pass < D / PC; pass++) {
+      if (D != DV && p_wave && pass >= DV / PC) break;
       char* mine = stage + c * row_bytes;
       if (p.dkdv_f32) {
 #pragma unroll
@@ -881,29 +968,29 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
 // Adds the parts' fp32 dK and dV in the order of the parts and writes them in the gradients' type and
 // strides.  A copy, bound by memory: 16 bytes per thread and part, four parts in flight.
 struct DkdvSumParams {
-  const float* parts;  // [part][dK, dV][batch, kv_len, kv heads, D]
-  char* dst[2];        // dK, dV
+  const float* parts[2];  // dK, dV: [part][batch, kv_len, kv heads, head_dim]
+  char* dst[2];
   int64_t sb[2], ss[2], sh[2];
-  int64_t total;       // 4-element pieces of one tensor
+  int64_t total[2];       // 4-element pieces of a tensor
+  int pieces[2];          // and of one of its rows
   int num_parts, kv_len, num_kv_heads;
   int f32;
 };
 
-template <class Tr, int D>
+template <class Tr>
 __global__ __launch_bounds__(256) void dkdv_sum_kernel(const DkdvSumParams p) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int which = blockIdx.y;
-  if (i >= p.total) return;
-  const float4* src = reinterpret_cast<const float4*>(p.parts) + which * p.total + i;
+  if (i >= p.total[which]) return;
+  const float4* src = reinterpret_cast<const float4*>(p.parts[which]) + i;
   float4 sum = src[0];
 #pragma unroll 4
   for (int part = 1; part < p.num_parts; part++) {
-    const float4 v = src[2 * p.total * part];
+    const float4 v = src[p.total[which] * part];
     sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
   }
-  constexpr int kPieces = D / 4;
-  int64_t row = i / kPieces;
-  const int d = (int)(i % kPieces) * 4;
+  int64_t row = i / p.pieces[which];
+  const int d = (int)(i % p.pieces[which]) * 4;
   const int head = (int)(row % p.num_kv_heads);
   row /= p.num_kv_heads;
   const int64_t at = row / p.kv_len * p.sb[which] + row % p.kv_len * p.ss[which] + head * p.sh[which] + d;
@@ -932,7 +1019,7 @@ __global__ __launch_bounds__(256) void dkdv_sum_kernel(const DkdvSumParams p) {
 // A function of the shapes, so that the workspace can be sized up front (at most 768 parts of 128 rows).
 int plan_dkdv_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int head_dim) {
   if (batch <= 0 || q_len <= 0 || kv_len <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return 1;
-  const int64_t items = (int64_t)batch * num_kv_heads * cdiv(kv_len, head_dim > 128 ? 64 : 128);
+  const int64_t items = (int64_t)batch * num_kv_heads * cdiv(kv_len, dkdv_kv_rows(head_dim));
   const int64_t steps = (int64_t)cdiv(q_len, kTile) * (num_heads / num_kv_heads);
   const int64_t one_round = min(kNumCus / items, steps / 8), two_rounds = min(2 * kNumCus / items, steps / 24),
                 three_rounds = min(3 * kNumCus / items, steps / 128);
@@ -948,12 +1035,12 @@ int reserve_lds(K kernel, int need, int bytes, LdsReservation* reservation, cons
 }
 
 // dQ launch: NW wavefronts (32 query rows each) per work-group, WPS per SIMD.
-template <class Tr, int D, int NW, int STAGES, int WPS = 2>
+template <class Tr, int D, int DV, int NW, int STAGES, int WPS = 2>
 int launch_dq(BwdParams p, hipStream_t stream) {
-  auto kernel = fa_bwd_dq_kernel<Tr, D, NW, WPS, STAGES>;
+  auto kernel = fa_bwd_dq_kernel<Tr, D, DV, NW, WPS, STAGES>;
   static LdsReservation done;
   constexpr int kLimit = kLdsPerCu / (4 * WPS / NW);  // work-groups per compute unit share the LDS
-  const int smem = DqSmem<D, STAGES>::kTotal + live_tiles_bytes(NW, p.n_kv_tiles);
+  const int smem = DqSmem<D, DV, STAGES>::kTotal + live_tiles_bytes(NW, p.n_kv_tiles);
   if (int rc = reserve_lds(kernel, smem, kLimit, &done, "the dQ kernel")) return rc;
   p.num_tiles = cdiv(p.q_len, NW * 32);
   p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, p.group}.grid();
@@ -961,13 +1048,13 @@ int launch_dq(BwdParams p, hipStream_t stream) {
   return check_launch("fa_bwd_dq_kernel");
 }
 
-template <class Tr, int D>
+template <class Tr, int D, int DV>
 int launch_bwd(BwdParams p, hipStream_t stream) {
   // a key sequence too long for the dQ kernel's largest configuration is refused before anything
   // is enqueued (the dK/dV kernel has no such limit)
   if (p.q_len > 0 && !(p.flags & KVAX_FA_SKIP_DQ)) {
-    const int need = D > 128 ? DqSmem<D, 2>::kTotal + live_tiles_bytes(4, p.n_kv_tiles)
-                             : DqSmem<D, 3>::kTotal + live_tiles_bytes(8, p.n_kv_tiles);
+    const int need = D > 128 ? DqSmem<D, DV, 2>::kTotal + live_tiles_bytes(4, p.n_kv_tiles)
+                             : DqSmem<D, DV, 3>::kTotal + live_tiles_bytes(8, p.n_kv_tiles);
     if (need > kLdsPerCu)
       return fail(KVAX_EUNSUPPORTED, "the dQ kernel needs %d bytes of LDS for tile bitmaps (limit %d): "
                   "sequence too long", need, kLdsPerCu);
@@ -987,7 +1074,7 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
   const bool run_dq = p.q_len > 0 && !(p.flags & KVAX_FA_SKIP_DQ);
   const bool run_dkdv = p.kv_len > 0 && !(p.flags & KVAX_FA_SKIP_DKDV);
   const bool dq_small =
-      DqSmem<D, kStagesSmall>::kTotal + live_tiles_bytes(4, p.n_kv_tiles) <= kLdsHalfCu;
+      DqSmem<D, DV, kStagesSmall>::kTotal + live_tiles_bytes(4, p.n_kv_tiles) <= kLdsHalfCu;
   // dK/dV runs one long work-group per compute unit: its light work items are dispatched last, by
   // decreasing number of live tiles, so that the launch does not end on a few long ones
   {
@@ -1001,49 +1088,65 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
     }
   }
   if (run_dq) {
-    if constexpr (D > 128) {
-      if (int rc = launch_dq<Tr, D, 4, 2, 1>(p, stream)) return rc;
+    if constexpr (D == 256) {
+      if (int rc = launch_dq<Tr, D, DV, 4, 2, 1>(p, stream)) return rc;
+    } else if constexpr (D > 128) {
+      // At 192 with 128 for the values eight wavefronts, two per SIMD, just fit their registers (with 192
+      // they spill 48 in the step: 175 against 120 us on 4k tokens, 16 heads) and pay where more
+      // work-groups than compute units remain (us, eight / four wavefronts, 16 heads): 2 x 4k tokens
+      // 201 / 225, 16k 785 / 1055, 6k 318 / 402; 4k 201 / 177, 2k 106 / 86.
+      [[maybe_unused]] const bool fills = (int64_t)p.batch * p.num_heads * cdiv(p.q_len, 256) > kNumCus;
+      if constexpr (DV == 128) {
+        if (fills && DqSmem<D, DV, 2>::kTotal + live_tiles_bytes(8, p.n_kv_tiles) <= kLdsPerCu) {
+          if (int rc = launch_dq<Tr, D, DV, 8, 2>(p, stream)) return rc;
+        } else {
+          if (int rc = launch_dq<Tr, D, DV, 4, 2, 1>(p, stream)) return rc;
+        }
+      } else {
+        if (int rc = launch_dq<Tr, D, DV, 4, 2, 1>(p, stream)) return rc;
+      }
     } else {
       if (dq_small) {
-        if (int rc = launch_dq<Tr, D, 4, kStagesSmall>(p, stream)) return rc;
+        if (int rc = launch_dq<Tr, D, DV, 4, kStagesSmall>(p, stream)) return rc;
       } else {
-        if (int rc = launch_dq<Tr, D, 8, 3>(p, stream)) return rc;
+        if (int rc = launch_dq<Tr, D, DV, 8, 3>(p, stream)) return rc;
       }
     }
   }
   // dK/dV: wavefronts in role pairs (see DkdvCfg)
   if (run_dkdv) {
     constexpr int NW = Cfg::kWaves;
-    auto kernel = fa_bwd_dkdv_kernel<Tr, D>;
+    auto kernel = fa_bwd_dkdv_kernel<Tr, D, DV>;
     static LdsReservation done;
     // live-tile bookkeeping for as many query tiles as the remaining LDS holds (a multiple of 64)
     constexpr int kLdsLimit = kLdsPerCu;
     int chunk = 64;
-    while (chunk < p.n_q_tiles && DkdvSmem<D>::kTotal + live_tiles_bytes(NW, chunk * 2) <= kLdsLimit) chunk *= 2;
+    while (chunk < p.n_q_tiles && DkdvSmem<D, DV>::kTotal + live_tiles_bytes(NW, chunk * 2) <= kLdsLimit) chunk *= 2;
     p.list_tiles = min(chunk, max(p.n_q_tiles, 1));
-    const int smem = DkdvSmem<D>::kTotal + live_tiles_bytes(NW, p.list_tiles);
+    const int smem = DkdvSmem<D, DV>::kTotal + live_tiles_bytes(NW, p.list_tiles);
     if (int rc = reserve_lds(kernel, smem, kLdsLimit, &done, "the dK/dV kernel")) return rc;
     p.num_tiles = cdiv(p.kv_len, Cfg::kKvRows);
     p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, p.dkdv_parts}.grid();
     DkdvSumParams sum{};
     if (p.dkdv_parts > 1) {  // the kernel leaves fp32 parts, dkdv_sum_kernel adds them
-      sum.parts = p.parts_ws;
+      const int64_t rows = (int64_t)p.batch * p.kv_len * p.num_kv_heads;
       sum.dst[0] = p.dk, sum.sb[0] = p.dk_sb, sum.ss[0] = p.dk_ss, sum.sh[0] = p.dk_sh;
       sum.dst[1] = p.dv, sum.sb[1] = p.dv_sb, sum.ss[1] = p.dv_ss, sum.sh[1] = p.dv_sh;
-      sum.total = (int64_t)p.batch * p.kv_len * p.num_kv_heads * D / 4;
+      sum.pieces[0] = D / 4, sum.pieces[1] = DV / 4;
+      sum.total[0] = rows * (D / 4), sum.total[1] = rows * (DV / 4);
+      sum.parts[0] = p.parts_ws, sum.parts[1] = p.parts_ws + rows * D * p.dkdv_parts;
       sum.num_parts = p.dkdv_parts, sum.kv_len = p.kv_len, sum.num_kv_heads = p.num_kv_heads;
       sum.f32 = p.dkdv_f32;
-      p.dk = (char*)p.parts_ws, p.dv = p.dk + sum.total * 16;
-      p.dk_part = p.dv_part = sum.total * 32;
-      p.dk_sh = p.dv_sh = D, p.dk_ss = p.dv_ss = (int64_t)p.num_kv_heads * D;
-      p.dk_sb = p.dv_sb = p.dk_ss * p.kv_len;
+      p.dk = (char*)sum.parts[0], p.dk_sh = D, p.dk_ss = (int64_t)p.num_kv_heads * D, p.dk_sb = p.dk_ss * p.kv_len;
+      p.dv = (char*)sum.parts[1], p.dv_sh = DV, p.dv_ss = (int64_t)p.num_kv_heads * DV, p.dv_sb = p.dv_ss * p.kv_len;
+      p.dk_part = sum.total[0] * 16, p.dv_part = sum.total[1] * 16;
       p.dkdv_f32 = 1;
     }
     p.dkdv_queue = tile_order_counters(p.order_ws, p.batch, p.num_tiles) + p.batch;
     hipLaunchKernelGGL(kernel, dim3(min(p.total_items, kNumCus)), dim3(NW * 64), smem, stream, p);
     if (int rc = check_launch("fa_bwd_dkdv_kernel")) return rc;
     if (p.dkdv_parts > 1) {
-      hipLaunchKernelGGL((dkdv_sum_kernel<Tr, D>), dim3((unsigned)((sum.total + 255) / 256), 2), dim3(256), 0, stream, sum);
+      hipLaunchKernelGGL(dkdv_sum_kernel<Tr>, dim3((unsigned)((sum.total[0] + 255) / 256), 2), dim3(256), 0, stream, sum);
       if (int rc = check_launch("dkdv_sum_kernel")) return rc;
     }
   }
@@ -1063,14 +1166,14 @@ static size_t delta_bytes(const kvax_fa_args* a) {
 // of the kv and query sequences, and the dispatch order of the dK/dV work items.
 static size_t parts_offset(const kvax_fa_args* a) {
   return delta_bytes(a) + tile_summary_bytes(a->batch, a->kv_len) + tile_summary_bytes(a->batch, a->q_len) +
-         tile_order_bytes(a->batch, cdiv(a->kv_len, a->head_dim > 128 ? 64 : 128));
+         tile_order_bytes(a->batch, cdiv(a->kv_len, dkdv_kv_rows(a->head_dim)));
 }
 static int dkdv_parts(const kvax_fa_args* a) {
   return plan_dkdv_parts(a->batch, a->q_len, a->kv_len, a->num_heads, a->num_kv_heads, a->head_dim);
 }
 static size_t dkdv_parts_bytes(const kvax_fa_args* a) {
   const int parts = dkdv_parts(a);
-  return parts == 1 ? 0 : (size_t)parts * 2 * a->batch * a->kv_len * a->num_kv_heads * a->head_dim * sizeof(float);
+  return parts == 1 ? 0 : (size_t)parts * a->batch * a->kv_len * a->num_kv_heads * (a->head_dim + value_head_dim(a)) * sizeof(float);
 }
 
 extern "C" size_t kvax_fa_bwd_workspace_bytes(const kvax_fa_args* a) {
@@ -1148,10 +1251,7 @@ extern "C" int kvax_fa_bwd(const kvax_fa_args* a, void* workspace, size_t worksp
   p.scale_log2_abs = fmaxf(fabsf(a->scale), 1e-30f) * 1.4426950408889634f;
   p.k_sign = a->scale < 0.f ? 0x80008000u : 0u;
   hipStream_t stream = (hipStream_t)stream_;
-  const bool bf16 = a->dtype == KVAX_BF16;
-  if (a->head_dim == 256)
-    return bf16 ? launch_bwd<Bf16, 256>(p, stream) : launch_bwd<F16, 256>(p, stream);
-  if (a->head_dim == 128)
-    return bf16 ? launch_bwd<Bf16, 128>(p, stream) : launch_bwd<F16, 128>(p, stream);
-  return bf16 ? launch_bwd<Bf16, 64>(p, stream) : launch_bwd<F16, 64>(p, stream);
+  return dispatch_heads(a, [&](auto tr, auto d, auto dv) {
+    return launch_bwd<decltype(tr), decltype(d)::value, decltype(dv)::value>(p, stream);
+  });
 }

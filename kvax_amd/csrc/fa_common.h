@@ -15,6 +15,8 @@
 #include <type_traits>
 #include <utility>
 
+#include "kvax_amd.h"
+
 namespace kvax {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -370,9 +372,22 @@ __device__ __forceinline__ int swz(int r) {
   // D == 128, 256: rows are one or two full turns of the 64 banks apart, so the chunk position
   // modulo 16 decides the banks and one 4-bit pattern serves both (at 256 it permutes the chunks
   // within each half of the row)
-  if (D >= 128) return ((r & 3) << 2) | ((r >> 2) & 3);
-  return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);  // D == 64: 8 chunks per row
+  if (D % 128 == 0) return ((r & 3) << 2) | ((r >> 2) & 3);
+  // D == 64: 8 chunks per row, two rows per turn of the banks.  D == 192: three groups of 8 chunks per
+  // row; group g of row r starts where group 0 of row r + g would at D == 64 (modulo the banks), so
+  // the same pattern within each group serves
+  return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
 }
+// The permutation stays within groups of this many chunks of a row: operand addresses that differ by
+// whole groups differ by a constant and share an address register.
+template <int D>
+constexpr int kSwzGroup = D % 128 == 0 ? 16 : 8;
+template <int D>
+constexpr int kNatRegs = kSwzGroup<D> / 2 < D / 16 ? kSwzGroup<D> / 2 : D / 16;  // two chunks per 16-element step
+template <int D>
+constexpr int kTrRegs = kSwzGroup<D> / 4 < D / 32 ? kSwzGroup<D> / 4 : D / 32;   // four per 32-column block
+template <int D>
+constexpr int kGroupBytes = kSwzGroup<D> * 16;
 
 // One asynchronous 16-byte-per-lane copy: the wave writes 1 KiB at LDS address `lds_addr`
 // (wave-uniform), lane i providing its own global source address.  Completion is tracked by
@@ -417,16 +432,17 @@ __device__ __forceinline__ void async_copy_b128(const char* sbase, uint32_t lane
 // kernels' time before it was reduced to one multiply per tile.
 template <int ROWS, int D, int NW>
 struct AsyncTileCopy {
-  static constexpr int kRowsPerCopy = 1024 / (D * 2);  // 4 (D = 128) or 8 (D = 64)
-  static constexpr int kCopies = ROWS / kRowsPerCopy;
+  static constexpr int kRowsPerCopy = 1024 / (D * 2);  // 4 (D = 128) or 8 (D = 64); 2 2/3 at D = 192
+  static constexpr int kCopies = ROWS * D * 2 / 1024;
   static constexpr int kPerWave = kCopies / NW;
   static constexpr int kChunks = D / 8;
   static_assert(kCopies % NW == 0, "copies must split evenly over the waves");
-  // Copy j of a wave covers the rows (j * NW + wave) * kRowsPerCopy + [0, kRowsPerCopy).  Up to
-  // head_dim 128 and with a multiple of four waves the swizzle term of a lane is the same in all of
-  // them, so one per-lane offset serves every copy and the scalar base moves on instead (vector
+  static_assert(ROWS * D * 2 % 1024 == 0, "a tile is a whole number of copies");
+  // Copy j of a wave covers the chunks (j * NW + wave) * 64 + [0, 64) of the tile.  Where these are whole
+  // rows and the copies of a wave lie multiples of 16 rows apart (the period of the swizzle), the swizzle
+  // term of a lane is the same in all of them, so one per-lane offset serves every copy and the scalar base moves on instead (vector
   // registers are what the kernels run out of first).
-  static constexpr bool kCompact = D <= 128 && NW % 4 == 0;
+  static constexpr bool kCompact = 1024 % (D * 2) == 0 && NW * kRowsPerCopy % 16 == 0;
   static constexpr int kOffsets = kCompact ? 1 : kPerWave;
   uint32_t lane_off[kOffsets];  // (row of the lane within the tile) * stride + chunk * 16, per copy
   int64_t stride;
@@ -436,10 +452,10 @@ struct AsyncTileCopy {
   // check it), so that one scalar base per tile plus 32-bit lane offsets address every copy.
   __device__ __forceinline__ AsyncTileCopy(int64_t row_stride_bytes, int wave, int lane)
       : stride(row_stride_bytes), wave_u(__builtin_amdgcn_readfirstlane(wave)), lane_(lane) {
-    const int rin = lane / kChunks, pos = lane % kChunks;
 #pragma unroll
     for (int j = 0; j < kOffsets; j++) {
-      const int r = (j * NW + wave_u) * kRowsPerCopy + rin;
+      const int at = (j * NW + wave_u) * 64 + lane;  // 16-byte chunk of the tile
+      const int r = at / kChunks, pos = at % kChunks;
       lane_off[j] = (uint32_t)(r * row_stride_bytes) + (uint32_t)((pos ^ swz<D>(r)) * 16);
     }
   }
@@ -473,12 +489,11 @@ struct AsyncTileCopy {
     } else {  // ragged tail: clamp each lane's row (32-bit offsets from the tile's base)
       int l = lane_;
       asm volatile("" : "+v"(l));  // keeps what follows from being computed ahead of a loop around the call
-      const int rin = l / kChunks, pos = l % kChunks;
       const int last = limit - 1 - row0;
 #pragma unroll
       for (int j = J0; j < J1; j++) {
         const int grp = j * NW + wave_u;
-        const int r = grp * kRowsPerCopy + rin;
+        const int r = (grp * 64 + l) / kChunks, pos = (grp * 64 + l) % kChunks;
         const uint32_t off = (uint32_t)min(r, last) * (uint32_t)stride + (uint32_t)((pos ^ swz<D>(r)) * 16);
         async_copy_b128(tile_base, off, tile_addr + grp * 1024);
       }
@@ -487,7 +502,7 @@ struct AsyncTileCopy {
 };
 template <int ROWS, int D, int NW>
 constexpr int async_tile_copies_per_wave() {
-  return ROWS / (1024 / (D * 2)) / NW;
+  return ROWS * D * 2 / 1024 / NW;
 }
 
 // Per-lane byte offsets into a swizzled tile.
@@ -519,6 +534,28 @@ __device__ __forceinline__ typename Tr::vec8 tr_read_a_swz(const char* tile_row0
   s16x4 hi = ds_read_tr16(tile_row0 + off_hi);
   s16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   return __builtin_bit_cast(typename Tr::vec8, v);
+}
+
+// Head sizes that are built: query/key and value head_dim alike, or 192 with 128.
+inline int value_head_dim(const kvax_fa_args* a) { return a->v_head_dim ? a->v_head_dim : a->head_dim; }
+inline int head_config(const kvax_fa_args* a) {
+  const int d = a->head_dim, dv = value_head_dim(a);
+  if (d == 192 && dv == 128) return 1;
+  return d == dv && (d == 64 || d == 128 || d == 192 || d == 256) ? 2 : 0;
+}
+// Calls f(traits, integral_constant<head_dim>, integral_constant<value head_dim>) for a checked call.
+template <class F>
+int dispatch_heads(const kvax_fa_args* a, F f) {
+  auto with_type = [&](auto d, auto dv) {
+    return a->dtype == KVAX_BF16 ? f(Bf16{}, d, dv) : f(F16{}, d, dv);
+  };
+  using std::integral_constant;
+  if (a->head_dim == 256) return with_type(integral_constant<int, 256>{}, integral_constant<int, 256>{});
+  if (a->head_dim == 192 && value_head_dim(a) == 128)
+    return with_type(integral_constant<int, 192>{}, integral_constant<int, 128>{});
+  if (a->head_dim == 192) return with_type(integral_constant<int, 192>{}, integral_constant<int, 192>{});
+  if (a->head_dim == 128) return with_type(integral_constant<int, 128>{}, integral_constant<int, 128>{});
+  return with_type(integral_constant<int, 64>{}, integral_constant<int, 64>{});
 }
 
 }  // namespace kvax

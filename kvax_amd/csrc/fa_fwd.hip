@@ -69,11 +69,11 @@ struct FwdParams {
   float* part_ml;             // [items, num_parts, part_rows, 2] running max (base 2) and sum
 };
 
-template <int D, int STAGES>
+template <int D, int DV, int STAGES>
 struct FwdSmem {
-  static constexpr int kTileBytes = kTK * D * 2;  // swizzled, unpadded
-  static constexpr int kIdBytes = 2 * kTK * 4;    // seg + pos
-  static constexpr int kStage = 2 * kTileBytes + kIdBytes;
+  static constexpr int kTileBytes = kTK * D * 2;   // K tile; swizzled, unpadded
+  static constexpr int kIds = kTileBytes + kTK * DV * 2;  // behind the V tile: seg + pos
+  static constexpr int kStage = kIds + 2 * kTK * 4;
   static constexpr int kTotal = STAGES * kStage;
 };
 
@@ -89,22 +89,25 @@ struct FwdSmem {
 // for all rows of the batch keep the work-groups equally long when the rows are not.
 // NARROW: split mode with at most 32 rows (decoding), where the four wavefronts share the arithmetic
 // of every tile instead of the rows (see the constants below).
-template <class Tr, int D, int MQ, int NW, int WPS, int STAGES, bool SPLIT, bool NARROW>
+template <class Tr, int D, int DV, int MQ, int NW, int WPS, int STAGES, bool SPLIT, bool NARROW>
 __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p) {
   using vec8 = typename Tr::vec8;
-  using Smem = FwdSmem<D, STAGES>;
+  using Smem = FwdSmem<D, DV, STAGES>;
   constexpr int TQ = NW * 32 * MQ;
   constexpr int KSTEPS = D / 16;  // contraction steps of S^T = K Q^T
-  constexpr int DT = D / 32;      // 32-row tiles of O^T
-  constexpr int RB = D * 2;       // bytes per tile row
-  constexpr int kCopies = 2 * async_tile_copies_per_wave<kTK, D, NW>() + 1;  // per wave and tile
+  constexpr int DT = DV / 32;     // 32-row tiles of O^T
+  constexpr int RB = D * 2, RBV = DV * 2;  // bytes per row of a K / V tile
+  constexpr int kCopies = async_tile_copies_per_wave<kTK, D, NW>() + async_tile_copies_per_wave<kTK, DV, NW>() + 1;  // per wave and tile
   static_assert(STAGES >= 2 && STAGES <= 4, "the loop below keeps STAGES - 1 tiles in flight");
   // NARROW (split mode with at most 32 rows, i.e. decoding): every wavefront takes the same rows and
   // a quarter of the arithmetic of a tile - wavefront w the key rows [32 (w & 1), +32) and, of
   // O^T += V^T P^T, the head-dim slices of half w >> 1 - instead of one wavefront working while three
   // wait.  The two key halves keep separate running maxima and leave separate partial results.
   static_assert(!NARROW || (SPLIT && NW == 4 && MQ == 1 && DT % 2 == 0), "narrow mode splits a tile four ways");
-  constexpr int KT = NARROW ? 1 : 2;         // 32-key halves of a tile per wavefront
+  // 32-key halves of a tile per wavefront that are worked on together, and one after the other: at
+  // head_dim 256 with two wavefronts per SIMD the registers hold the scores of one half at a time
+  constexpr int HALVES = D == 256 && WPS == 2 ? 2 : 1;
+  constexpr int KT = NARROW || HALVES == 2 ? 1 : 2;
   constexpr int DTO = NARROW ? DT / 2 : DT;  // 32-row slices of O^T per wavefront
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -178,7 +181,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   if (!SPLIT && t_hi <= t_lo) {
     // No row of the tile can attend to anything (padding queries): zeros for O and lse, and nothing
     // is read.  Whole rows, 16 bytes per lane.
-    constexpr int kChunks = D * 2 / 16;
+    constexpr int kChunks = DV * 2 / 16;
     const int rows = min(TQ, p.q_len - q0);
     for (int i = tid; i < rows * kChunks; i += NW * 64)
       *reinterpret_cast<uint4*>(obase + (int64_t)(q0 + i / kChunks) * p.o_ss * 2 + (i % kChunks) * 16) =
@@ -299,9 +302,13 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
     // offsets from the start of the LDS block, not addresses
     constexpr bool kAddresses = D >= 128;
     const uint32_t addr0 = kAddresses ? smem_addr : 0u;
-    uint32_t nat_addr[KSTEPS], tr_addr[DTO][2];
+    // (steps whole swizzle groups apart share a register; narrow mode's second half of the head-dim
+    // slices may start in the middle of a group)
+    // (at one wavefront per SIMD there is room for a register per step)
+    constexpr int kNat = WPS == 1 ? KSTEPS : kNatRegs<D>, kTr = NARROW || WPS == 1 ? DTO : kTrRegs<DV>;
+    uint32_t nat_addr[kNat], tr_addr[kTr][2];
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) {
+    for (int ks = 0; ks < kNat; ks++) {
       nat_addr[ks] = addr0 + 32 * kt0 * RB + nat_offset<D>(c, ks, h);
       // opaque to the optimiser, which would otherwise keep the summands and add them again per read
       // (only where the loop below exists once per stage: elsewhere a scalar stage offset is added per
@@ -309,20 +316,21 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
       if constexpr (kStaticStages) asm volatile("" : "+v"(nat_addr[ks]));
     }
 #pragma unroll
-    for (int dt = 0; dt < DTO; dt++) {
-      tr_addr[dt][0] = addr0 + Smem::kTileBytes + 32 * kt0 * RB + tr_offset<D>(lane, dt0 + dt, 0);
-      tr_addr[dt][1] = addr0 + Smem::kTileBytes + 32 * kt0 * RB + tr_offset<D>(lane, dt0 + dt, 1);
+    for (int dt = 0; dt < kTr; dt++) {
+      tr_addr[dt][0] = addr0 + Smem::kTileBytes + 32 * kt0 * RBV + tr_offset<DV>(lane, dt0 + dt, 0);
+      tr_addr[dt][1] = addr0 + Smem::kTileBytes + 32 * kt0 * RBV + tr_offset<DV>(lane, dt0 + dt, 1);
       if constexpr (kStaticStages) asm volatile("" : "+v"(tr_addr[dt][0]), "+v"(tr_addr[dt][1]));
     }
 
     const int32_t* id_src = (wave & 1) ? kv_pos : kv_seg;
-    const AsyncTileCopy<kTK, D, NW> copy_k(p.k_ss * 2, wave, lane), copy_v(p.v_ss * 2, wave, lane);
+    const AsyncTileCopy<kTK, D, NW> copy_k(p.k_ss * 2, wave, lane);
+    const AsyncTileCopy<kTK, DV, NW> copy_v(p.v_ss * 2, wave, lane);
     auto issue = [&](int tile, int stage) {
       const uint32_t base = smem_addr + stage * Smem::kStage;
       copy_k(kbase, tile * kTK, p.kv_len, base);
       copy_v(vbase, tile * kTK, p.kv_len, base + Smem::kTileBytes);
       async_copy_b32(id_src + min(tile * kTK + lane, p.kv_len - 1),
-                     __builtin_amdgcn_readfirstlane(base + 2 * Smem::kTileBytes + (wave & 1) * (kTK * 4)));
+                     __builtin_amdgcn_readfirstlane(base + Smem::kIds + (wave & 1) * (kTK * 4)));
     };
 
     {
@@ -358,10 +366,12 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
       if ((e0 >> (24 + wave)) & 1) {
         const int kv0 = t * kTK;
         const char* ktile = smem + stage * Smem::kStage;
-        const int32_t* ids = reinterpret_cast<const int32_t*>(ktile + 2 * Smem::kTileBytes);
+        const int32_t* ids = reinterpret_cast<const int32_t*>(ktile + Smem::kIds);
 
+#pragma unroll 1
+        for (int hf = 0; hf < HALVES; hf++) {
         // ---- S^T = K Q^T -----------------------------------------------------------------
-        f32x16 s[KT][MQ];  // key half kt0 + kt
+        f32x16 s[KT][MQ];  // key half kt0 + kt + hf
 #pragma unroll
         for (int kt = 0; kt < KT; kt++)
 #pragma unroll
@@ -373,8 +383,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
           vec8 a[KT];
 #pragma unroll
           for (int kt = 0; kt < KT; kt++)
-            a[kt] = kAddresses ? lds_load<vec8>(nat_addr[ks] + stage * Smem::kStage + 32 * kt * RB)
-                               : *reinterpret_cast<const vec8*>(ktile + 32 * kt * RB + nat_addr[ks]);
+            a[kt] = kAddresses ? lds_load<vec8>(nat_addr[ks % kNat] + stage * Smem::kStage + 32 * (kt + hf) * RB +
+                                                ks / kNat * kGroupBytes<D>)
+                               : *reinterpret_cast<const vec8*>(ktile + 32 * (kt + hf) * RB + nat_addr[ks]);
 #pragma unroll
           for (int kt = 0; kt < KT; kt++)
 #pragma unroll
@@ -395,7 +406,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
           for (int kt = 0; kt < KT; kt++)
 #pragma unroll
             for (int qt = 0; qt < MQ; qt++)
-              mask_c_tile<true>(s[kt][qt], ids, ids + kTK, 32 * (kt0 + kt), kv0, h, qseg[qt], qpos[qt],
+              mask_c_tile<true>(s[kt][qt], ids, ids + kTK, 32 * (kt0 + kt + hf), kv0, h, qseg[qt], qpos[qt],
                                 col_lo[qt], col_width[qt], -INFINITY);
         }
 
@@ -455,12 +466,13 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
           for (int st = 0; st < 2; st++)
 #pragma unroll
             for (int dt = 0; dt < DTO; dt++) {
-              const uint32_t at = stage * Smem::kStage + (32 * kt + 16 * st) * RB;
-              const vec8 a = kAddresses ? tr_read_a_at<Tr>(tr_addr[dt][0] + at, tr_addr[dt][1] + at)
+              const uint32_t at = stage * Smem::kStage + (32 * (kt + hf) + 16 * st) * RBV + dt / kTr * kGroupBytes<DV>;
+              const vec8 a = kAddresses ? tr_read_a_at<Tr>(tr_addr[dt % kTr][0] + at, tr_addr[dt % kTr][1] + at)
                                         : tr_read_a_swz<Tr>(smem + at, tr_addr[dt][0], tr_addr[dt][1]);
 #pragma unroll
               for (int qt = 0; qt < MQ; qt++) o[dt][qt] = Tr::mfma(a, pb[kt][st][qt], o[dt][qt]);
             }
+        }
       }
 #pragma unroll
       for (int k = 0; k < kAhead; k++) e[k] = e[k + 1];
@@ -489,7 +501,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
     if (row_in[0] && prow < p.part_rows) {
       const int64_t part = ((int64_t)item * p.num_splits + split) * (NARROW ? 2 : 1) + kt0;
       const int64_t slot = part * p.part_rows + prow;
-      float* po = p.part_o + slot * D + 32 * dt0;
+      float* po = p.part_o + slot * DV + 32 * dt0;
 #pragma unroll
       for (int dt = 0; dt < DTO; dt++)
 #pragma unroll
@@ -516,7 +528,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
     const float inv = alive ? 1.f / l : 0.f;
     if (row_in[0] && h == 0) lse[qrow[0]] = alive ? m_run[0] + fast_log2(l) : 0.f;
     __syncthreads();  // every wavefront has read its last tile
-    constexpr int kRowBytes = D * 2, kChunks = kRowBytes / 16, kRowsPerStore = 64 / kChunks;
+    constexpr int kRowBytes = DV * 2, kChunks = kRowBytes / 16;
+    static_assert(NW * 32 * kRowBytes <= Smem::kTotal, "a wavefront's part of the tile space");
+    constexpr int kSwz = kChunks % 16 == 0 ? kChunks - 1 : 7;  // chunks are permuted within a power of two of them
     char* stage = smem + wave * (32 * kRowBytes);
     char* mine = stage + c * kRowBytes;
 #pragma unroll
@@ -526,12 +540,12 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
         uint2 u;
         u.x = Tr::pack2(o[dt][0][4 * g4 + 0] * inv, o[dt][0][4 * g4 + 1] * inv);
         u.y = Tr::pack2(o[dt][0][4 * g4 + 2] * inv, o[dt][0][4 * g4 + 3] * inv);
-        *reinterpret_cast<uint2*>(mine + (((4 * dt + g4) ^ (c & (kChunks - 1))) * 16) + 8 * h) = u;
+        *reinterpret_cast<uint2*>(mine + (((4 * dt + g4) ^ (c & kSwz)) * 16) + 8 * h) = u;
       }
 #pragma unroll
-    for (int r0 = 0; r0 < 32; r0 += kRowsPerStore) {
-      const int row = r0 + lane / kChunks, chunk = lane % kChunks;
-      const uint4 v = *reinterpret_cast<const uint4*>(stage + row * kRowBytes + ((chunk ^ (row & (kChunks - 1))) * 16));
+    for (int i = 0; i < 32 * kChunks; i += 64) {
+      const int row = (i + lane) / kChunks, chunk = (i + lane) % kChunks;
+      const uint4 v = *reinterpret_cast<const uint4*>(stage + row * kRowBytes + ((chunk ^ (row & kSwz)) * 16));
       const int qr = q0 + wave * 32 + row;
       if (qr < p.q_len) *reinterpret_cast<uint4*>(obase + (int64_t)qr * p.o_ss * 2 + chunk * 16) = v;
     }
@@ -587,7 +601,7 @@ template <class Tr, int D>
 __global__ __launch_bounds__(256, 1) void fa_fwd_wide_kernel(const FwdParams p) {
   using vec8 = typename Tr::vec8;
   constexpr int NW = 4, MQ = 2, STAGES = 2;
-  using Smem = FwdSmem<D, STAGES>;
+  using Smem = FwdSmem<D, D, STAGES>;
   constexpr int TQ = NW * 32 * MQ;
   constexpr int KSTEPS = D / 16, DT = D / 32, RB = D * 2;
   constexpr int kCopies = 2 * async_tile_copies_per_wave<kTK, D, NW>() + 1;
@@ -1026,13 +1040,16 @@ struct FwdPlan {
   size_t summary_bytes = 0, list_bytes = 0;
   size_t total_bytes() const { return summary_bytes + part_o_bytes + part_ml_bytes + list_bytes; }
 };
-FwdPlan plan_forward(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int head_dim,
+// LDS of one stage of the K/V ring.
+constexpr int fwd_stage_bytes(int d_qk, int d_v) { return kTK * (d_qk + d_v) * 2 + 2 * kTK * 4; }
+
+FwdPlan plan_forward(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int d_qk, int d_v,
                      bool want_wide) {
   FwdPlan plan;
   if (batch <= 0 || q_len <= 0 || kv_len <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return plan;
   const int n_kv_tiles = cdiv(kv_len, kTileRows);
   plan.summary_bytes = tile_summary_bytes(batch, kv_len);
-  if (want_wide && head_dim == 128) {  // lists of live tiles per 256 query rows, shared by the heads
+  if (want_wide && d_qk == 128 && d_v == 128) {  // lists of live tiles per 256 query rows, shared by the heads
     const size_t bytes = tile_list_bytes(batch, q_len, kWideTileRows, kv_len);
     if (bytes > 0 && bytes <= kMaxTileListBytes && live_tiles_bytes(8, n_kv_tiles) <= kLdsPerCu) {
       plan.wide = true;
@@ -1041,8 +1058,9 @@ FwdPlan plan_forward(int batch, int q_len, int kv_len, int num_heads, int num_kv
   }
   const int64_t regular = (int64_t)batch * num_heads * cdiv(q_len, kSplitTileRows);
   // the ring of the four-wavefront configuration (see launch_fwd_auto) and its share of the LDS
-  const int ring_bytes = (2 * kTK * head_dim * 2 + 2 * kTK * 4) * (head_dim == 64 ? 3 : 2);
-  if (ring_bytes + live_tiles_bytes(4, n_kv_tiles) > (head_dim == 256 ? kLdsPerCu : kLdsHalfCu)) return plan;
+  const int ring_bytes = fwd_stage_bytes(d_qk, d_v) * (d_qk == 64 ? 3 : 2);
+  const bool alone = d_qk > 128;  // one work-group per compute unit
+  if (ring_bytes + live_tiles_bytes(4, n_kv_tiles) > (alone ? kLdsPerCu : kLdsHalfCu)) return plan;
   if (q_len >= kSplitTileRows && regular >= 256) return plan;
   plan.split_mode = true;
   plan.list_bytes = 0;
@@ -1050,7 +1068,7 @@ FwdPlan plan_forward(int batch, int q_len, int kv_len, int num_heads, int num_kv
   const int64_t rows = (int64_t)q_len * (num_heads / num_kv_heads);
   const int64_t items = (int64_t)batch * num_kv_heads * ((rows + kSplitTileRows - 1) / kSplitTileRows);
   // windows of one size for every item, at most 64 per item
-  const int64_t resident = (head_dim == 256 ? 1 : 2) * kNumCus;
+  const int64_t resident = (alone ? 1 : 2) * kNumCus;
   int64_t max_splits = items >= resident ? 1 : resident / items;
   max_splits = max_splits < 64 ? max_splits : 64;
   int window = cdiv(n_kv_tiles, (int)max_splits);
@@ -1063,14 +1081,14 @@ FwdPlan plan_forward(int batch, int q_len, int kv_len, int num_heads, int num_kv
   if (plan.num_parts > 1) {
     plan.part_rows = (int)(rows < kSplitTileRows ? rows : kSplitTileRows);
     const size_t slots = (size_t)items * plan.num_parts * plan.part_rows;
-    plan.part_o_bytes = (slots * head_dim * sizeof(float) + 15) / 16 * 16;
+    plan.part_o_bytes = (slots * d_v * sizeof(float) + 15) / 16 * 16;
     plan.part_ml_bytes = (slots * 2 * sizeof(float) + 15) / 16 * 16;
   }
   if (plan.narrow()) plan.summary_bytes = 0;
   return plan;
 }
 
-template <class Tr, int D, int MQ, int NW, int WPS, int STAGES = 3, bool SPLIT = false, bool NARROW = false>
+template <class Tr, int D, int DV, int MQ, int NW, int WPS, int STAGES = 3, bool SPLIT = false, bool NARROW = false>
 int launch_fwd(const FwdParams& p0, hipStream_t stream) {
   FwdParams p = p0;
   constexpr int TQ = NW * 32 * MQ;
@@ -1084,8 +1102,8 @@ int launch_fwd(const FwdParams& p0, hipStream_t stream) {
     p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_q_tiles, p.group}.grid();
   }
   if (p.batch * p.num_heads * p.num_q_tiles == 0) return KVAX_OK;
-  auto kernel = fa_fwd_kernel<Tr, D, MQ, NW, WPS, STAGES, SPLIT, NARROW>;
-  const int smem = FwdSmem<D, STAGES>::kTotal + live_tiles_bytes(NW, p.n_kv_tiles);
+  auto kernel = fa_fwd_kernel<Tr, D, DV, MQ, NW, WPS, STAGES, SPLIT, NARROW>;
+  const int smem = FwdSmem<D, DV, STAGES>::kTotal + live_tiles_bytes(NW, p.n_kv_tiles);
   constexpr int kWgPerCu = (WPS * 4 / NW) > 0 ? (WPS * 4 / NW) : 1;
   constexpr int kMaxSmem = kLdsPerCu / kWgPerCu;
   if (smem > kMaxSmem)
@@ -1099,9 +1117,9 @@ int launch_fwd(const FwdParams& p0, hipStream_t stream) {
     // a work-group per row where that is about what the chip holds at once and there is something to deal
     const int rows = p.batch * p.num_kv_heads * p.num_q_tiles * p.part_rows;
     if (rows <= 4 * kNumCus && p.num_parts > kCombineBatch)
-      hipLaunchKernelGGL((fa_fwd_combine_kernel<Tr, D, true>), dim3(rows), dim3(256), 0, stream, p, TQ, rows);
+      hipLaunchKernelGGL((fa_fwd_combine_kernel<Tr, DV, true>), dim3(rows), dim3(256), 0, stream, p, TQ, rows);
     else
-      hipLaunchKernelGGL((fa_fwd_combine_kernel<Tr, D, false>), dim3(cdiv(rows, 256 / (D / 4))), dim3(256), 0, stream, p,
+      hipLaunchKernelGGL((fa_fwd_combine_kernel<Tr, DV, false>), dim3(cdiv(rows, 256 / (DV / 4))), dim3(256), 0, stream, p,
                          TQ, rows);
     return check_launch("fa_fwd_combine_kernel");
   }
@@ -1116,7 +1134,7 @@ int launch_fwd_wide(const FwdParams& p0, hipStream_t stream) {
   p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_q_tiles, p.group}.grid();
   if (p.batch * p.num_heads * p.num_q_tiles == 0) return KVAX_OK;
   auto kernel = fa_fwd_wide_kernel<Tr, D>;
-  constexpr int smem = FwdSmem<D, 2>::kTotal;
+  constexpr int smem = FwdSmem<D, D, 2>::kTotal;
   static LdsReservation reservation;
   if (int rc = reservation.ensure(kernel, kLdsPerCu, "the wide forward kernel")) return rc;
   hipLaunchKernelGGL(kernel, dim3(p.total_items), dim3(256), smem, stream, p);
@@ -1126,21 +1144,28 @@ int launch_fwd_wide(const FwdParams& p0, hipStream_t stream) {
 // Two work-groups of four wavefronts per compute unit (each hides the other's prologue, barriers
 // and final stores) whenever the tile bitmaps of the sequence fit beside the smaller ring;
 // otherwise one work-group of eight wavefronts.
-template <class Tr, int D>
+template <class Tr, int D, int DV>
 int launch_fwd_auto(const FwdParams& p, hipStream_t stream) {
-  if constexpr (D == 256) {
-    // 128 accumulator registers for O and 64 for the Q fragments: one wavefront per SIMD, one
-    // work-group of four per compute unit, two 64.5 KB stages
-    if (p.split_mode && p.num_parts > p.num_splits) return launch_fwd<Tr, D, 1, 4, 1, 2, true, true>(p, stream);
-    if (p.split_mode) return launch_fwd<Tr, D, 1, 4, 1, 2, true>(p, stream);
-    return launch_fwd<Tr, D, 1, 4, 1, 2>(p, stream);
+  const bool narrow = p.split_mode && p.num_parts > p.num_splits;
+  if constexpr (D > 128) {
+    // Two stages leave no room for a second work-group on a compute unit: eight wavefronts, two per SIMD,
+    // where more work-groups than compute units remain and their bookkeeping fits, else four.  us, eight /
+    // four wavefronts, 16 heads, at 192 with 128: 2 x 4k tokens 140 / 144, 6k 210 / 245, 16k (documents of
+    // 4k) 515 / 657; 4k 132 / 110, 2k 71 / 52; at 256: 6k 322 / 476, 16k 774 / 1214; 4k 201 / 206, 3k 151 /
+    // 143.
+    if (narrow) return launch_fwd<Tr, D, DV, 1, 4, 1, 2, true, true>(p, stream);
+    if (p.split_mode) return launch_fwd<Tr, D, DV, 1, 4, 1, 2, true>(p, stream);
+    const bool fills = (int64_t)p.batch * p.num_heads * cdiv(p.q_len, 256) > kNumCus;
+    if (fills && FwdSmem<D, DV, 2>::kTotal + live_tiles_bytes(8, p.n_kv_tiles) <= kLdsPerCu)
+      return launch_fwd<Tr, D, DV, 1, 8, 2, 2>(p, stream);
+    return launch_fwd<Tr, D, DV, 1, 4, 1, 2>(p, stream);
   } else {
     constexpr int kStagesSmall = D == 128 ? 2 : 3;
-    if (p.split_mode && p.num_parts > p.num_splits) return launch_fwd<Tr, D, 1, 4, 2, kStagesSmall, true, true>(p, stream);
-    if (p.split_mode) return launch_fwd<Tr, D, 1, 4, 2, kStagesSmall, true>(p, stream);
-    const int small = FwdSmem<D, kStagesSmall>::kTotal + live_tiles_bytes(4, p.n_kv_tiles);
-    if (small <= kLdsHalfCu) return launch_fwd<Tr, D, 1, 4, 2, kStagesSmall>(p, stream);
-    return launch_fwd<Tr, D, 1, 8, 2, 3>(p, stream);
+    if (narrow) return launch_fwd<Tr, D, DV, 1, 4, 2, kStagesSmall, true, true>(p, stream);
+    if (p.split_mode) return launch_fwd<Tr, D, DV, 1, 4, 2, kStagesSmall, true>(p, stream);
+    const int small = FwdSmem<D, DV, kStagesSmall>::kTotal + live_tiles_bytes(4, p.n_kv_tiles);
+    if (small <= kLdsHalfCu) return launch_fwd<Tr, D, DV, 1, 4, 2, kStagesSmall>(p, stream);
+    return launch_fwd<Tr, D, DV, 1, 8, 2, 3>(p, stream);
   }
 }
 
@@ -1153,8 +1178,9 @@ int validate_fa_common(const kvax_fa_args* a) {
   if (a->num_heads % a->num_kv_heads)
     return fail(KVAX_EINVAL, "num_heads %d is not a multiple of num_kv_heads %d", a->num_heads,
                 a->num_kv_heads);
-  if (a->head_dim != 64 && a->head_dim != 128 && a->head_dim != 256)
-    return fail(KVAX_EUNSUPPORTED, "head_dim %d is not built (64, 128 and 256 are)", a->head_dim);
+  if (a->v_head_dim < 0 || head_config(a) == 0)
+    return fail(KVAX_EUNSUPPORTED, "head_dim %d with value head_dim %d is not built (64, 128, 192, 256 and 192 with "
+                "128 are)", a->head_dim, value_head_dim(a));
   if (a->dtype != KVAX_BF16 && a->dtype != KVAX_F16)
     return fail(KVAX_EUNSUPPORTED, "dtype %d is not supported (bf16 and f16 are)", a->dtype);
   if (a->flags & ~(KVAX_FA_DKDV_F32 | KVAX_FA_SKIP_DELTA | KVAX_FA_SKIP_DQ | KVAX_FA_SKIP_DKDV | KVAX_FA_FWD_WIDE))
@@ -1185,7 +1211,7 @@ extern "C" size_t kvax_fa_fwd_workspace_bytes(const kvax_fa_args* a) {
   if (!a || a->batch < 0 || a->kv_len < 0) return 0;
   // see FwdPlan
   return plan_forward(a->batch, a->q_len, a->kv_len, a->num_heads, a->num_kv_heads, a->head_dim,
-                                    (a->flags & KVAX_FA_FWD_WIDE) != 0).total_bytes();
+                                    value_head_dim(a), (a->flags & KVAX_FA_FWD_WIDE) != 0).total_bytes();
 }
 
 // Scratch memory of kvax_fa_fwd_static: one copy per GPU the library runs on, held until the
@@ -1279,7 +1305,7 @@ int fa_fwd_impl(const kvax_fa_args* a, void* workspace, kvax_stream_t stream_) {
   p.kv_tiles = (const int4*)workspace;
   p.n_kv_tiles = cdiv(a->kv_len, kTileRows);
   const FwdPlan plan = plan_forward(a->batch, a->q_len, a->kv_len, a->num_heads, a->num_kv_heads, a->head_dim,
-                                    (a->flags & KVAX_FA_FWD_WIDE) != 0);
+                                    value_head_dim(a), (a->flags & KVAX_FA_FWD_WIDE) != 0);
   p.split_mode = plan.split_mode;
   p.num_splits = plan.num_splits;
   p.num_parts = plan.num_parts;
@@ -1292,8 +1318,8 @@ int fa_fwd_impl(const kvax_fa_args* a, void* workspace, kvax_stream_t stream_) {
   p.list_stride = (int)tile_list_stride(p.n_kv_tiles);
   hipStream_t stream = (hipStream_t)stream_;
   if (!plan.wide) {  // too long for the largest configuration: refuse before anything is enqueued
-    const int ring = (2 * kTK * a->head_dim * 2 + 2 * kTK * 4) * (a->head_dim == 256 ? 2 : 3);
-    const int need = ring + live_tiles_bytes(a->head_dim == 256 ? 4 : 8, p.n_kv_tiles);
+    const int ring = fwd_stage_bytes(a->head_dim, value_head_dim(a)) * (a->head_dim > 128 ? 2 : 3);
+    const int need = ring + live_tiles_bytes(a->head_dim > 128 ? 4 : 8, p.n_kv_tiles);
     if (need > kLdsPerCu)
       return fail(KVAX_EUNSUPPORTED, "kv_len %d needs %d bytes of LDS for tile bitmaps (limit %d)",
                   a->kv_len, need, kLdsPerCu);
@@ -1310,11 +1336,8 @@ int fa_fwd_impl(const kvax_fa_args* a, void* workspace, kvax_stream_t stream_) {
   }
   if (plan.wide)
     return a->dtype == KVAX_BF16 ? launch_fwd_wide<Bf16, 128>(p, stream) : launch_fwd_wide<F16, 128>(p, stream);
-  const bool bf16 = a->dtype == KVAX_BF16;
-  if (a->head_dim == 256)
-    return bf16 ? launch_fwd_auto<Bf16, 256>(p, stream) : launch_fwd_auto<F16, 256>(p, stream);
-  if (a->head_dim == 128)
-    return bf16 ? launch_fwd_auto<Bf16, 128>(p, stream) : launch_fwd_auto<F16, 128>(p, stream);
-  return bf16 ? launch_fwd_auto<Bf16, 64>(p, stream) : launch_fwd_auto<F16, 64>(p, stream);
+  return dispatch_heads(a, [&](auto tr, auto d, auto dv) {
+    return launch_fwd_auto<decltype(tr), decltype(d)::value, decltype(dv)::value>(p, stream);
+  });
 }
 }  // namespace

@@ -29,9 +29,10 @@ from kvax_amd.utils.sharding import context_parallel_degree
 from kvax_amd.utils.specs import get_attention_specs
 from kvax_amd.utils.typing import AttentionMask, DeviceArray
 
-SUPPORTED_HEAD_DIMS = (64, 128, 256)  # what the kernels are built for
+# (query/key, value) head dims the kernels are built for, smallest work first
+BUILT_HEAD_DIMS = ((64, 64), (128, 128), (192, 128), (192, 192), (256, 256))
 # What ``flash_attention`` takes for query/key: the reference's list (flash_attention_triton.py:1397).
-# Sizes between the built ones (16, 32, 192) and a different value head_dim are zero-padded.
+# Other sizes are zero-padded to the first built pair that holds them.
 ACCEPTED_HEAD_DIMS = (16, 32, 64, 128, 192, 256)
 _DTYPES = {torch.bfloat16: _native.KVAX_BF16, torch.float16: _native.KVAX_F16}
 
@@ -77,8 +78,8 @@ def _check_inputs(query, key, value):
         raise ValueError("query and key/value disagree on batch size or head_dim")
     if d not in ACCEPTED_HEAD_DIMS:
         raise ValueError(f"Attention hid_dim can take values {list(ACCEPTED_HEAD_DIMS)}")
-    if not 1 <= value.shape[3] <= SUPPORTED_HEAD_DIMS[-1]:
-        raise ValueError(f"value head_dim {value.shape[3]} is outside 1..{SUPPORTED_HEAD_DIMS[-1]}")
+    if not 1 <= value.shape[3] <= BUILT_HEAD_DIMS[-1][1]:
+        raise ValueError(f"value head_dim {value.shape[3]} is outside 1..{BUILT_HEAD_DIMS[-1][1]}")
     if hq % hkv != 0:
         raise ValueError(f"num_heads {hq} must be divisible by num_kv_heads {hkv}")
 
@@ -92,7 +93,7 @@ def _base_args(query, key, value, q_pos, q_seg, kv_pos, kv_seg, scale, fwd_param
     a.kv_pos, a.kv_seg = kv_pos.data_ptr(), kv_seg.data_ptr()
     a.q_strides, a.k_strides, a.v_strides = _strides3(query), _strides3(key), _strides3(value)
     a.batch, a.q_len, a.kv_len = b, sq, sk
-    a.num_heads, a.num_kv_heads, a.head_dim = hq, hkv, d
+    a.num_heads, a.num_kv_heads, a.head_dim, a.v_head_dim = hq, hkv, d, value.shape[3]
     a.fwd_query_block, a.fwd_kv_block = fwd_params.query_block_size, fwd_params.kv_block_size
     a.bwd_query_block, a.bwd_kv_block = bwd_params.query_block_size, bwd_params.kv_block_size
     a.dtype = _DTYPES[query.dtype]
@@ -107,7 +108,7 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
 
 def flash_attention_forward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, fwd_mask, scale,
                             fwd_params, bwd_params, buffers=None, static_scratch=False, flags=0):
-    """One device's forward: returns (out like query, lse fp32 [batch, heads, q_len]).
+    """One device's forward: returns (out like query with the value's head_dim, lse fp32 [batch, heads, q_len]).
     ``buffers`` = (out, lse) lets a caller reuse its output tensors.  With ``static_scratch`` (and
     ``buffers``) the call goes through ``kvax_fa_fwd_static`` and allocates no device memory: the
     scratch memory is the library's own fixed buffer, shared by all calls on the GPU.  ``flags``:
@@ -116,7 +117,7 @@ def flash_attention_forward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, fwd
     if buffers is not None:
         out, lse = buffers
     else:
-        out = torch.empty_like(query)
+        out = torch.empty_like(query) if value.shape[3] == d else query.new_empty((b, sq, hq, value.shape[3]))
         lse = torch.empty((b, hq, sq), dtype=torch.float32, device=query.device)
     a = _base_args(query, key, value, q_pos, q_seg, kv_pos, kv_seg, scale, fwd_params, bwd_params)
     a.out, a.lse, a.o_strides = out.data_ptr(), lse.data_ptr(), _strides3(out)
@@ -255,7 +256,7 @@ def flash_attention(
     layouts; the kernels trust it, so ids that return to an earlier value give wrong results
     without an error.  Ids need not be sorted or dense (``5 5 2 2 7`` is fine).
     Query/key head dims 16, 32, 64, 128, 192, 256 and any value head dim up to 256 are taken (the
-    kernels run at 64, 128 or 256; other sizes are zero-padded here).
+    kernels run at 64, 128, 192 and 256 and at 192 with 128 for the values; others are zero-padded here).
     ``memory_optimized_gqa_backward`` is accepted and has no effect: dK/dV are always reduced
     over the query heads of a group inside the kernel, which is what the flag asks for.
     ``debug`` (passed to the Triton launcher in the reference) checks the precondition below on the
@@ -290,16 +291,16 @@ def flash_attention(
     # columns of P V, so the tensors are padded to the next built size and the output is cut back
     # (autograd does the same to the gradients).
     d_qk, d_v = query.shape[3], value.shape[3]
-    d_run = next(d for d in SUPPORTED_HEAD_DIMS if d >= max(d_qk, d_v))
-    if d_qk != d_run:
-        query = torch.nn.functional.pad(query, (0, d_run - d_qk))
-        key = torch.nn.functional.pad(key, (0, d_run - d_qk))
-    if d_v != d_run:
-        value = torch.nn.functional.pad(value, (0, d_run - d_v))
+    run_qk, run_v = next(r for r in BUILT_HEAD_DIMS if r[0] >= d_qk and r[1] >= d_v)
+    if d_qk != run_qk:
+        query = torch.nn.functional.pad(query, (0, run_qk - d_qk))
+        key = torch.nn.functional.pad(key, (0, run_qk - d_qk))
+    if d_v != run_v:
+        value = torch.nn.functional.pad(value, (0, run_v - d_v))
     out = _FlashAttentionFn.apply(
         query, key, value, query_positions, query_segment_ids, kv_positions, kv_segment_ids,
         tuple(mask), float(scale), fwd_params, bwd_params, cp)
-    return out if d_v == d_run else out[..., :d_v]
+    return out if d_v == run_v else out[..., :d_v]
 
 
 def _check_documents_are_contiguous(segment_ids: torch.Tensor, name: str) -> None:

@@ -1,0 +1,79 @@
+"""The kernels built for query/key head_dim 192, with value head_dim 128 and 192 (tiles of 384-byte rows, operand
+sizes that differ between the two contractions), and for 256: every forward path (one query, short and long query
+sequences), the backward, ragged lengths, padding, strided tensors and the pairs that are padded to them, against
+the dense CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from kvax_amd import create_attention_mask, flash_attention
+from kvax_amd.ops.flash_attention import flash_attention_backward, flash_attention_forward
+from kvax_amd.utils import FlashAttentionParamsConfig, attention_specs
+from kvax_amd.utils.benchmarking import generate_random_segments_lengths, make_random_attention_inputs
+from oracle import attention_oracle as ao
+from tests.tolerances import OPERAND_ROUNDING, check_close
+
+pytestmark = pytest.mark.gpu
+SPEC = ("data", None, "model", None)
+P = FlashAttentionParamsConfig(64, 64)
+
+
+def _inputs(b, sq, sk, hq, hkv, d, dv, pad, docs, device, dtype=torch.bfloat16):
+    data, scale = make_random_attention_inputs(
+        b, sq, sk, hq, hkv, d, dv, seed=sq + sk + d + dv, num_pad_tokens=pad, start_query_position=max(sk - sq, 0),
+        list_of_segment_lengths=generate_random_segments_lengths(min(sq, sk), docs), device=device)
+    return [t.to(dtype) for t in data[:3]], data[3:], scale
+
+
+def _host(tensors):
+    return [t.detach().float().cpu().numpy() if t.dtype.is_floating_point else t.cpu().numpy() for t in tensors]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b, sq, sk, hq, hkv, d, dv, pad, docs", [
+    (2, 1, 5000, 8, 2, 192, 128, 0, 1),      # one query: four wavefronts share a tile, partial results of 128 and 192 columns
+    (2, 1, 5000, 8, 2, 192, 192, 0, 1),
+    (1, 48, 2000, 16, 4, 192, 128, 0, 1),    # split, two row tiles
+    (1, 200, 3001, 4, 2, 192, 192, 0, 1),
+    (2, 640, 640, 32, 32, 192, 128, 60, 4),  # one work-group of eight wavefronts per compute unit, ragged query tile
+    (2, 520, 1111, 32, 16, 192, 192, 30, 3),
+    (2, 640, 640, 32, 32, 256, 256, 60, 4),
+    (2, 300, 300, 4, 2, 128, 160, 0, 2),     # padded to 192
+    (1, 300, 300, 4, 2, 192, 40, 0, 2),
+    (1, 300, 300, 4, 2, 64, 224, 0, 2),      # padded to 256
+])
+def test_forward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, dtype):
+    qkv, ids, scale = _inputs(b, sq, sk, hq, hkv, d, dv, pad, docs, device, dtype)
+    with attention_specs(SPEC, SPEC):
+        mask = create_attention_mask(*ids, fwd_params=P)
+        out = flash_attention(*qkv, *ids, mask, scale=scale, fwd_params=P)
+    assert out.shape == (b, sq, hq, dv)
+    ref, _ = ao.attention_forward(*_host(qkv), *_host(ids), scale)
+    check_close("out", out, ref)
+    assert not out[ids[1] == -1].any()
+
+
+@pytest.mark.parametrize("b, sq, sk, hq, hkv, d, dv, pad, docs, fp32", [
+    (2, 640, 640, 4, 2, 192, 128, 65, 3, True),
+    (1, 1000, 1000, 6, 2, 192, 192, 77, 9, True),   # ragged
+    (1, 129, 65, 4, 4, 192, 128, 0, 1, False),      # the smallest number of tiles and a row beyond
+    (3, 1280, 1280, 32, 32, 192, 128, 100, 4, False),  # more items than compute units: one part each
+    (3, 1280, 1280, 32, 32, 256, 256, 100, 4, False),
+    (1, 1000, 1000, 6, 2, 256, 256, 77, 9, True),
+])
+def test_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32):
+    (q, k, v), ids, scale = _inputs(b, sq, sk, hq, hkv, d, dv, pad, docs, device)
+    # heads before the sequence in memory, as a caller with [batch, heads, seq, dim] tensors passes them
+    q, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, v))
+    dout = torch.randn((b, sq, hq, dv), generator=torch.Generator().manual_seed(2)).to(q.dtype).to(device)
+    with attention_specs(SPEC, SPEC):
+        masks = create_attention_mask(*ids, fwd_params=P, bwd_params=P, calc_bwd_mask=True)
+    out, lse = flash_attention_forward(q, k, v, *ids, masks[0], scale, P, P)
+    grads = flash_attention_backward(q, k, v, *ids, masks[1], masks[2], out, lse, dout, scale, P, P, dkdv_fp32=fp32)
+    heads = None if hq < 32 else [1]
+    refs = ao.attention_backward(*_host((q, k, v)), *_host(ids), scale, *_host([dout]), dtype=np.float64, heads=heads)
+    if heads:
+        grads, refs = ([x[:, :, 1:2] for x in grads], [r[:, :, 1:2] if r.shape[2] > 1 else r for r in refs])
+    for name, got, ref in zip(("dq", "dk", "dv"), grads, refs):
+        check_close(name, got, ref, rel=OPERAND_ROUNDING)
+    assert not grads[0][ids[1] == -1].any() and not grads[1][ids[3] == -1].any() and not grads[2][ids[3] == -1].any()
