@@ -14,7 +14,9 @@
 //                                    for the "full" predicate); sentinel fix-ups applied in
 //                                    place.
 //
-// Work is O(S + n_outer * n_inner / 64) instead of the reference's O(n_outer * S) re-reads.
+// Work is O(S + n_outer * n_inner / 64) instead of the reference's O(n_outer * S) re-reads.  Sequences
+// of up to kFusedTokens are done in one launch instead (fused_masks_kernel): the two passes are a launch
+// and a trip to memory each, and nothing else.
 #include "common.h"
 
 namespace kvax {
@@ -103,17 +105,10 @@ struct BoundsParams {
   int skip_pad;
 };
 
-// grid: (ceil(max_outer / kWavesPerGroup), batch * max_shards, num_jobs)
-__global__ __launch_bounds__(kWave* kWavesPerGroup) void block_bounds_kernel(BoundsParams p, int max_shards) {
-  const BoundsJob& job = p.jobs[blockIdx.z];
-  const int lane = threadIdx.x % kWave;
-  const int o = blockIdx.x * kWavesPerGroup + threadIdx.x / kWave;
-  const int b = blockIdx.y / max_shards;
-  const int shard = blockIdx.y % max_shards;
-  if (o >= job.n_outer || shard >= job.num_shards) return;
-  const int n_inner = job.n_inner_total / job.num_shards;
-  const int4 os = job.outer[(size_t)b * job.n_outer + o];
-  const int4* inner = job.inner + (size_t)b * job.n_inner_total + (size_t)shard * n_inner;
+// The bounds of outer block o of batch row b (by one wavefront): `os` is its summary, `inner` the n_inner
+// summaries of the inner blocks of the shard.
+__device__ __forceinline__ void write_bounds(const BoundsJob& job, const BoundsParams& p, const int4 os,
+                                             const int4* inner, int n_inner, int b, int shard, int o, int lane) {
   const bool osame = os.x == os.y;
   int lower = n_inner, upper = 0, lower_full = n_inner, upper_full = 0;
   if (p.skip_pad && osame && os.x == p.pad_id) {
@@ -159,6 +154,92 @@ __global__ __launch_bounds__(kWave* kWavesPerGroup) void block_bounds_kernel(Bou
     job.lower_full[idx] = lower_full;
     job.upper_full[idx] = upper_full;
   }
+}
+
+// grid: (ceil(max_outer / kWavesPerGroup), batch * max_shards, num_jobs)
+__global__ __launch_bounds__(kWave* kWavesPerGroup) void block_bounds_kernel(BoundsParams p, int max_shards) {
+  const BoundsJob& job = p.jobs[blockIdx.z];
+  const int o = blockIdx.x * kWavesPerGroup + threadIdx.x / kWave;
+  const int b = blockIdx.y / max_shards;
+  const int shard = blockIdx.y % max_shards;
+  if (o >= job.n_outer || shard >= job.num_shards) return;
+  const int n_inner = job.n_inner_total / job.num_shards;
+  write_bounds(job, p, job.outer[(size_t)b * job.n_outer + o],
+               job.inner + (size_t)b * job.n_inner_total + (size_t)shard * n_inner, n_inner, b, shard, o,
+               threadIdx.x % kWave);
+}
+
+// Both passes in one launch for short sequences: every work-group summarises all inner blocks of its batch
+// row and mask, and kFusedOuter outer blocks, into LDS, and then works out their bounds.  The ids are read
+// once per work-group instead of once, which costs less than the second launch and trip to memory while
+// they are few.  16 lanes share a block, each with up to eight of its tokens in flight, so that four lane
+// exchanges per value reduce four blocks at once.  us in the kernels, two launches against one, 128-token
+// blocks: three masks of 2k tokens 7.4 / 4.8, one mask of 4 rows of 2k keys 7.3 / 4.1, three masks of 2 x
+// 8k 7.3 / 8.1, of 32k 7.4 / 15.7.
+constexpr int kFusedTokens = 4096;
+constexpr int kFusedOuter = 64;
+constexpr int kFusedInner = 2048;  // summaries that fit the LDS of a work-group
+constexpr int kFusedBlockSize = 512;  // beyond, 16 lanes are too few for a block
+constexpr int kFusedThreads = 1024;
+struct FusedParams {
+  BoundsParams bounds;
+  SummaryJob outer[KVAX_MAX_MASKS], inner[KVAX_MAX_MASKS];  // `out` unused
+};
+
+// Summary of one block by the 16 lanes `sub` = 0 .. 15 (all get it).
+__device__ __forceinline__ int4 summarise_block(const SummaryJob& job, int b, int block, int32_t pad_id, int sub) {
+  const int32_t* pos = job.pos + (size_t)b * job.len;
+  const int32_t* seg = job.seg + (size_t)b * job.len;
+  const int start = block * job.block_size, size = block < job.n_blocks ? job.block_size : 0;
+  int4 r = make_int4(kInt32Max, kInt32Min, kInt32Max, kInt32Min);
+  constexpr int kInFlight = 8;
+  for (int i0 = sub; i0 < size; i0 += 16 * kInFlight) {
+    int32_t s[kInFlight], q[kInFlight];
+#pragma unroll
+    for (int j = 0; j < kInFlight; j++) {
+      const int t = start + i0 + 16 * j;
+      const bool in = i0 + 16 * j < size && t < job.len;
+      s[j] = in ? seg[t] : -1;
+      q[j] = in ? pos[t] : job.pos_fill;
+    }
+#pragma unroll
+    for (int j = 0; j < kInFlight; j++) {
+      if (i0 + 16 * j >= size) continue;
+      const int32_t id = s[j] == -1 ? pad_id : s[j];
+      r.x = min(r.x, id), r.y = max(r.y, id), r.z = min(r.z, q[j]), r.w = max(r.w, q[j]);
+    }
+  }
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) {
+    r.x = min(r.x, __shfl_xor(r.x, off));
+    r.y = max(r.y, __shfl_xor(r.y, off));
+    r.z = min(r.z, __shfl_xor(r.z, off));
+    r.w = max(r.w, __shfl_xor(r.w, off));
+  }
+  return r;
+}
+
+// grid: (ceil(max_outer / kFusedOuter), batch, num_jobs); LDS: the inner summaries
+__global__ __launch_bounds__(kFusedThreads) void fused_masks_kernel(FusedParams p) {
+  extern __shared__ int4 inner[];
+  __shared__ int4 outer[kFusedOuter];
+  const BoundsJob& job = p.bounds.jobs[blockIdx.z];
+  const int b = blockIdx.y, o0 = blockIdx.x * kFusedOuter;
+  if (o0 >= job.n_outer) return;
+  const int slot = threadIdx.x / 16, sub = threadIdx.x % 16;
+  static_assert(kFusedThreads / 16 == kFusedOuter, "a group of 16 lanes per outer block");
+  const int4 os = summarise_block(p.outer[blockIdx.z], b, o0 + slot, p.bounds.pad_id, sub);
+  if (sub == 0) outer[slot] = os;
+  for (int i0 = 0; i0 < job.n_inner_total; i0 += kFusedThreads / 16) {
+    const int4 is = summarise_block(p.inner[blockIdx.z], b, i0 + slot, p.bounds.pad_id, sub);
+    if (sub == 0 && i0 + slot < job.n_inner_total) inner[i0 + slot] = is;
+  }
+  __syncthreads();
+  const int n_inner = job.n_inner_total / job.num_shards;
+  const int last = min(kFusedOuter, job.n_outer - o0);
+  for (int k = threadIdx.x / kWave; k < last; k += kFusedThreads / kWave)
+    for (int shard = 0; shard < job.num_shards; shard++)
+      write_bounds(job, p.bounds, outer[k], inner + shard * n_inner, n_inner, b, shard, o0 + k, threadIdx.x % kWave);
 }
 
 struct SummaryKey {
@@ -262,7 +343,7 @@ extern "C" int kvax_mask_build(const int32_t* q_pos, const int32_t* q_seg, const
   SummaryParams sp{};
   sp.num_jobs = num_keys;
   sp.pad_id = pad_ids[0];
-  int max_blocks = 0;
+  int max_blocks = 0, max_block_size = 0;
   for (int k = 0; k < num_keys; k++) {
     SummaryJob& j = sp.jobs[k];
     j.pos = keys[k].kv ? kv_pos : q_pos;
@@ -273,6 +354,7 @@ extern "C" int kvax_mask_build(const int32_t* q_pos, const int32_t* q_seg, const
     j.n_blocks = keys[k].n_blocks;
     j.pos_fill = keys[k].kv ? kInt32Max : -1;
     max_blocks = max_blocks > j.n_blocks ? max_blocks : j.n_blocks;
+    max_block_size = max_block_size > j.block_size ? max_block_size : j.block_size;
   }
   BoundsParams bp{};
   bp.num_jobs = num_masks;
@@ -307,6 +389,19 @@ extern "C" int kvax_mask_build(const int32_t* q_pos, const int32_t* q_seg, const
     j.upper_full = d.upper_full;
     max_outer = max_outer > j.n_outer ? max_outer : j.n_outer;
     max_shards = max_shards > j.num_shards ? max_shards : j.num_shards;
+  }
+  if (max_outer > 0 && q_len <= kFusedTokens && kv_len <= kFusedTokens && max_blocks <= kFusedInner &&
+      max_block_size <= kFusedBlockSize) {
+    FusedParams fp{};
+    fp.bounds = bp;
+    for (int m = 0; m < num_masks; m++) {
+      const SummaryJob &qs = sp.jobs[qk[m]], &ks = sp.jobs[kk[m]];
+      fp.outer[m] = bp.jobs[m].kv_outer ? ks : qs;
+      fp.inner[m] = bp.jobs[m].kv_outer ? qs : ks;
+    }
+    hipLaunchKernelGGL(fused_masks_kernel, dim3(cdiv(max_outer, kFusedOuter), batch, num_masks), dim3(kFusedThreads),
+                       max_blocks * sizeof(int4), stream, fp);
+    return check_launch("fused_masks_kernel");
   }
   if (max_blocks > 0) {
     dim3 grid(cdiv(max_blocks, kWavesPerGroup), batch, num_keys);

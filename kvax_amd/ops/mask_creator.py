@@ -3,7 +3,7 @@
 Host-side mirror of the reference's kvax/ops/mask_creator.py: same function names, arguments,
 defaults and return types (``tuple[AttentionMask, ...]`` of length 1 or 3 whose fields are
 int32 ``[batch, shards, n_outer_blocks]``).  The device work is one call into the C ABI
-(``kvax_mask_build``), which builds all requested masks with two kernel launches.
+(``kvax_mask_build``), which builds all requested masks with one or two kernel launches.
 """
 from __future__ import annotations
 
@@ -80,7 +80,7 @@ def build_masks(
 ) -> list[AttentionMask]:
     """Build one mask per ``(query_block_size, kv_block_size, kv_outer)`` request in one call.
 
-    The host side of a call is kept short (it is most of the call's latency: the two kernels take
+    The host side of a call is kept short (it is most of the call's latency: the kernels take
     under 10 us): one device allocation holds the workspace and every mask, whose tensors are views
     of it."""
     if not 1 <= len(requests) <= _native.KVAX_MAX_MASKS:
