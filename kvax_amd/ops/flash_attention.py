@@ -20,6 +20,7 @@ import ctypes as C
 import torch
 
 from kvax_amd import _native
+from kvax_amd.ops.mask_creator import _raw_stream
 from kvax_amd.utils.common import (
     FlashAttentionParamsConfig,
     get_default_flash_attention_params,
@@ -37,26 +38,40 @@ ACCEPTED_HEAD_DIMS = (16, 32, 64, 128, 192, 256)
 _DTYPES = {torch.bfloat16: _native.KVAX_BF16, torch.float16: _native.KVAX_F16}
 
 
+_Int64x3, _Pointerx4 = C.c_int64 * 3, C.c_void_p * 4
+
+
 def _strides3(t: torch.Tensor):
-    if t.stride(3) != 1:
+    s0, s1, s2, s3 = t.stride()
+    if s3 != 1:
         raise ValueError("the head_dim axis must be contiguous")
-    return (C.c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))
+    return _Int64x3(s0, s1, s2)
 
 
 def _mask_ptrs(mask) -> "C.c_void_p * 4":
     arrays = mask.flatten() if isinstance(mask, AttentionMask) else tuple(mask)
-    out = (C.c_void_p * 4)()
-    for i, a in enumerate(arrays):
+    for a in arrays:
         if a.dtype != torch.int32 or not a.is_contiguous():
             raise ValueError("mask arrays must be contiguous int32")
-        out[i] = a.data_ptr()
-    return out
+    return _Pointerx4(*[a.data_ptr() for a in arrays])
 
 
 def _ids(x: torch.Tensor, name: str, shape) -> torch.Tensor:
-    if tuple(x.shape) != tuple(shape):
+    if x.shape != shape:
         raise ValueError(f"{name} has shape {tuple(x.shape)}, expected {tuple(shape)}")
+    if x.dtype is torch.int32 and x.is_contiguous():
+        return x
     return x.to(torch.int32).contiguous()
+
+
+def _call(fn, args, workspace, device) -> int:
+    """Calls ``fn(args, workspace, bytes, stream)`` on the device's current stream, entering the device
+    only where it is not the current one (the guard and a stream object around the handle are 5 us of a
+    forward call of 38)."""
+    if torch.cuda.current_device() == device.index:
+        return fn(C.byref(args), workspace.data_ptr(), workspace.numel(), _raw_stream(device.index))
+    with torch.cuda.device(device):
+        return fn(C.byref(args), workspace.data_ptr(), workspace.numel(), _raw_stream(device.index))
 
 
 def _check_inputs(query, key, value):
@@ -131,10 +146,7 @@ def flash_attention_forward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, fwd
         _native.check(rc, "kvax_fa_fwd_static")
         return out, lse
     ws = _workspace(lib.kvax_fa_fwd_workspace_bytes(C.byref(a)), query.device)
-    with torch.cuda.device(query.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.kvax_fa_fwd(C.byref(a), ws.data_ptr(), ws.numel(), C.c_void_p(stream))
-    _native.check(rc, "kvax_fa_fwd")
+    _native.check(_call(lib.kvax_fa_fwd, a, ws, query.device), "kvax_fa_fwd")
     return out, lse
 
 
@@ -174,15 +186,13 @@ def flash_attention_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, dq
         raise _native.KvaxNativeError("libkvax_amd.so was built without kvax_fa_bwd")
     if ws is None:
         ws = _workspace(lib.kvax_fa_bwd_workspace_bytes(C.byref(a)), query.device)
-    with torch.cuda.device(query.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.kvax_fa_bwd(C.byref(a), ws.data_ptr(), ws.numel(), C.c_void_p(stream))
-    _native.check(rc, "kvax_fa_bwd")
+    _native.check(_call(lib.kvax_fa_bwd, a, ws, query.device), "kvax_fa_bwd")
     return dq, dk, dv
 
 
 def _contiguous(mask):
-    return tuple(a.contiguous() for a in (mask.flatten() if isinstance(mask, AttentionMask) else mask))
+    arrays = mask.flatten() if isinstance(mask, AttentionMask) else mask
+    return tuple(a if a.is_contiguous() else a.contiguous() for a in arrays)
 
 
 class _FlashAttentionFn(torch.autograd.Function):
