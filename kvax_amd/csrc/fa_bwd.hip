@@ -788,11 +788,13 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
         for (int mt = 0; mt < UNITS; mt++)
 #pragma unroll
           for (int i = 0; i < 16; i++) x[mt][i] = 0.f;
-        // The order is fenced: with scheduling groups instead, the compiler gave up the reads ahead in this
-        // kernel up to head_dim 128 and waited for every operand (dK/dV 2426 -> 2392 us on 32k tokens, 4574
-        // -> 4448 on 4 x 16k short documents, 186 -> 174 on 4k tokens, heads 32/8).
+        // The order is fenced: with scheduling groups instead, the compiler gave up the reads ahead at
+        // head_dim 128 and waited for every operand (dK/dV 2426 -> 2392 us on 32k tokens, 4574 -> 4448 on
+        // 4 x 16k short documents, 186 -> 174 on 4k tokens, heads 32/8).  At 64 it does so, too, but mixes
+        // the short contraction with what is around it, which is better (one document of 16k, heads 16/4:
+        // 1533 against 1620).
 #define KVAX_CONTRACT(n, regs)                                                                                       \
-  {                                                                                                                  \
+  if constexpr (D > 64) {                                                                                            \
     constexpr int N = UNITS * ((n) / 16), kAheadOps = 4;                                                             \
     vec8 op[N];                                                                                                      \
     auto read = [&](int i) {                                                                                         \
@@ -806,7 +808,17 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
       if (i + kAheadOps < N) op[i + kAheadOps] = read(i + kAheadOps);                                                \
       __builtin_amdgcn_sched_barrier(0);                                                                             \
     }                                                                                                                \
-  }
+  } else {                                                                                                           \
+  _Pragma("unroll") for (int ks = 0; ks < (n) / 16; ks++)                                                            \
+      _Pragma("unroll") for (int mt = 0; mt < UNITS; mt++)                                                           \
+          x[mt] = Tr::mfma(*reinterpret_cast<const vec8*>(rows_a + 32 * mt * ((n) * 2) + nat_off[ks % (regs)] +      \
+                                                          ks / (regs) * kGroupBytes<n>), frag[ks], x[mt]);           \
+  __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);                                                                 \
+  _Pragma("unroll") for (int i = 0; i < UNITS * ((n) / 16) - 4; i++) {                                               \
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                               \
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                                                               \
+  }                                                                                                                  \
+  __builtin_amdgcn_sched_group_barrier(0x008, 4, 0); }
         if constexpr (D == DV) {
           KVAX_CONTRACT(D, kNatQ)
         } else if (p_wave) {

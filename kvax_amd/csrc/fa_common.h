@@ -475,9 +475,8 @@ struct AsyncTileCopy {
   // holds the last rows): every row is row limit - 1.
   template <int J0, int J1>
   __device__ __forceinline__ void part(const char* gbase, int row0, int limit, uint32_t tile_addr) const {
-    row0 = min(row0, limit - 1);
-    const char* tile_base = gbase + (int64_t)row0 * stride;
     if (row0 + ROWS <= limit) {  // whole tile in range (uniform): scalar bases + fixed lane offsets
+      const char* tile_base = gbase + (int64_t)row0 * stride;
       const uint32_t lds = tile_addr + wave_u * 1024;
 #pragma unroll
       for (int j = J0; j < J1; j++) {
@@ -489,7 +488,8 @@ struct AsyncTileCopy {
     } else {  // ragged tail: clamp each lane's row (32-bit offsets from the tile's base)
       int l = lane_;
       asm volatile("" : "+v"(l));  // keeps what follows from being computed ahead of a loop around the call
-      const int last = limit - 1 - row0;
+      const int first = min(row0, limit - 1), last = limit - 1 - first;
+      const char* tile_base = gbase + (int64_t)first * stride;
 #pragma unroll
       for (int j = J0; j < J1; j++) {
         const int grp = j * NW + wave_u;
