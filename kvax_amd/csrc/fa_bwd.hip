@@ -97,6 +97,23 @@ __device__ __forceinline__ Range merged_range(const int32_t* const mask[4], int6
   return r;
 }
 
+// A stationary MFMA operand.  PINNED, at one wavefront per SIMD: put into the accumulation registers for
+// good (left to itself the register allocator parks such fragments there, too, but copies them back in
+// front of every use: 100 copies per 32 MFMAs in the dQ kernel at head_dim 256).  8k tokens, heads 16/4 of
+// 256: dQ 387 -> 350 us, dK/dV 769 -> 732; 4k tokens, 16 heads of 192: dQ 122 -> 114.
+template <class Vec8, bool PINNED>
+__device__ __forceinline__ Vec8 operand(uint4 u) {
+  if constexpr (PINNED) {
+    uint32_t a0, a1, a2, a3;
+    asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a0) : "v"(u.x));
+    asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a1) : "v"(u.y));
+    asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a2) : "v"(u.z));
+    asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a3) : "v"(u.w));
+    u = make_uint4(a0, a1, a2, a3);
+  }
+  return __builtin_bit_cast(Vec8, u);
+}
+
 // ---------------------------------------------------------------------------------------------
 // dQ: one work-group = NW wavefronts x 32 query rows of one (batch, head); streams the live K/V
 // tiles through a ring of LDS stages filled by asynchronous copies.
@@ -255,9 +272,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
   if (n_live > 0) {
     vec8 qf[KSTEPS], dof[VSTEPS];
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) qf[ks] = __builtin_bit_cast(vec8, qraw[ks]);
+    for (int ks = 0; ks < KSTEPS; ks++) qf[ks] = operand<vec8, WPS == 1>(qraw[ks]);
 #pragma unroll
-    for (int ks = 0; ks < VSTEPS; ks++) dof[ks] = __builtin_bit_cast(vec8, draw[ks]);
+    for (int ks = 0; ks < VSTEPS; ks++) dof[ks] = operand<vec8, WPS == 1>(draw[ks]);
     int nat_off[kNat], nat_off_v[kNatV], tr_off[kTr][2];
 #pragma unroll
     for (int ks = 0; ks < kNat; ks++) nat_off[ks] = nat_offset<D>(c, ks, h);
@@ -312,22 +329,44 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
           f32x16 s, dp;
 #pragma unroll
           for (int i2 = 0; i2 < 16; i2++) s[i2] = 0.f, dp[i2] = 0.f;
+          // Fenced above head_dim 128, see the dK/dV kernel: at 192 with 128 178 -> 171 us on 2 x 4k tokens, 16
+          // heads.  At 128 the scheduling groups are heeded well enough and the freedom they leave is better:
+          // 1484 us on 32k tokens, heads 32/8, against 1508 fenced.
+          if constexpr (D > 128) {
+            constexpr int N = KSTEPS + VSTEPS, kAheadOps = WPS == 2 && D > 128 ? 3 : 4;
+            vec8 op[N];
+            // operand i: K and V rows in turn while there are both, then K rows
+            auto is_v = [](int i) { return i < 2 * VSTEPS && i % 2 == 1; };
+            auto step = [](int i) { return i < 2 * VSTEPS ? i / 2 : i - VSTEPS; };
+            auto read = [&](int i) {
+              const int ks = step(i);
+              return is_v(i) ? *reinterpret_cast<const vec8*>(vtile + 32 * kt * RBV + nat_off_v[ks % kNatV] + ks / kNatV * kGroupBytes<DV>)
+                             : *reinterpret_cast<const vec8*>(ktile + 32 * kt * RB + nat_off[ks % kNat] + ks / kNat * kGroupBytes<D>);
+            };
 #pragma unroll
-          for (int ks = 0; ks < KSTEPS; ks++) {
-            const vec8 ka = *reinterpret_cast<const vec8*>(ktile + 32 * kt * RB + nat_off[ks % kNat] + ks / kNat * kGroupBytes<D>);
-            s = Tr::mfma(ka, qf[ks], s);
-            if (ks < VSTEPS) {
-              const vec8 va = *reinterpret_cast<const vec8*>(vtile + 32 * kt * RBV + nat_off_v[ks % kNatV] + ks / kNatV * kGroupBytes<DV>);
-              dp = Tr::mfma(va, dof[ks], dp);
+            for (int i = 0; i < kAheadOps; i++) op[i] = read(i);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+              if (is_v(i)) dp = Tr::mfma(op[i], dof[step(i)], dp);
+              else s = Tr::mfma(op[i], qf[step(i)], s);
+              if (i + kAheadOps < N) op[i + kAheadOps] = read(i + kAheadOps);
+              __builtin_amdgcn_sched_barrier(0);
             }
-          }
-          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+          } else {
 #pragma unroll
-          for (int i2 = 0; i2 < KSTEPS + VSTEPS - 4; i2++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            for (int ks = 0; ks < KSTEPS; ks++) {
+              s = Tr::mfma(*reinterpret_cast<const vec8*>(ktile + 32 * kt * RB + nat_off[ks]), qf[ks], s);
+              dp = Tr::mfma(*reinterpret_cast<const vec8*>(vtile + 32 * kt * RBV + nat_off_v[ks]), dof[ks], dp);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+            for (int i2 = 0; i2 < KSTEPS + VSTEPS - 4; i2++) {
+              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+              __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
           }
-          __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
           // K^T operands of this block's dQ update, requested before the element-wise work
           // (with two wavefronts per SIMD above head_dim 128 there are no registers to do that in)
           constexpr bool kLean = WPS == 2 && D > 128;
@@ -608,7 +647,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
         uint4 u = make_uint4(0, 0, 0, 0);
         if (in && (ks < VSTEPS || p_wave)) u = *reinterpret_cast<const uint4*>(base + (16 * ks + 8 * h) * 2);
         u.x ^= sign, u.y ^= sign, u.z ^= sign, u.w ^= sign;
-        frag[ks] = __builtin_bit_cast(vec8, u);
+        frag[ks] = operand<vec8, Cfg::kWps == 1>(u);
       }
     }
     // Operand addresses.  The P wave reads rows of Q and columns of dO, the S wave rows of dO and
