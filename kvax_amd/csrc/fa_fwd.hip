@@ -368,6 +368,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
         const char* ktile = smem + stage * Smem::kStage;
         const int32_t* ids = reinterpret_cast<const int32_t*>(ktile + Smem::kIds);
 
+        [[maybe_unused]] bool raised = false;  // the running maximum, by the first half of the tile
 #pragma unroll 1
         for (int hf = 0; hf < HALVES; hf++) {
         // ---- S^T = K Q^T -----------------------------------------------------------------
@@ -428,8 +429,13 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
           // rescaled: 64 multiplies per lane) only when some row's maximum has grown by more than
           // kRescaleStep, i.e. the exponentials below may reach 2^kRescaleStep instead of 1 - exact
           // in the final O = acc / l and lse = m + log2(l), and no loss for a floating-point P.
-          // With a plain running maximum some of a wavefront's 32 rows raise it in most tiles.
-          if (__any(mx * cs > m_run[qt] + kRescaleStep)) {
+          // With a plain running maximum some of a wavefront's 32 rows raise it in most tiles.  A tile that
+          // is worked on by halves and raises it in the first raises it in the second, too, to the
+          // maximum of the whole tile, the exponential of which is exactly 1: short rows depend on that
+          // (left to the second half's own growth O is 1.6 % further from float64).
+          bool raise = __any(mx * cs > m_run[qt] + kRescaleStep);
+          if constexpr (HALVES == 2) raised = raise = raise || raised;
+          if (raise) {
             const float m_new = fmaxf(m_run[qt], mx * cs);
             const float alpha = fast_exp2(m_run[qt] - m_new);
             l_run[qt] *= alpha;

@@ -77,3 +77,27 @@ def test_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32):
     for name, got, ref in zip(("dq", "dk", "dv"), grads, refs):
         check_close(name, got, ref, rel=OPERAND_ROUNDING)
     assert not grads[0][ids[1] == -1].any() and not grads[1][ids[3] == -1].any() and not grads[2][ids[3] == -1].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_weight_of_the_largest_score_is_exact(device, dtype):
+    """The key with a row's largest score enters with weight 1, which the 16-bit P holds exactly, also where the tile is worked
+    on by halves and the key lies in the second one, with little above the first one's maximum."""
+    b, sq, sk, h, d, top = 3, 640, 64, 32, 256, 41  # eight wavefronts, one tile
+    g = torch.Generator(device=device).manual_seed(3)
+    q, k, v = (torch.randn((b, n, h, d), generator=g, device=device, dtype=dtype) for n in (sq, sk, sk))
+    q *= 0.25
+    q[..., 0] = 4.0
+    k[..., 0] = 0.0
+    k[:, top] = 0.0
+    k[:, top, :, 0] = 8.0  # score 2 for every row; the others are N(0, 1/16)
+    v[:, :top] = v[:, top + 1:] = 0.0
+    ids = [torch.zeros((b, n), dtype=torch.int32, device=device) for n in (sq, sq, sk, sk)]
+    with attention_specs(SPEC, SPEC):
+        out = flash_attention(q, k, v, *ids, create_attention_mask(*ids, fwd_params=P), scale=d ** -0.5, fwd_params=P)
+    scores = [torch.mm(q[i, :, j].double(), k[i, :, j].double().t().contiguous()) * d ** -0.5 for i in range(b) for j in range(h)]
+    assert all((s.argmax(dim=1) == top).all() for s in scores)
+    weights = torch.stack([torch.softmax(s, dim=1)[:, top] for s in scores]).reshape(b, h, sq).transpose(1, 2)
+    ref = (weights[..., None] * v[:, top:top + 1].double()).cpu().numpy()
+    # what remains is the fp32 sum of the weights and the rounding of the result
+    check_close("out", out, ref, atol=1e-5)
