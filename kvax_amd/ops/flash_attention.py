@@ -56,6 +56,22 @@ def _mask_ptrs(mask) -> "C.c_void_p * 4":
     return _Pointerx4(*[a.data_ptr() for a in arrays])
 
 
+def _check_mask(mask, name: str, batch: int, length: int, block: int, shards: int = 1) -> None:
+    """The kernels index a mask by batch row, shard and outer block and cannot see where it ends: a mask
+    made for another number of shards or other lengths is refused here.  (A single row may be longer than
+    the tensors, e.g. the mask of a whole prompt with the first queries of it.)"""
+    rows = batch * shards
+    if rows == 0 or length == 0 or block <= 0:
+        return  # nothing is read, or the library refuses the block size
+    blocks = -(-length // block)
+    for a in mask.flatten() if isinstance(mask, AttentionMask) else mask:
+        if a.shape == (batch, shards, blocks):
+            continue
+        if shards > 1 or (a.numel() < blocks if rows == 1 else a.numel() != rows * blocks):
+            raise ValueError(f"the {name} mask has shape {tuple(a.shape)}, expected {(batch, shards, blocks)}: build it "
+                             "with the block sizes, lengths and mesh of the call")
+
+
 def _ids(x: torch.Tensor, name: str, shape) -> torch.Tensor:
     if x.shape != shape:
         raise ValueError(f"{name} has shape {tuple(x.shape)}, expected {tuple(shape)}")
@@ -129,6 +145,7 @@ def flash_attention_forward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, fwd
     scratch memory is the library's own fixed buffer, shared by all calls on the GPU.  ``flags``:
     ``_native.KVAX_FA_FWD_WIDE`` selects the kernel variant with 64 query rows per wavefront."""
     b, sq, hq, d = query.shape
+    _check_mask(fwd_mask, "forward", b, sq, fwd_params.query_block_size)
     if buffers is not None:
         out, lse = buffers
     else:
@@ -165,6 +182,8 @@ def flash_attention_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, dq
     ``dkdv_fp32`` asks for the kernels' fp32 accumulators (to sum them over devices).  ``dkdv_shards``:
     the query axis holds that many context shards and ``dkdv_mask`` a row of bounds for each."""
     kv_dtype = torch.float32 if dkdv_fp32 else key.dtype
+    _check_mask(dq_mask, "dQ", query.shape[0], query.shape[1], bwd_params.kv_block_size)
+    _check_mask(dkdv_mask, "dK/dV", key.shape[0], key.shape[1], bwd_params.kv_block_size, dkdv_shards)
     if buffers is not None:  # (dq, dk, dv, workspace) reused across calls, e.g. by the benchmark
         dq, dk, dv, ws = buffers
     else:

@@ -3,6 +3,7 @@ shared library loads and exports every symbol the header declares, and the ops r
 without a GPU instead of falling back."""
 import ctypes
 import re
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -10,6 +11,7 @@ import pytest
 import torch
 
 import kvax_amd
+import kvax_amd.ops.flash_attention  # noqa: F401
 from kvax_amd import _native
 from kvax_amd.utils import (
     PADDING_SEGMENT_ID,
@@ -23,7 +25,9 @@ from kvax_amd.utils.common import get_default_flash_attention_params, pad_to_blo
 from kvax_amd.utils.math import get_multi_head_attention_tflops
 from kvax_amd.utils.permutation import generate_shard_indices
 from kvax_amd.utils.specs import get_attention_specs
+from kvax_amd.utils.typing import AttentionMask
 
+flash_attention_module = sys.modules["kvax_amd.ops.flash_attention"]  # (the package exports a function of that name)
 ROOT = Path(__file__).resolve().parent.parent
 CP = (("data", "context", None, None), ("data", None, None, None))
 
@@ -271,3 +275,51 @@ def test_error_strings_are_per_thread():
     for t in threads:
         t.join()
     assert not problems, problems[:3]
+
+
+def _zero_mask(*shape):
+    return AttentionMask(*torch.zeros((4, *shape), dtype=torch.int32).unbind(0))
+
+
+@pytest.mark.parametrize("batch, shards, blocks, given, fine", [
+    (2, 4, 8, (2, 4, 8), True),
+    (2, 4, 8, (2, 1, 8), False),    # built for one device
+    (2, 4, 8, (2, 2, 8), False),    # built for fewer shards
+    (2, 4, 8, (2, 8, 8), False),    # for more
+    (2, 4, 8, (4, 2, 8), False),    # the right size with other rows
+    (2, 4, 8, (2, 4, 7), False),    # shorter keys
+    (1, 4, 8, (1, 1, 32), False),
+    (2, 1, 8, (2, 1, 8), True),
+    (2, 1, 8, (2, 8), True),        # no axis for the one shard
+    (2, 1, 8, (1, 1, 8), False),
+    (2, 1, 8, (2, 1, 9), False),    # rows would be taken from the wrong place
+    (1, 1, 8, (1, 1, 9), True),     # one row that goes on beyond the tensors
+    (1, 1, 8, (1, 1, 7), False),
+])
+def test_masks_of_other_shapes_are_refused_before_the_library_call(batch, shards, blocks, given, fine):
+    """The gradients' entry point under context parallelism, on host tensors: it must not get past the check."""
+    n, block = blocks * 32, 32
+    p = FlashAttentionParamsConfig(block, block)
+    q, k = (torch.zeros((batch, n, 1, 64), dtype=torch.bfloat16) for _ in range(2))
+    ids = [torch.zeros((batch, n), dtype=torch.int32) for _ in range(4)]
+    lse = torch.zeros((batch, 1, n))
+    names = ("dQ", "dK/dV")
+    for which, name in enumerate(names):
+        masks = [_zero_mask(batch, 1, blocks), _zero_mask(batch, shards, blocks)]
+        if which == 0 and shards > 1:
+            continue
+        masks[which] = _zero_mask(*given)
+        if fine:
+            for mask, mask_name, m_shards in zip(masks, names, (1, shards)):
+                flash_attention_module._check_mask(mask, mask_name, batch, n, block, m_shards)
+        else:
+            with pytest.raises(ValueError, match=f"the {name} mask has shape"):
+                flash_attention_module.flash_attention_backward(q, k, k, *ids, *masks, q, lse, q, 1.0, p, p, dkdv_shards=shards)
+            if shards == 1:
+                with pytest.raises(ValueError, match="the forward mask has shape"):
+                    flash_attention_module.flash_attention_forward(q, k, k, *ids, masks[which], 1.0, p, p)
+
+
+@pytest.mark.parametrize("batch, length, block", [(0, 64, 32), (1, 0, 32), (1, 64, 0)])
+def test_masks_that_are_not_read_are_not_checked(batch, length, block):
+    flash_attention_module._check_mask(_zero_mask(3, 1, 5), "forward", batch, length, block)

@@ -3,7 +3,7 @@ permutation kernel."""
 import pytest
 import torch
 
-from kvax_amd import FlashAttentionParamsConfig, Mesh, attention_specs, create_attention_mask
+from kvax_amd import FlashAttentionParamsConfig, Mesh, attention_specs, create_attention_mask, flash_attention
 from kvax_amd.ops.flash_attention import flash_attention_backward, flash_attention_forward
 from kvax_amd.utils.benchmarking import generate_random_segments_lengths, make_random_attention_inputs
 from kvax_amd.utils.permutation import apply_permutation, generate_shard_indices
@@ -50,6 +50,20 @@ def test_shards_in_one_call_equal_shard_by_shard(device, sq, sk, cp, block, head
         assert (a - b).abs().max() <= 2 ** -8 * b.abs().max() and (a - b).norm() <= 1e-3 * b.norm(), name
     if pad:
         assert not got[1][:, sk - pad:].any() and not got[2][:, sk - pad:].any()
+
+
+@pytest.mark.parametrize("built_for", [1, 2, 8])
+def test_masks_of_another_mesh_are_refused(device, built_for):
+    data, scale = make_random_attention_inputs(2, 512, 512, 4, 2, 64, 64, seed=5, device=device)
+    p = FlashAttentionParamsConfig(32, 32)
+    meshes = [Mesh({"data": 1, "context": cp, "model": 1}) for cp in (built_for, 4)]
+    leaf = data[0].requires_grad_(True)
+    with attention_specs(*CP_SPECS):
+        masks = create_attention_mask(*data[3:], fwd_params=p, bwd_params=p, calc_bwd_mask=True, mesh=meshes[0])
+        out = flash_attention(*data, masks, scale=scale, fwd_params=p, bwd_params=p, mesh=meshes[1])
+        with pytest.raises(ValueError, match="the dK/dV mask has shape"):
+            out.backward(torch.ones_like(out))
+    assert leaf.grad is None
 
 
 @pytest.mark.parametrize("shape, chunks, dtype", [
