@@ -31,6 +31,8 @@ def generate_shard_indices(num_shards: int, reverse: bool = False) -> list[int]:
 
 def _permute_on_device(x: torch.Tensor, num_shards: int, reverse: bool) -> torch.Tensor:
     x = x.contiguous()
+    if x.data_ptr() % 4:  # a view may start anywhere in its storage
+        x = x.clone()
     out = torch.empty_like(x)
     chunk_bytes = x.numel() // (x.shape[0] * num_shards) * x.element_size()
     with torch.cuda.device(x.device):

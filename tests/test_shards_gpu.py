@@ -81,3 +81,22 @@ def test_chunk_permutation(device, shape, chunks, dtype):
         leaf, g = x.clone().requires_grad_(True), torch.randn_like(x)
         apply_permutation([leaf], chunks, False)[0].backward(g)
         assert torch.equal(leaf.grad, apply_permutation([g], chunks, True)[0])
+
+
+def _by_index(x, chunks, reverse=False):
+    order = torch.tensor(generate_shard_indices(chunks, reverse), device=x.device)
+    return x.reshape(x.shape[0], chunks, -1).index_select(1, order).reshape(x.shape)
+
+
+@pytest.mark.parametrize("dtype, width", [(torch.bfloat16, 2), (torch.bool, 4), (torch.int8, 4), (torch.float32, 1)])
+def test_chunk_permutation_of_a_view_at_any_offset(device, dtype, width):
+    """A batch of one is contiguous wherever it starts in its storage; so is its gradient."""
+    base = (torch.randn((1, 1 + 8 * width), device=device) * 3).to(dtype)
+    x = base[:, 1:].view(1, 8, width)
+    assert x.is_contiguous() and (x.data_ptr() % 4 or dtype == torch.float32)
+    assert torch.equal(apply_permutation([x], 4, False)[0], _by_index(x, 4))
+    assert torch.equal(apply_permutation([x], 4, True)[0], _by_index(x, 4, True))
+    if dtype.is_floating_point:
+        leaf = torch.randn((1, 8, width), device=device).to(dtype).requires_grad_(True)
+        apply_permutation([leaf], 4, False)[0].backward(x)
+        assert torch.equal(leaf.grad, _by_index(x, 4, True))
