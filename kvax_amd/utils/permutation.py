@@ -30,7 +30,8 @@ def generate_shard_indices(num_shards: int, reverse: bool = False) -> list[int]:
 
 
 def _permute_on_device(x: torch.Tensor, num_shards: int, reverse: bool) -> torch.Tensor:
-    x = x.contiguous()
+    # bytes are copied: a conjugate or a negative must be in memory first
+    x = x.resolve_conj().resolve_neg().contiguous()
     if x.data_ptr() % 4:  # a view may start anywhere in its storage
         x = x.clone()
     out = torch.empty_like(x)

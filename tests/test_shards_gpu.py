@@ -100,3 +100,13 @@ def test_chunk_permutation_of_a_view_at_any_offset(device, dtype, width):
         leaf = torch.randn((1, 8, width), device=device).to(dtype).requires_grad_(True)
         apply_permutation([leaf], 4, False)[0].backward(x)
         assert torch.equal(leaf.grad, _by_index(x, 4, True))
+
+
+def test_chunk_permutation_of_lazily_conjugated_and_negated_tensors(device):
+    x = torch.randn((2, 8, 3), device=device, dtype=torch.complex64)
+    for y in (x.conj(), x.conj().imag):
+        assert y.is_conj() or y.is_neg()
+        assert torch.equal(apply_permutation([y], 4, False)[0], _by_index(y.resolve_conj().resolve_neg(), 4))
+    leaf = x.clone().requires_grad_(True)
+    apply_permutation([leaf], 4, False)[0].backward(x.conj())
+    assert torch.equal(leaf.grad, _by_index(x.conj().resolve_conj(), 4, True))
