@@ -10,6 +10,7 @@ from __future__ import annotations
 from typing import Sequence
 
 import torch
+from torch.autograd import forward_ad
 
 from kvax_amd import _native
 from kvax_amd.utils.sharding import get_query_context_mesh_axis_size
@@ -55,11 +56,23 @@ class _PermuteChunks(torch.autograd.Function):
         return _permute(grad, ctx.num_shards, not ctx.reverse), None, None
 
 
+def _is_plain(x: torch.Tensor) -> bool:
+    """Whether x is memory and nothing else: no subclass, and no transform (vmap, forward-mode, batched
+    gradients) or tracer that has to see the operations applied to it."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    functorch = torch._C._functorch
+    return type(x) in (torch.Tensor, torch.nn.Parameter) and x.layout is torch.strided and not (
+        torch._C._are_functorch_transforms_active() or functorch.is_functorch_wrapped_tensor(x)
+        or functorch.is_legacy_batchedtensor(x) or torch._C._len_torch_dispatch_stack()
+        or x._is_zerotensor() or forward_ad.unpack_dual(x).tangent is not None)
+
+
 def _permute(x: torch.Tensor, num_shards: int, reverse: bool) -> torch.Tensor:
-    """One tensor, permuted by the copy kernel; tensors it does not take (on the host, or in pieces that
-    are not a multiple of 4 bytes) by an index."""
-    if x.is_cuda and x.numel() and x.shape[0] <= 65535 and \
-            x.numel() // (x.shape[0] * num_shards) * x.element_size() % 4 == 0:
+    """One tensor, permuted by the copy kernel; tensors it does not take (on the host, in pieces that are
+    not a multiple of 4 bytes, more than a grid holds, or not plain memory) by an index."""
+    if x.is_cuda and _is_plain(x) and x.numel() and x.shape[0] <= 65535 and num_shards % 2 == 0 and \
+            num_shards <= 65534 and x.numel() // (x.shape[0] * num_shards) * x.element_size() % 4 == 0:
         return _PermuteChunks.apply(x, num_shards, reverse)
     order = generate_shard_indices(num_shards, reverse=reverse)
     idx = torch.as_tensor(order, device=x.device, dtype=torch.long)

@@ -110,3 +110,28 @@ def test_chunk_permutation_of_lazily_conjugated_and_negated_tensors(device):
     leaf = x.clone().requires_grad_(True)
     apply_permutation([leaf], 4, False)[0].backward(x.conj())
     assert torch.equal(leaf.grad, _by_index(x.conj().resolve_conj(), 4, True))
+
+
+def test_chunk_permutation_under_transforms(device):
+    """What an indexed copy composes with: function transforms, forward mode, batched gradients, second derivatives, tracing."""
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    x, t = torch.randn((2, 2, 8, 3), device=device)
+    many = torch.randn((5, 2, 8, 3), device=device)
+    f = lambda y: apply_permutation([y], 4, False)[0]
+    want = torch.stack([_by_index(y, 4) for y in many])
+    assert torch.equal(torch.func.vmap(f)(many), want)
+    assert torch.equal(torch.func.jvp(f, (x,), (t,))[1], _by_index(t, 4))
+    assert torch.equal(torch.func.grad(lambda y: (f(y) * t).sum())(x), _by_index(t, 4, True))
+    with forward_ad.dual_level():
+        assert torch.equal(forward_ad.unpack_dual(f(forward_ad.make_dual(x, t))).tangent, _by_index(t, 4))
+    leaf = x.clone().requires_grad_(True)
+    got = torch.autograd.grad(f(leaf), leaf, many, is_grads_batched=True)[0]
+    assert torch.equal(got, torch.stack([_by_index(y, 4, True) for y in many]))
+    first = torch.autograd.grad((f(leaf) ** 2 * t).sum(), leaf, create_graph=True)[0]
+    second = torch.autograd.grad(first.sum(), leaf)[0]
+    torch.testing.assert_close(second, 2 * _by_index(t, 4, True))
+    assert torch.equal(make_fx(f)(x)(t), _by_index(t, 4))
+    assert torch.equal(torch.compile(f, backend="eager", fullgraph=True)(t), _by_index(t, 4))
+    assert type(f(torch.nn.Parameter(x))) is torch.Tensor
