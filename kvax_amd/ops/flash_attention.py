@@ -48,6 +48,15 @@ def _strides3(t: torch.Tensor):
     return _Int64x3(s0, s1, s2)
 
 
+def _addressable(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or a copy of it where the kernels cannot address it: rows of 16-byte pieces, less than 2^24
+    elements apart."""
+    s0, s1, s2, s3 = t.stride()
+    if s3 == 1 and (s0 | s1 | s2) % 8 == 0 and s1 < 1 << 24 and t.data_ptr() % 16 == 0:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
 def _mask_ptrs(mask) -> "C.c_void_p * 4":
     arrays = mask.flatten() if isinstance(mask, AttentionMask) else tuple(mask)
     for a in arrays:
@@ -249,6 +258,8 @@ class _FlashAttentionFn(torch.autograd.Function):
                 or key.shape[1] % bwd.kv_block_size:
             raise ValueError(
                 "backward needs sequence lengths divisible by the backward block sizes")
+        if query.shape[3] == 192:
+            dout = _addressable(dout)
         dq, dk, dv = flash_attention_backward(
             query, key, value, q_pos, q_seg, kv_pos, kv_seg, _contiguous(masks[1]), _contiguous(masks[2]),
             out, lse, dout, ctx.scale, ctx.fwd_params, bwd, dkdv_shards=cp)
@@ -326,6 +337,8 @@ def flash_attention(
         key = torch.nn.functional.pad(key, (0, run_qk - d_qk))
     if d_v != run_v:
         value = torch.nn.functional.pad(value, (0, run_v - d_v))
+    if run_qk == 192:  # taken with any strides and offset, like the sizes that are padded
+        query, key, value = _addressable(query), _addressable(key), _addressable(value)
     out = _FlashAttentionFn.apply(
         query, key, value, query_positions, query_segment_ids, kv_positions, kv_segment_ids,
         tuple(mask), float(scale), fwd_params, bwd_params, cp)

@@ -101,3 +101,42 @@ def test_weight_of_the_largest_score_is_exact(device, dtype):
     ref = (weights[..., None] * v[:, top:top + 1].double()).cpu().numpy()
     # what remains is the fp32 sum of the weights and the rounding of the result
     check_close("out", out, ref, atol=1e-5)
+
+
+def _odd_rows(t):  # a slice of rows of width + 4
+    return torch.nn.functional.pad(t, (0, 4))[..., :t.shape[3]]
+
+
+def _odd_offset(t):
+    return torch.nn.functional.pad(t.reshape(-1), (1, 0))[1:].view(t.shape)
+
+
+def _columns(t):  # the head_dim axis is not contiguous
+    return t.transpose(2, 3).contiguous().transpose(2, 3)
+
+
+def _expanded(t):  # one row for all
+    return t[:, :1, :1, :1].expand(t.shape)
+
+
+@pytest.mark.parametrize("d, dv", [(192, 128), (192, 192), (64, 192)])
+@pytest.mark.parametrize("view_q, view_k, view_v, view_dout", [
+    (_odd_rows, _odd_rows, _odd_rows, _odd_rows), (_odd_offset,) * 4, (_columns,) * 4,
+    (_odd_rows, _odd_offset, _columns, _expanded),
+])
+def test_any_strides_at_192(device, d, dv, view_q, view_k, view_v, view_dout):
+    """Rows that the kernels cannot address, in the inputs and in the gradient of the output: the same bits as from contiguous
+    tensors."""
+    (q, k, v), ids, scale = _inputs(1, 128, 192, 4, 2, d, dv, 0, 2, device)
+    dout = torch.randn((1, 128, 4, dv), generator=torch.Generator().manual_seed(2)).to(q.dtype).to(device)
+    with attention_specs(SPEC, SPEC):
+        masks = create_attention_mask(*ids, fwd_params=P, bwd_params=P, calc_bwd_mask=True)
+
+        def run(q, k, v, dout):
+            leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+            out = flash_attention(*leaves, *ids, masks, scale=scale, fwd_params=P, bwd_params=P)
+            return out.detach(), *torch.autograd.grad(out, leaves, dout)
+
+        given = [view(t) for view, t in zip((view_q, view_k, view_v, view_dout), (q, k, v, dout))]
+        for got, want in zip(run(*given), run(*(t.contiguous().clone() for t in given))):
+            assert torch.equal(got, want)
