@@ -974,7 +974,8 @@ __global__ __launch_bounds__(256) void fa_fwd_combine_kernel(const FwdParams p, 
     float4 o[kCombineBatch];
 #pragma unroll
     for (int s = 0; s < kCombineBatch; s++) {
-      // parts beyond the last: its values again, with no weight
+      // beyond the last part: its values again, which are set to zero below (with no weight alone an
+      // infinity among them would become NaN)
       const int64_t slot = slot0 + (int64_t)min(s0 + s, p.num_parts - 1) * p.part_rows;
       ml[s] = *reinterpret_cast<const float2*>(p.part_ml + slot * 2);
       o[s] = *reinterpret_cast<const float4*>(p.part_o + slot * D + d);
@@ -988,7 +989,9 @@ __global__ __launch_bounds__(256) void fa_fwd_combine_kernel(const FwdParams p, 
     m = m_new;
 #pragma unroll
     for (int s = 0; s < kCombineBatch; s++) {
-      const float w = s0 + s < p.num_parts && ml[s].y > 0.f ? fast_exp2(ml[s].x - m) : 0.f;
+      const bool in = s0 + s < p.num_parts;
+      o[s] = make_float4(in ? o[s].x : 0.f, in ? o[s].y : 0.f, in ? o[s].z : 0.f, in ? o[s].w : 0.f);
+      const float w = in && ml[s].y > 0.f ? fast_exp2(ml[s].x - m) : 0.f;
       l += ml[s].y * w;
       acc.x += o[s].x * w, acc.y += o[s].y * w, acc.z += o[s].z * w, acc.w += o[s].w * w;
     }

@@ -462,3 +462,23 @@ def test_wide_forward_kernel_restarting_positions(device):
     data = (q, k, v) + w.ids(device)
     out, _ = _forward_with_flags(data, w.scale, 128, True)
     check(out[:1], _sampled_heads_oracle("doc32k", [5, 26]), data[4][:1], heads=[5, 26])
+
+
+@pytest.mark.parametrize("q_len", [1, 40])  # halves of the windows / whole windows as partial results
+@pytest.mark.parametrize("windows", [2, 3, 5, 6, 7])  # the merge takes four results at a time
+def test_split_forward_keeps_an_infinity(device, q_len, windows):
+    """A value that is infinite in every key of the last window: the column is infinite, whatever the number of windows, and
+    the others are what they are without it."""
+    g = torch.Generator(device=device).manual_seed(windows)
+    q = torch.randn((1, q_len, 4, 128), generator=g, device=device, dtype=torch.bfloat16)
+    k, v = (torch.randn((1, 256 * windows, 4, 128), generator=g, device=device, dtype=torch.bfloat16) for _ in range(2))
+    ids = [torch.zeros((1, n), dtype=torch.int32, device=device) for n in (q_len, q_len, 256 * windows, 256 * windows)]
+    p = FlashAttentionParamsConfig(64, 64)
+    with attention_specs(("data", None, "model", None), ("data", None, "model", None)):
+        mask = create_attention_mask(*ids, fwd_params=p)
+        want = flash_attention(q, k, v, *ids, mask, scale=0.1, fwd_params=p)
+        v[:, -256:, :, 5] = float("inf")
+        got = flash_attention(q, k, v, *ids, mask, scale=0.1, fwd_params=p)
+    assert (got[..., 5] == float("inf")).all()
+    got[..., 5] = want[..., 5]
+    assert torch.equal(got, want)
