@@ -134,11 +134,14 @@ __device__ __forceinline__ void write_bounds(const BoundsJob& job, const BoundsP
       }
       const unsigned long long am = __ballot(attend);
       const unsigned long long fm = __ballot(full);
-      if (am) {
+      // Kept behind branches: of the rounds of 64 blocks few hold any to attend, and executed in all of
+      // them the updates are a chain of scalar work (three masks of 8 x 128k tokens in blocks of 64: 91.6
+      // against 85.2 us, with one document per row 96.4 against 91.5).
+      if (__builtin_expect(am != 0, 0)) {
         lower = min(lower, base + (int)__ffsll((long long)am) - 1);
         upper = max(upper, base + 64 - (int)__clzll((long long)am));
       }
-      if (fm) {
+      if (__builtin_expect(fm != 0, 0)) {
         lower_full = min(lower_full, base + (int)__ffsll((long long)fm) - 1);
         upper_full = max(upper_full, base + 64 - (int)__clzll((long long)fm));
       }
