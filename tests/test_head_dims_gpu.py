@@ -35,7 +35,7 @@ def _host(tensors):
     (2, 1, 5000, 8, 2, 192, 192, 0, 1),
     (1, 48, 2000, 16, 4, 192, 128, 0, 1),    # split, two row tiles
     (1, 200, 3001, 4, 2, 192, 192, 0, 1),
-    (2, 640, 640, 32, 32, 192, 128, 60, 4),  # one work-group of eight wavefronts per compute unit, ragged query tile
+    (2, 640, 640, 32, 32, 192, 128, 60, 4),  # work-groups of four wavefronts, ragged query tile
     (2, 520, 1111, 32, 16, 192, 192, 30, 3),
     (2, 640, 640, 32, 32, 256, 256, 60, 4),
     (2, 300, 300, 4, 2, 128, 160, 0, 2),     # padded to 192
@@ -62,7 +62,11 @@ def test_forward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, dtype):
     (1, 1000, 1000, 6, 2, 256, 256, 77, 9, True),
 ])
 def test_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32):
-    (q, k, v), ids, scale = _inputs(b, sq, sk, hq, hkv, d, dv, pad, docs, device)
+    _check_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32, torch.bfloat16)
+
+
+def _check_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32, dtype):
+    (q, k, v), ids, scale = _inputs(b, sq, sk, hq, hkv, d, dv, pad, docs, device, dtype)
     # heads before the sequence in memory, as a caller with [batch, heads, seq, dim] tensors passes them
     q, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, v))
     dout = torch.randn((b, sq, hq, dv), generator=torch.Generator().manual_seed(2)).to(q.dtype).to(device)
@@ -70,13 +74,34 @@ def test_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32):
         masks = create_attention_mask(*ids, fwd_params=P, bwd_params=P, calc_bwd_mask=True)
     out, lse = flash_attention_forward(q, k, v, *ids, masks[0], scale, P, P)
     grads = flash_attention_backward(q, k, v, *ids, masks[1], masks[2], out, lse, dout, scale, P, P, dkdv_fp32=fp32)
-    heads = None if hq < 32 else [1]
+    heads = None if hq < 32 else [1, hq - 1]
     refs = ao.attention_backward(*_host((q, k, v)), *_host(ids), scale, *_host([dout]), dtype=np.float64, heads=heads)
     if heads:
-        grads, refs = ([x[:, :, 1:2] for x in grads], [r[:, :, 1:2] if r.shape[2] > 1 else r for r in refs])
+        grads, refs = ([x[:, :, heads] for x in grads], [r[:, :, heads] for r in refs])
     for name, got, ref in zip(("dq", "dk", "dv"), grads, refs):
         check_close(name, got, ref, rel=OPERAND_ROUNDING)
     assert not grads[0][ids[1] == -1].any() and not grads[1][ids[3] == -1].any() and not grads[2][ids[3] == -1].any()
+
+
+# Work-groups of eight wavefronts: more than 256 of them (3 x 32 heads x 3 tiles of 256 rows, the last one ragged).
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d, dv", [(192, 128), (192, 192), (256, 256)])
+def test_forward_with_eight_wavefronts(device, d, dv, dtype):
+    (q, k, v), ids, scale = _inputs(3, 640, 640, 32, 32, d, dv, 60, 4, device, dtype)
+    with attention_specs(SPEC, SPEC):
+        mask = create_attention_mask(*ids, fwd_params=P)
+    out, lse = flash_attention_forward(q, k, v, *ids, mask[0], scale, P, P)
+    ref, ref_lse = ao.attention_forward(*_host((q, k, v)), *_host(ids), scale)
+    check_close("out", out, ref)
+    # in units of log2; fp32 sums of 256 products of 16-bit numbers of magnitude 1 (256 * 2^-24 * 256 * 0.64 / 16) and of 640 weights
+    np.testing.assert_allclose(lse.cpu().numpy() * np.log(2.0), ref_lse, rtol=0, atol=2e-4)
+    assert not out[ids[1] == -1].any()
+
+
+def test_backward_with_eight_wavefronts_float16(device):
+    _check_backward(device, 3, 640, 640, 32, 32, 192, 128, 60, 4, True, torch.float16)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
