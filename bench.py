@@ -258,7 +258,7 @@ def measure(args, name, block, steps, warmup, device_tensors=False):
     out = torch.empty_like(q)
     lse = torch.empty((w.batch, w.num_heads, w.q_len), dtype=torch.float32, device=dev)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    ws = torch.empty(backward_workspace_bytes(q, k) + 16, dtype=torch.uint8, device=dev)
+    ws = torch.empty(backward_workspace_bytes(q, k, v) + 16, dtype=torch.uint8, device=dev)
     SQ, SK = _native.KVAX_FA_SKIP_DQ, _native.KVAX_FA_SKIP_DKDV
 
     fwd_flags = _native.KVAX_FA_FWD_WIDE if args.fwd_wide else 0

@@ -176,11 +176,15 @@ def flash_attention_forward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, fwd
     return out, lse
 
 
-def backward_workspace_bytes(query, key) -> int:
-    """Size of the scratch buffer ``kvax_fa_bwd`` needs for these shapes (delta + tile summaries)."""
+def backward_workspace_bytes(query, key, value=None) -> int:
+    """Size of the scratch buffer ``kvax_fa_bwd`` needs for these shapes: delta, tile summaries, the
+    dispatch order and, where several work-groups share a dK/dV work item, their fp32 results (up to 101 MB
+    at head_dim 128 and 256, 151 MB at 192).  Without ``value`` its head_dim is taken to be the key's, which is
+    enough for any."""
     a = _native.FaArgs()
     a.batch, a.q_len, a.num_heads = query.shape[0], query.shape[1], query.shape[2]
     a.kv_len, a.num_kv_heads, a.head_dim = key.shape[1], key.shape[2], key.shape[3]
+    a.v_head_dim = 0 if value is None else value.shape[3]
     return int(_native.lib().kvax_fa_bwd_workspace_bytes(C.byref(a)))
 
 

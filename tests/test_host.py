@@ -323,3 +323,10 @@ def test_masks_of_other_shapes_are_refused_before_the_library_call(batch, shards
 @pytest.mark.parametrize("batch, length, block", [(0, 64, 32), (1, 0, 32), (1, 64, 0)])
 def test_masks_that_are_not_read_are_not_checked(batch, length, block):
     flash_attention_module._check_mask(_zero_mask(3, 1, 5), "forward", batch, length, block)
+
+
+def test_backward_workspace_knows_the_value_head_dim():
+    """16 parts of one work item of 128 keys, fp32: the value columns are counted as they are."""
+    q, k, v = (torch.empty((1, n, h, d), device="meta") for n, h, d in ((2048, 8, 192), (128, 1, 192), (128, 1, 128)))
+    sizes = [flash_attention_module.backward_workspace_bytes(q, k, *more) for more in ((), (k,), (v,))]
+    assert sizes[0] == sizes[1] == sizes[2] + 16 * 128 * (192 - 128) * 4
