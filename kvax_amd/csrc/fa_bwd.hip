@@ -629,12 +629,17 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   __syncthreads();
   const int n_live = *live_count;
   // every head of the group walks the same list; this part's share of the (head, list entry) pairs
-  const int pairs = n_live * p.group;
-  const int pair_lo = (int)((int64_t)pairs * member / p.dkdv_parts);
-  const int steps = ((int)((int64_t)pairs * (member + 1) / p.dkdv_parts) - pair_lo) * SUB;
+  // (the divisions are a microsecond of an item: 16 rows of 1k tokens, 16 heads of 64, 184 -> 181 us without)
+  int pair_lo = 0, pair_hi = n_live * p.group, first_head = 0;
+  if (p.dkdv_parts > 1) {
+    pair_lo = (int)((int64_t)(n_live * p.group) * member / p.dkdv_parts);
+    pair_hi = (int)((int64_t)(n_live * p.group) * (member + 1) / p.dkdv_parts);
+    first_head = n_live ? pair_lo / n_live : 0;
+  }
+  const int steps = (pair_hi - pair_lo) * SUB;
 
   if (steps > 0) {
-    const int first_head = pair_lo / n_live, first_li = pair_lo - first_head * n_live;
+    const int first_li = pair_lo - first_head * n_live;
     // stationary fragments: K (negated when the scale is negative) for the P wave, V for the S wave
     // (VSTEPS of them)
     vec8 frag[KSTEPS];
