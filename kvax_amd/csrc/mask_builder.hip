@@ -14,9 +14,9 @@
 //                                    for the "full" predicate); sentinel fix-ups applied in
 //                                    place.
 //
-// Work is O(S + n_outer * n_inner / 64) instead of the reference's O(n_outer * S) re-reads.  Sequences
-// of up to kFusedTokens are done in one launch instead (fused_masks_kernel): the two passes are a launch
-// and a trip to memory each, and nothing else.
+// Work is O(S + n_outer * n_inner / 64) instead of the reference's O(n_outer * S) re-reads.  Short
+// sequences in few blocks (kFusedTokens, kFusedBlocks) are done in one launch instead
+// (fused_masks_kernel): the two passes are a launch and a trip to memory each, and nothing else.
 #include "common.h"
 
 namespace kvax {
@@ -176,12 +176,14 @@ __global__ __launch_bounds__(kWave* kWavesPerGroup) void block_bounds_kernel(Bou
 // row and mask, and kFusedOuter outer blocks, into LDS, and then works out their bounds.  The ids are read
 // once per work-group instead of once, which costs less than the second launch and trip to memory while
 // they are few.  16 lanes share a block, each with up to eight of its tokens in flight, so that four lane
-// exchanges per value reduce four blocks at once.  us in the kernels, two launches against one, 128-token
-// blocks: three masks of 2k tokens 7.4 / 4.8, one mask of 4 rows of 2k keys 7.3 / 4.1, three masks of 2 x
-// 8k 7.3 / 8.1, of 32k 7.4 / 15.7.
+// exchanges per value reduce four blocks at once.  us in the kernels of three masks, two launches / one: 2k
+// tokens in blocks of 128 7.5 / 4.8, 4k 7.6 / 5.7, 8 rows of 4k 8.0 / 6.3, in blocks of 64 7.7 / 8.0, of 512
+// 8.1 / 8.6, of 32 (128 blocks, the line) 7.7 / 9.9; the host launches once, so that a call takes 16.5
+// instead of 18.8 all the same.  Beyond the lines 2 x 8k 7.3 / 8.1, 32k 7.4 / 15.7, 4k in blocks of 16 7.8 /
+// 13.6, of 4 12.7 / 41, 2k in blocks of 1 21 / 73.
 constexpr int kFusedTokens = 4096;
 constexpr int kFusedOuter = 64;
-constexpr int kFusedInner = 2048;  // summaries that fit the LDS of a work-group
+constexpr int kFusedBlocks = 128;  // each 64 of them are one more round of the work-group
 constexpr int kFusedBlockSize = 512;  // beyond, 16 lanes are too few for a block
 constexpr int kFusedThreads = 1024;
 struct FusedParams {
@@ -393,7 +395,7 @@ extern "C" int kvax_mask_build(const int32_t* q_pos, const int32_t* q_seg, const
     max_outer = max_outer > j.n_outer ? max_outer : j.n_outer;
     max_shards = max_shards > j.num_shards ? max_shards : j.num_shards;
   }
-  if (max_outer > 0 && q_len <= kFusedTokens && kv_len <= kFusedTokens && max_blocks <= kFusedInner &&
+  if (max_outer > 0 && q_len <= kFusedTokens && kv_len <= kFusedTokens && max_blocks <= kFusedBlocks &&
       max_block_size <= kFusedBlockSize) {
     FusedParams fp{};
     fp.bounds = bp;

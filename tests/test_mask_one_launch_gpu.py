@@ -1,5 +1,5 @@
 """The mask builder's one-launch kernel and the line to the two-launch pair: edges of its groups of 16 lanes, of 64
-outer blocks, of the summaries' room and of the lengths, block sizes that are no multiple of 16, and query shards,
+outer blocks, of the number of blocks and of the lengths, block sizes that are no multiple of 16, and query shards,
 bit for bit against the oracle."""
 import numpy as np
 import pytest
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("sq, sk, qbs, kbs, batch, shards", [
     (1, 1, 1, 1, 1, 1), (17, 15, 16, 16, 3, 1), (1000, 333, 48, 100, 2, 1), (1040, 4096, 16, 128, 2, 1),
-    (2048, 2048, 1, 1, 1, 1), (2049, 2048, 1, 16, 1, 1),    # as many blocks as there is room for, and one more
+    (2048, 2048, 16, 16, 2, 1), (2048, 2049, 16, 16, 1, 1), (128, 128, 1, 1, 2, 1), (129, 128, 1, 1, 1, 1),  # 128 blocks, and one more
+    (2048, 2048, 1, 1, 1, 1), (2049, 2048, 1, 16, 1, 1),
     (3000, 4000, 512, 512, 2, 1), (3000, 4000, 513, 129, 2, 1),
     (4096, 4096, 128, 128, 1, 1), (4096, 4097, 128, 128, 1, 1), (1, 4096, 128, 64, 4, 1),
     (4096, 3072, 64, 128, 2, 8), (32768, 32768, 128, 128, 1, 4),
