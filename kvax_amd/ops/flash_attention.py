@@ -74,9 +74,11 @@ def _check_mask(mask, name: str, batch: int, length: int, block: int, shards: in
         return  # nothing is read, or the library refuses the block size
     blocks = -(-length // block)
     for a in mask.flatten() if isinstance(mask, AttentionMask) else mask:
-        if a.shape == (batch, shards, blocks):
-            continue
-        if shards > 1 or (a.numel() < blocks if rows == 1 else a.numel() != rows * blocks):
+        if shards > 1:
+            fits = a.shape == (batch, shards, blocks)
+        else:
+            fits = a.numel() == rows * blocks or rows == 1 and a.numel() > blocks
+        if not fits:
             raise ValueError(f"the {name} mask has shape {tuple(a.shape)}, expected {(batch, shards, blocks)}: build it "
                              "with the block sizes, lengths and mesh of the call")
 
