@@ -236,7 +236,7 @@ def measure(args, name, block, steps, warmup, device_tensors=False):
         torch.cuda.synchronize()
         mask_ms = m0.elapsed_time(m1) / reps
         # the same calls without the host in the way: `reps` of them captured in one HIP graph (kernels
-        # only, no memset nodes) and replayed, which leaves the device time of a call's two kernels
+        # only, no memset nodes) and replayed, which leaves the device time of a call's kernels
         mask_gpu_ms = None
         try:
             graph = torch.cuda.CUDAGraph()

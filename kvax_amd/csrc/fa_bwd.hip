@@ -98,9 +98,11 @@ __device__ __forceinline__ Range merged_range(const int32_t* const mask[4], int6
 }
 
 // A stationary MFMA operand.  PINNED, at one wavefront per SIMD: put into the accumulation registers for
-// good (left to itself the register allocator parks such fragments there, too, but copies them back in
-// front of every use: 100 copies per 32 MFMAs in the dQ kernel at head_dim 256).  8k tokens, heads 16/4 of
-// 256: dQ 387 -> 350 us, dK/dV 769 -> 732; 4k tokens, 16 heads of 192: dQ 122 -> 114.
+// good (left to itself the register allocator parks such fragments there, too, and copies them back for
+// their use: 36 copies per 32 MFMAs in the dQ kernel at head_dim 256, 16 per 16 in dK/dV, none at 192).  8k
+// tokens, heads 16/4 of 256, without / with it in turn on one machine: dQ 409 / 398 us, dK/dV 828 / 798; dQ
+// at 192 equal.  Nothing looks into inline asm for the two wait states between such a write and an MFMA
+// that reads it: the loops that do lie behind a barrier.
 template <class Vec8, bool PINNED>
 __device__ __forceinline__ Vec8 operand(uint4 u) {
   if constexpr (PINNED) {
@@ -1140,8 +1142,8 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
       DqSmem<D, DV, kStagesSmall>::kTotal + live_tiles_bytes(4, p.n_kv_tiles) <= kLdsHalfCu;
   // dK/dV runs one long work-group per compute unit: its light work items are dispatched last, by
   // decreasing number of live tiles, so that the launch does not end on a few long ones.  With no more
-  // items (parts included) than compute units all start at once and the order decides nothing: a training
-  // step of 2k tokens, heads 8/2 of 64, takes 114 us instead of 121 without the 6 us launch.
+  // items (parts included) than compute units all start at once and the order decides nothing: a launch of
+  // 6 us less (2k tokens, heads 8/2 of 64).
   {
     const int items = cdiv(p.kv_len, Cfg::kKvRows);
     if (run_dkdv && items >= kMinOrderedItems && items <= kMaxOrderedItems &&

@@ -947,8 +947,8 @@ __global__ __launch_bounds__(256, 1) void fa_fwd_wide_kernel(const FwdParams p) 
 // dealt to its groups of D / 4 threads and the groups' results merged through LDS; for calls with few
 // rows and many parts (decoding), where a thread that walks all parts makes the call wait.  One
 // work-group per row with one element per thread, as it was, against this: 512 queries against 24k keys
-// (16384 rows x 4 parts) 21.7 -> 8.0 us, 64 rows x 128 parts (one row of 64k keys) 22.5 -> 4.9, 256 x 16
-// (8 rows of 32k keys) 5.3 -> 4.3.
+// (16384 rows x 4 parts) 21.7 -> 8.2 us, 64 rows x 128 parts (one row of 64k keys) 22.5 -> 5.2, 256 x 16
+// (8 rows of 32k keys) 5.3 -> 4.5.
 constexpr int kCombineBatch = 4;
 template <class Tr, int D, bool SPREAD>
 __global__ __launch_bounds__(256) void fa_fwd_combine_kernel(const FwdParams p, int tile_rows, int total_rows) {
@@ -1160,8 +1160,8 @@ int launch_fwd_auto(const FwdParams& p, hipStream_t stream) {
     // Two stages leave no room for a second work-group on a compute unit: eight wavefronts, two per SIMD,
     // where more work-groups than compute units remain and their bookkeeping fits, else four.  us, eight /
     // four wavefronts, 16 heads, at 192 with 128: 2 x 4k tokens 140 / 144, 6k 210 / 245, 16k (documents of
-    // 4k) 515 / 657; 4k 132 / 110, 2k 71 / 52; at 256: 6k 322 / 476, 16k 774 / 1214; 4k 201 / 206, 3k 151 /
-    // 143.
+    // 4k) 515 / 657; 4k 132 / 110, 2k 71 / 52; at 256: 6k 342 / 479, 16k 806 / 1178; 4k 218 / 222, 3k 169 /
+    // 155.
     if (narrow) return launch_fwd<Tr, D, DV, 1, 4, 1, 2, true, true>(p, stream);
     if (p.split_mode) return launch_fwd<Tr, D, DV, 1, 4, 1, 2, true>(p, stream);
     const bool fills = (int64_t)p.batch * p.num_heads * cdiv(p.q_len, 256) > kNumCus;

@@ -2,8 +2,8 @@
 
 The reference checks its context-parallel path against its tensor-parallel one
 (tests/test_attention.py:520-828): queries (and K/V) permuted for load balance, sharded along the
-sequence, must give the same result as the unsharded run once un-permuted.  Here the shards run
-one after another on the single GPU; the expectations are the same, plus the dense oracle.
+sequence, must give the same result as the unsharded run once un-permuted.  Here the shards
+share each call on the single GPU; the expectations are the same, plus the dense oracle.
 """
 import numpy as np
 import pytest
