@@ -107,6 +107,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   // 32-key halves of a tile per wavefront that are worked on together, and one after the other: at
   // head_dim 256 with two wavefronts per SIMD the registers hold the scores of one half at a time
   constexpr int HALVES = D == 256 && WPS == 2 ? 2 : 1;
+  static_assert(HALVES == 1 || MQ == 1, "`raised` below is that of one set of rows");
   constexpr int KT = NARROW || HALVES == 2 ? 1 : 2;
   constexpr int DTO = NARROW ? DT / 2 : DT;  // 32-row slices of O^T per wavefront
   extern __shared__ __attribute__((aligned(16))) char smem[];
