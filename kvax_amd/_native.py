@@ -108,6 +108,26 @@ def lib() -> C.CDLL:
     return l
 
 
+_host = None
+
+
+def host():
+    """The extension module with the host side of the calls, bound to the library's functions."""
+    global _host
+    if _host is None:
+        l = lib()
+        try:
+            from kvax_amd import _host as module
+        except ImportError as e:
+            raise KvaxNativeError(
+                f"kvax_amd._host cannot be imported ({e}): run `python -m kvax_amd.csrc.build`") from e
+        module.bind(*[C.cast(f, C.c_void_p).value for f in (
+            l.kvax_fa_fwd_workspace_bytes, l.kvax_fa_fwd, l.kvax_fa_bwd_workspace_bytes, l.kvax_fa_bwd,
+            l.kvax_mask_workspace_bytes, l.kvax_mask_build)])
+        _host = module
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = lib().kvax_last_error().decode(errors="replace")

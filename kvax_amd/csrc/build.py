@@ -17,6 +17,8 @@ ROOT = PKG.parent
 LIB = PKG / "libkvax_amd.so"
 OBJ = CSRC / "build"
 
+HOST = PKG / "_host.so"  # host.cpp: the host side of the calls, a Python extension module
+
 SOURCES = ["abi.cpp", "mask_builder.hip", "fa_tiles.hip", "permute.hip", "fa_fwd.hip", "fa_bwd.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -45,6 +47,23 @@ def _compile(src: str, extra: list[str]) -> Path:
     return out
 
 
+def _compile_host() -> Path:
+    """The extension module ``kvax_amd._host``: plain C++ against torch's headers and libraries."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{ROOT / 'include'}", f"-isystem{root / 'include'}", f"-isystem{root / 'include/torch/csrc/api/include'}",
+           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host.cpp"), "-o", str(HOST),
+           f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{r.stderr}")
+    return HOST
+
+
 def build(extra_flags: list[str] | None = None, jobs: int = 4, lib: Path | None = None) -> Path:
     """Compile and link; ``lib`` overrides the output path (used for experimental variants,
     loaded by pointing the KVAX_AMD_LIB environment variable at them)."""
@@ -55,7 +74,10 @@ def build(extra_flags: list[str] | None = None, jobs: int = 4, lib: Path | None 
     extra = list(extra_flags or [])
     sources = [s for s in SOURCES if (CSRC / s).exists()]
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_compile_host) if lib is None else None
         objs = list(ex.map(lambda s: _compile(s, extra), sources))
+        if host is not None:
+            host.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

@@ -20,7 +20,7 @@ import ctypes as C
 import torch
 
 from kvax_amd import _native
-from kvax_amd.ops.mask_creator import _raw_stream
+from kvax_amd.ops.mask_creator import _current_device, _raw_stream
 from kvax_amd.utils.common import (
     FlashAttentionParamsConfig,
     get_default_flash_attention_params,
@@ -224,6 +224,10 @@ def flash_attention_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, dq
     return dq, dk, dv
 
 
+def _arrays(mask):
+    return mask.flatten() if isinstance(mask, AttentionMask) else mask
+
+
 def _contiguous(mask):
     arrays = mask.flatten() if isinstance(mask, AttentionMask) else mask
     return tuple(a if a.is_contiguous() else a.contiguous() for a in arrays)
@@ -238,6 +242,20 @@ class _FlashAttentionFn(torch.autograd.Function):
                 bwd_params, cp):
         b, sq = query.shape[:2]
         sk = key.shape[1]
+        if cp == 1 or sq % cp == 0 and sq // cp % fwd_params.query_block_size == 0:
+            # the plain case in native code; None: nothing done, something is to be converted or refused
+            index = _current_device()
+            done = _native.host().forward(
+                query, key, value, q_pos, q_seg, kv_pos, kv_seg, _arrays(masks[0]), scale,
+                fwd_params.query_block_size, fwd_params.kv_block_size, bwd_params.query_block_size,
+                bwd_params.kv_block_size, index, _raw_stream(index))
+            if done is not None:
+                out, lse, rc = done
+                _native.check(rc, "kvax_fa_fwd")
+                ctx.save_for_backward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, out, lse)
+                ctx.masks, ctx.scale, ctx.cp = masks, scale, cp
+                ctx.fwd_params, ctx.bwd_params = fwd_params, bwd_params
+                return out
         q_pos, q_seg = _ids(q_pos, "query_positions", (b, sq)), _ids(q_seg, "query_segment_ids", (b, sq))
         kv_pos, kv_seg = _ids(kv_pos, "kv_positions", (b, sk)), _ids(kv_seg, "kv_segment_ids", (b, sk))
         if sq % cp:
@@ -266,6 +284,15 @@ class _FlashAttentionFn(torch.autograd.Function):
                 "backward needs sequence lengths divisible by the backward block sizes")
         if query.shape[3] == 192:
             dout = _addressable(dout)
+        index = _current_device()
+        done = _native.host().backward(
+            query, key, value, q_pos, q_seg, kv_pos, kv_seg, _arrays(masks[1]), _arrays(masks[2]), out, lse, dout,
+            ctx.scale, ctx.fwd_params.query_block_size, ctx.fwd_params.kv_block_size, bwd.query_block_size,
+            bwd.kv_block_size, cp, index, _raw_stream(index))
+        if done is not None:
+            dq, dk, dv, rc = done
+            _native.check(rc, "kvax_fa_bwd")
+            return (dq, dk, dv) + (None,) * 9
         dq, dk, dv = flash_attention_backward(
             query, key, value, q_pos, q_seg, kv_pos, kv_seg, _contiguous(masks[1]), _contiguous(masks[2]),
             out, lse, dout, ctx.scale, ctx.fwd_params, bwd, dkdv_shards=cp)

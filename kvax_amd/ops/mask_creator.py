@@ -45,6 +45,12 @@ except AttributeError:  # pragma: no cover - older or newer torch without the pr
         return torch.cuda.current_stream(index).cuda_stream
 
 
+try:
+    _current_device = torch._C._cuda_getDevice
+except AttributeError:  # pragma: no cover - a torch without GPU support
+    _current_device = torch.cuda.current_device
+
+
 def _layout(lib, batch, q_len, kv_len, requests, num_q_shards):
     """Where the masks of a call lie in its one allocation (in int32 words after the workspace), and
     the workspace size; a function of the shapes and block sizes, remembered per distinct call."""
@@ -85,6 +91,16 @@ def build_masks(
     of it."""
     if not 1 <= len(requests) <= _native.KVAX_MAX_MASKS:
         raise ValueError(f"between 1 and {_native.KVAX_MAX_MASKS} masks per call")
+    if query_positions.is_cuda:
+        # the plain case in native code; None: nothing done, something is to be converted or refused
+        index = _current_device()
+        done = _native.host().masks(
+            query_positions, query_segment_ids, kv_positions, kv_segment_ids, tuple(requests),
+            1 if skip_pad_tokens else 0, num_q_shards, index, _raw_stream(index))
+        if done is not None:
+            rc, arrays = done
+            _native.check(rc, "kvax_mask_build")
+            return [AttentionMask(*arrays[i:i + 4]) for i in range(0, len(arrays), 4)]
     q_pos = _as_ids(query_positions, "query_positions")
     q_seg = _as_ids(query_segment_ids, "query_segment_ids")
     kv_pos = _as_ids(kv_positions, "kv_positions")

@@ -1,0 +1,108 @@
+"""The host side of the calls in native code (kvax_amd/csrc/host.cpp): the plain case gives what the general path in Python
+gives, bit for bit, and everything else is left to that path."""
+import pytest
+import torch
+
+from kvax_amd import FlashAttentionParamsConfig, Mesh, _native, attention_specs, create_attention_mask, flash_attention
+
+ONE = (("data", None, "model", None), ("data", None, "model", None))
+CP = (("data", "context", None, None), ("data", None, None, None))
+
+
+class _Spy:
+    """The native module; `taken` counts the calls it took, with `off` it takes none."""
+
+    def __init__(self, real, off):
+        self.real, self.off, self.taken = real, off, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            done = None if self.off else getattr(self.real, name)(*args)
+            if done is not None:
+                self.taken.append(name)
+            return done
+        return call
+
+
+def test_what_is_not_on_the_gpu_is_left_alone():
+    host = _native.host()
+    ids = torch.zeros((1, 64), dtype=torch.int32)
+    x = torch.zeros((1, 64, 2, 64), dtype=torch.bfloat16)
+    mask = (torch.zeros((1, 1, 1), dtype=torch.int32),) * 4
+    assert host.masks(ids, ids, ids, ids, ((64, 64, False),), 1, 1, 0, 0) is None
+    assert host.forward(x, x, x, ids, ids, ids, ids, mask, 1.0, 64, 64, 64, 64, 0, 0) is None
+    assert host.backward(x, x, x, ids, ids, ids, ids, mask, mask, x, x, x, 1.0, 64, 64, 64, 64, 1, 0, 0) is None
+    for bad in (None, 3, "x"):
+        assert host.masks(bad, ids, ids, ids, ((64, 64, False),), 1, 1, 0, 0) is None
+        assert host.forward(bad, x, x, ids, ids, ids, ids, mask, 1.0, 64, 64, 64, 64, 0, 0) is None
+    with pytest.raises(TypeError):
+        host.forward(x)
+
+
+# name -> (batch, q_len, kv_len, heads, kv heads, head_dim, value head_dim, shards, forward, backward in native code)
+CASES = {
+    "plain": (2, 192, 192, 4, 2, 64, 64, 1, True, True),
+    "one_row": (1, 128, 128, 4, 4, 128, 128, 1, True, True),
+    "values_narrower": (1, 128, 128, 4, 2, 192, 128, 1, True, True),
+    "ragged_forward": (3, 77, 130, 4, 1, 128, 128, 1, True, None),
+    "shards": (1, 256, 256, 4, 2, 128, 128, 2, True, True),
+    "transposed_views": (2, 128, 128, 4, 2, 64, 64, 1, True, True),
+    "int64_ids": (2, 128, 128, 4, 2, 64, 64, 1, False, True),
+    "ids_not_contiguous": (2, 128, 128, 4, 2, 64, 64, 1, False, True),
+    "mask_not_contiguous": (2, 128, 128, 4, 2, 64, 64, 1, False, False),
+    "gradient_expanded": (1, 128, 128, 4, 2, 64, 64, 1, True, False),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", CASES)
+def test_same_bits_as_the_general_path(name, monkeypatch):
+    b, sq, sk, hq, hkv, d, dv, cp, fwd_native, bwd_native = CASES[name]
+    g = torch.Generator(device="cuda").manual_seed(1)
+    draw = lambda *s: torch.randn(s, generator=g, device="cuda", dtype=torch.bfloat16)
+    q, k, v = draw(b, sq, hq, d), draw(b, sk, hkv, d), draw(b, sk, hkv, dv)
+    if name == "transposed_views":
+        q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
+    dout = torch.ones((), device="cuda", dtype=torch.bfloat16).expand(b, sq, hq, dv) if name == "gradient_expanded" else draw(b, sq, hq, dv)
+    ids = []
+    for n in (sq, sk):
+        pos = torch.arange(n, device="cuda", dtype=torch.int32).expand(b, n).contiguous()
+        ids += [pos, (pos >= 50).int() - (pos >= n - 5).int() * 2]  # two documents and padding
+    if name == "int64_ids":
+        ids = [x.long() for x in ids]
+    if name == "ids_not_contiguous":
+        ids = [torch.stack([x, x], 2)[..., 0] for x in ids]
+    params = FlashAttentionParamsConfig(query_block_size=64, kv_block_size=64)
+    mesh = Mesh({"data": 1, "context": cp, "model": 1}) if cp > 1 else None
+    real = _native.host()
+
+    def run(spy):
+        monkeypatch.setattr(_native, "host", lambda: spy)
+        with attention_specs(*(CP if cp > 1 else ONE)):
+            masks = create_attention_mask(*ids, fwd_params=params, bwd_params=params, calc_bwd_mask=True, mesh=mesh)
+            arrays = [a for m in masks for a in m.flatten()]
+            if name == "mask_not_contiguous":
+                masks = tuple(type(m)(*[torch.stack([a, a], -1)[..., 0] for a in m.flatten()]) for m in masks)
+            x = [t.detach().requires_grad_(True) for t in (q, k, v)]
+            out = flash_attention(*x, *ids, masks, scale=d ** -0.5, fwd_params=params, bwd_params=params, mesh=mesh)
+            grads = torch.autograd.grad(out, x, dout) if bwd_native is not None else []
+        return arrays + [out.detach(), *grads]
+
+    spy = _Spy(real, off=False)
+    got, want = run(spy), run(_Spy(real, off=True))
+    assert ("forward" in spy.taken) == fwd_native and ("backward" in spy.taken) == bool(bwd_native)
+    for a, e in zip(got, want):
+        assert a.shape == e.shape and a.stride() == e.stride() and a.dtype == e.dtype and torch.equal(a, e)
+
+
+@pytest.mark.gpu
+def test_errors_of_the_library_reach_the_caller():
+    q = torch.zeros((1, 64, 2, 68), device="cuda", dtype=torch.bfloat16)[..., :64]  # rows not of 16-byte pieces
+    ids = torch.zeros((1, 64), device="cuda", dtype=torch.int32)
+    params = FlashAttentionParamsConfig(query_block_size=64, kv_block_size=64)
+    with attention_specs(*ONE):
+        mask = create_attention_mask(ids, ids, ids, ids, fwd_params=params)
+        with pytest.raises(_native.KvaxNativeError, match="multiples of 8"):
+            flash_attention(q, q, q, ids, ids, ids, ids, mask, fwd_params=params, bwd_params=params)
+
+
