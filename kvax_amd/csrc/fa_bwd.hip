@@ -71,24 +71,27 @@ struct BwdParams {
   float scale, scale_log2;
   float scale_log2_abs;  // |scale| * log2(e) > 0, used with K negated when the scale is negative
   uint32_t k_sign;       // 0x80008000 when the scale is negative
+  int dq_head_shift;     // log2 of the heads per dQ work-group (see heads_shift)
 };
 
 // ---------------------------------------------------------------------------------------------
 // Merged range of the streamed axis for a work-group that covers several mask blocks of the
-// stationary axis: union of [lower, upper), intersection of [lower_full, upper_full), in elements.
+// stationary axis: union of [lower, upper) over the blocks that are its `own`, intersection of [lower_full, upper_full)
+// over all of [blk0, blk1], in elements.
 // ---------------------------------------------------------------------------------------------
 struct Range {
   int lo, hi, flo, fhi;
 };
 
+template <class Own>
 __device__ __forceinline__ Range merged_range(const int32_t* const mask[4], int64_t base, int blk0,
-                                              int blk1, int unit, int limit) {
+                                              int blk1, int unit, int limit, Own own) {
   Range r{0x7fffffff, 0, 0, 0x7fffffff};
   for (int blk = blk0; blk <= blk1; blk++) {
     const int l_ = mask[0][base + blk] * unit, u_ = mask[1][base + blk] * unit;
     r.flo = max(r.flo, mask[2][base + blk] * unit);
     r.fhi = min(r.fhi, mask[3][base + blk] * unit);
-    if (u_ > l_) {
+    if (u_ > l_ && own(blk)) {
       r.lo = min(r.lo, l_);
       r.hi = max(r.hi, u_);
     }
@@ -148,13 +151,20 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
   const int c = lane % 32, h = lane / 32;
 
   int group, rank, g;
-  const ItemMap items{p.batch * p.num_kv_heads, p.num_tiles, p.group};
+  const int head_shift = kHeadsPerWorkGroup<D> ? p.dq_head_shift : 0;
+  const ItemMap items{p.batch * p.num_kv_heads, p.num_tiles, p.group >> head_shift};
   if (!items.decode(blockIdx.x, group, rank, g)) return;
   const int kv_head = group % p.num_kv_heads;
   const int b = group / p.num_kv_heads;
   const int q_tile = p.num_tiles - 1 - rank;
-  const int head = kv_head * p.group + g;
-  const int q0 = q_tile * TQ;
+  // rows of a work-group per head, the wavefront's head among those of the work-group and its block of rows
+  const int TR = TQ >> head_shift;
+  static_assert(NW == 4 || NW == 8, "wavefronts are dealt to heads by shifts");
+  const int wave_shift = (NW == 8 ? 3 : 2) - head_shift;
+  const int row_block = kHeadsPerWorkGroup<D> ? wave & ((1 << wave_shift) - 1) : wave;
+  const int head0 = kv_head * p.group + (g << head_shift);
+  const int head = kHeadsPerWorkGroup<D> ? head0 + (wave >> wave_shift) : head0;
+  const int q0 = q_tile * TR;
 
   const int32_t* kv_seg = p.kv_seg + (int64_t)b * p.kv_len;
   const int32_t* kv_pos = p.kv_pos + (int64_t)b * p.kv_len;
@@ -163,8 +173,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
 
   const int qbs = p.bk, kbs = p.bq;  // the dQ mask swaps the backward block sizes
   const int64_t mbase = (int64_t)b * p.n_dq_blocks;
-  const Range r = merged_range(p.dq_mask, mbase, q0 / qbs,
-                               min((q0 + TQ - 1) / qbs, p.n_dq_blocks - 1), kbs, p.kv_len);
+  // (the full ranges over TQ rows whatever the rows per head: see the forward)
+  const Range r = merged_range(p.dq_mask, mbase, q0 / TQ * TQ / qbs, min((q0 / TQ * TQ + TQ - 1) / qbs, p.n_dq_blocks - 1),
+                               kbs, p.kv_len, [&](int blk) { return blk >= q0 / qbs && blk <= (q0 + TR - 1) / qbs; });
   const int t_lo = r.lo / kTile;
   const int t_hi = r.hi > r.lo ? (r.hi + kTile - 1) / kTile : t_lo;
   const int tf_lo = (r.flo + kTile - 1) / kTile, tf_hi = r.fhi / kTile;
@@ -173,20 +184,22 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
     // No row of the tile can attend to anything (padding queries): zeros for dQ and delta, and
     // nothing is read.  Whole rows, 16 bytes per lane.
     constexpr int kChunks = D * 2 / 16;
-    const int rows = min(TQ, p.q_len - q0);
-    char* dq0 = p.dq + ((int64_t)b * p.dq_sb + (int64_t)head * p.dq_sh) * 2;
-    for (int i = tid; i < rows * kChunks; i += NW * 64)
-      *reinterpret_cast<uint4*>(dq0 + (int64_t)(q0 + i / kChunks) * p.dq_ss * 2 + (i % kChunks) * 16) =
-          make_uint4(0, 0, 0, 0);
-    for (int i = tid; i < rows; i += NW * 64)
-      p.delta[((int64_t)b * p.num_heads + head) * p.q_len + q0 + i] = 0.f;
+    const int rows = min(TR, p.q_len - q0);
+    for (int hd = head0; hd < head0 + (1 << head_shift); hd++) {
+      char* dq0 = p.dq + ((int64_t)b * p.dq_sb + (int64_t)hd * p.dq_sh) * 2;
+      for (int i = tid; i < rows * kChunks; i += NW * 64)
+        *reinterpret_cast<uint4*>(dq0 + (int64_t)(q0 + i / kChunks) * p.dq_ss * 2 + (i % kChunks) * 16) =
+            make_uint4(0, 0, 0, 0);
+      for (int i = tid; i < rows; i += NW * 64)
+        p.delta[((int64_t)b * p.num_heads + hd) * p.q_len + q0 + i] = 0.f;
+    }
     return;
   }
 
   // per-lane query column.  Its ids, its row of the block mask and lse are read without waiting
   // for one another (index 0 stands in for rows beyond the sequence), as are dO, O, Q and the first
   // 64 tile summaries below: one trip to memory for the whole prologue instead of several in a row.
-  const int qrow = q0 + wave * 32 + c;
+  const int qrow = q0 + row_block * 32 + c;
   const bool in = qrow < p.q_len;
   const int qi = in ? qrow : 0;
   const int qseg_raw = p.q_seg[(int64_t)b * p.q_len + qi];
@@ -449,7 +462,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
       for (int i = 0; i < 32 * kChunks; i += 64) {
         const int row = (i + lane) / kChunks, chunk = (i + lane) % kChunks;
         const uint4 v = *reinterpret_cast<const uint4*>(stage + row * kRowBytes + ((chunk ^ (row & kSwz)) * 16));
-        const int qr = q0 + wave * 32 + row;
+        const int qr = q0 + row_block * 32 + row;
         if (qr < p.q_len) *reinterpret_cast<uint4*>(dq0 + (int64_t)qr * p.dq_ss * 2 + pass * kRowBytes + chunk * 16) = v;
       }
     }
@@ -599,7 +612,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   const int q_first = shard * p.shard_rows;
   const int64_t mbase = ((int64_t)b * p.num_shards + shard) * p.n_kv_blocks;
   const Range r = merged_range(p.dkdv_mask, mbase, k0 / kbs,
-                               min((k0 + TKV - 1) / kbs, p.n_kv_blocks - 1), qbs, p.shard_rows);
+                               min((k0 + TKV - 1) / kbs, p.n_kv_blocks - 1), qbs, p.shard_rows, [](int) { return true; });
   if (r.hi <= r.lo) continue;
   const int t_lo = (q_first + r.lo) / kTile;
   const int t_hi = (q_first + r.hi + kTile - 1) / kTile;
@@ -1107,8 +1120,9 @@ int launch_dq(BwdParams p, hipStream_t stream) {
   constexpr int kLimit = kLdsPerCu / (4 * WPS / NW);  // work-groups per compute unit share the LDS
   const int smem = DqSmem<D, DV, STAGES>::kTotal + live_tiles_bytes(NW, p.n_kv_tiles);
   if (int rc = reserve_lds(kernel, smem, kLimit, &done, "the dQ kernel")) return rc;
-  p.num_tiles = cdiv(p.q_len, NW * 32);
-  p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, p.group}.grid();
+  p.dq_head_shift = kHeadsPerWorkGroup<D> ? heads_shift(p.group, NW) : 0;
+  p.num_tiles = cdiv(p.q_len, NW * 32 >> p.dq_head_shift);
+  p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, p.group >> p.dq_head_shift}.grid();
   hipLaunchKernelGGL(kernel, dim3(p.total_items), dim3(NW * 64), smem, stream, p);
   return check_launch("fa_bwd_dq_kernel");
 }

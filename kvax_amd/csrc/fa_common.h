@@ -177,6 +177,23 @@ struct ItemMap {
 };
 
 
+// The wavefronts of a forward or dQ work-group take 32 rows each: as many heads of the GQA group as there are wavefronts
+// (2^shift of them, where they divide the group), and 32-row blocks of the same heads for the rest.  The heads share the
+// key tiles and the mask, so with a head per wavefront all of them have the same live tiles and none waits at the
+// barrier of a tile that is live for others only, as with 128 rows of one head (us, 128 rows of one head -> this): 4 x 16k tokens
+// in bidirectional documents of 512, heads 64/8, forward 2404 -> 2296, dQ 3168 -> 3032; 32k in causal ones of 2k, 32/8,
+// 1154 -> 1135, 1554 -> 1531; 2 x 8k in blocks of 64, documents of 300, 189 -> 174, 259 -> 235; 8 x 1k, 101 -> 95, 144 -> 131.
+// Nothing on one long document or with one head per group.
+// At head_dim 256 it does not pay: the forward spills 2 registers more (8k tokens, heads 16/4: 236 -> 253 us), dQ
+// is equal on documents and 1.4 % slower on one long one.
+template <int D>
+constexpr bool kHeadsPerWorkGroup = D <= 192;
+inline int heads_shift(int group, int waves) {
+  int shift = 0;
+  while (group % (2 << shift) == 0 && (2 << shift) <= waves) shift++;
+  return shift;
+}
+
 // Item queues of a launch whose work-groups stay on their compute units and take work items until
 // none is left, instead of one work-group per item: the dK/dV kernel, whose items are long and take
 // a whole compute unit.  (Within an XCD the hardware hands the work-groups of a launch to the four

@@ -67,6 +67,7 @@ struct FwdParams {
   int part_rows;              // rows per tile that have a partial (<= TQ)
   float* part_o;              // [items, num_parts, part_rows, D] unnormalised O
   float* part_ml;             // [items, num_parts, part_rows, 2] running max (base 2) and sum
+  int head_shift;             // log2 of the heads per work-group (see heads_shift), not in split mode
 };
 
 template <int D, int DV, int STAGES>
@@ -117,6 +118,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   const int c = lane % 32, h = lane / 32;
   const int kt0 = NARROW ? (wave & 1) : 0, dt0 = NARROW ? (wave >> 1) * DTO : 0;
 
+  const int head_shift = SPLIT || !kHeadsPerWorkGroup<D> ? 0 : p.head_shift;
   // ---- work item: heads of a GQA group adjacent, long (late) query tiles first -------------
   int group, rank, g = 0, split = 0, item = 0;
   if (SPLIT) {
@@ -133,14 +135,20 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
     item = group * p.num_q_tiles + tile;
     rank = p.num_q_tiles - 1 - tile;
   } else {
-    const ItemMap items{p.batch * p.num_kv_heads, p.num_q_tiles, p.group};
+    const ItemMap items{p.batch * p.num_kv_heads, p.num_q_tiles, p.group >> head_shift};
     if (!items.decode(blockIdx.x, group, rank, g)) return;
   }
   const int q_tile = p.num_q_tiles - 1 - rank;
   const int kv_head = group % p.num_kv_heads;
   const int b = group / p.num_kv_heads;
-  const int head = kv_head * p.group + g;  // split mode: first head of the group
-  const int q0 = q_tile * TQ;              // split mode: in (query, head) pairs
+  // rows of a work-group per head, the wavefront's head among those of the work-group and its block of rows
+  const int TR = TQ >> head_shift;
+  static_assert(NW == 4 || NW == 8, "wavefronts are dealt to heads by shifts");
+  const int wave_shift = (NW == 8 ? 3 : 2) - head_shift;
+  const int row_block = kHeadsPerWorkGroup<D> ? wave & ((1 << wave_shift) - 1) : wave;
+  const int head0 = kv_head * p.group + (g << head_shift);  // the work-group's first head
+  const int head = kHeadsPerWorkGroup<D> ? head0 + (wave >> wave_shift) : head0;  // split mode: first head of the group
+  const int q0 = q_tile * TR;                               // split mode: in (query, head) pairs
   const int rows_total = SPLIT ? p.q_len * p.group : p.q_len;
 
   const int32_t* q_seg = p.q_seg + (int64_t)b * p.q_len;
@@ -157,14 +165,17 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   // query blocks it covers, intersection of the full ranges (element units) ---------------------
   int lo = 0x7fffffff, hi = 0, flo = 0, fhi = 0x7fffffff;
   {
-    const int qb0 = (SPLIT ? q0 / p.group : q0) / p.qbs;
-    const int qb1 = min((SPLIT ? (q0 + TQ - 1) / p.group : q0 + TQ - 1) / p.qbs, p.n_qblocks - 1);
-    for (int qb = qb0; qb <= qb1; qb++) {
+    // The full ranges are intersected over TQ rows whatever the rows per head: ids that come back after another id (which
+    // the entry point excludes) make the mask claim too much, and what used to be right there stays right.
+    const int first = SPLIT ? q0 / p.group : q0, last = SPLIT ? (q0 + TQ - 1) / p.group : q0 + TR - 1;
+    const int window = SPLIT ? first : q0 / TQ * TQ;
+    const int qb1 = min((SPLIT ? last : window + TQ - 1) / p.qbs, p.n_qblocks - 1);
+    for (int qb = window / p.qbs; qb <= qb1; qb++) {
       const int64_t mi = (int64_t)b * p.n_qblocks + qb;
       const int l_ = p.lower[mi] * p.kbs, u_ = p.upper[mi] * p.kbs;
       flo = max(flo, p.lower_full[mi] * p.kbs);
       fhi = min(fhi, p.upper_full[mi] * p.kbs);
-      if (u_ > l_) {
+      if (u_ > l_ && qb >= first / p.qbs && qb <= last / p.qbs) {
         lo = min(lo, l_);
         hi = max(hi, u_);
       }
@@ -183,11 +194,13 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
     // No row of the tile can attend to anything (padding queries): zeros for O and lse, and nothing
     // is read.  Whole rows, 16 bytes per lane.
     constexpr int kChunks = DV * 2 / 16;
-    const int rows = min(TQ, p.q_len - q0);
-    for (int i = tid; i < rows * kChunks; i += NW * 64)
-      *reinterpret_cast<uint4*>(obase + (int64_t)(q0 + i / kChunks) * p.o_ss * 2 + (i % kChunks) * 16) =
-          make_uint4(0, 0, 0, 0);
-    for (int i = tid; i < rows; i += NW * 64) lse[q0 + i] = 0.f;
+    const int rows = min(TR, p.q_len - q0);
+    for (int hd = head0; hd < head0 + (1 << head_shift); hd++) {
+      char* o = p.out + ((int64_t)b * p.o_sb + (int64_t)hd * p.o_sh) * 2;
+      for (int i = tid; i < rows * kChunks; i += NW * 64)
+        *reinterpret_cast<uint4*>(o + (int64_t)(q0 + i / kChunks) * p.o_ss * 2 + (i % kChunks) * 16) = make_uint4(0, 0, 0, 0);
+      for (int i = tid; i < rows; i += NW * 64) p.lse[((int64_t)b * p.num_heads + hd) * p.q_len + q0 + i] = 0.f;
+    }
     return;
   }
 
@@ -204,7 +217,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   int lower_raw[MQ], upper_raw[MQ];
 #pragma unroll
   for (int qt = 0; qt < MQ; qt++) {
-    const int row = q0 + (NARROW ? qt : wave * MQ + qt) * 32 + c;
+    const int row = q0 + (NARROW ? qt : row_block * MQ + qt) * 32 + c;
     row_in[qt] = row < rows_total;
     qrow[qt] = SPLIT ? row / p.group : row;
     lane_head[qt] = SPLIT ? head + row % p.group : head;
@@ -553,7 +566,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
     for (int i = 0; i < 32 * kChunks; i += 64) {
       const int row = (i + lane) / kChunks, chunk = (i + lane) % kChunks;
       const uint4 v = *reinterpret_cast<const uint4*>(stage + row * kRowBytes + ((chunk ^ (row & kSwz)) * 16));
-      const int qr = q0 + wave * 32 + row;
+      const int qr = q0 + row_block * 32 + row;
       if (qr < p.q_len) *reinterpret_cast<uint4*>(obase + (int64_t)qr * p.o_ss * 2 + chunk * 16) = v;
     }
     return;
@@ -1108,8 +1121,10 @@ int launch_fwd(const FwdParams& p0, hipStream_t stream) {
     p.total_items = p.batch * p.num_kv_heads * p.num_q_tiles * p.num_splits;
   } else {
     p.num_splits = p.num_parts = 1;
-    p.num_q_tiles = cdiv(p.q_len, TQ);
-    p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_q_tiles, p.group}.grid();
+    static_assert(SPLIT || MQ == 1, "the wavefronts of a head hold 32 rows each");
+    p.head_shift = kHeadsPerWorkGroup<D> ? heads_shift(p.group, NW) : 0;
+    p.num_q_tiles = cdiv(p.q_len, TQ >> p.head_shift);
+    p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_q_tiles, p.group >> p.head_shift}.grid();
   }
   if (p.batch * p.num_heads * p.num_q_tiles == 0) return KVAX_OK;
   auto kernel = fa_fwd_kernel<Tr, D, DV, MQ, NW, WPS, STAGES, SPLIT, NARROW>;

@@ -65,6 +65,31 @@ def test_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32):
     _check_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32, torch.bfloat16)
 
 
+# Work-groups of the forward and of dQ take one, two, four or eight heads of a group (the largest power of two that divides it
+# and is no more than the wavefronts): every group size with a remainder, rows that end inside a 32-row block, whole tiles of
+# padding.  (dK and dV come from a kernel that does not know of it.)
+@pytest.mark.parametrize("group", [1, 2, 3, 4, 6, 8, 16])
+@pytest.mark.parametrize("n, d, dv", [(173, 64, 64), (173, 128, 128), (173, 192, 128), (397, 192, 128)])
+def test_heads_of_a_group_share_a_work_group(device, group, n, d, dv):
+    hkv = 2
+    batch = -(-320 // (hkv * group * -(-n // 256)))  # so many that eight wavefronts run, and the key sequence is not divided
+    (q, k, v), ids, scale = _inputs(batch, n, n, hkv * group, hkv, d, dv, 44, 3, device)
+    dout = torch.randn((batch, n, hkv * group, dv), generator=torch.Generator().manual_seed(2)).to(q.dtype).to(device)
+    with attention_specs(SPEC, SPEC):
+        masks = create_attention_mask(*ids, fwd_params=P, bwd_params=P, calc_bwd_mask=True)
+    out, lse = flash_attention_forward(q, k, v, *ids, masks[0], scale, P, P)
+    dq = flash_attention_backward(q, k, v, *ids, masks[1], masks[2], out, lse, dout, scale, P, P)[0]
+    rows = [0, batch - 1]
+    q, k, v, dout, out, dq = (t[rows] for t in (q, k, v, dout, out, dq))
+    ids = [t[rows] for t in ids]
+    heads = sorted({0, hkv * group // 2 - 1, hkv * group // 2, hkv * group - 1})
+    ref, _ = ao.attention_forward(*_host((q, k, v)), *_host(ids), scale)
+    check_close("out", out, ref)
+    ref = ao.attention_backward(*_host((q, k, v)), *_host(ids), scale, *_host([dout]), dtype=np.float64, heads=heads)[0]
+    check_close("dq", dq[:, :, heads], ref[:, :, heads], rel=OPERAND_ROUNDING)
+    assert not out[ids[1] == -1].any() and not dq[ids[1] == -1].any()
+
+
 def _check_backward(device, b, sq, sk, hq, hkv, d, dv, pad, docs, fp32, dtype):
     (q, k, v), ids, scale = _inputs(b, sq, sk, hq, hkv, d, dv, pad, docs, device, dtype)
     # heads before the sequence in memory, as a caller with [batch, heads, seq, dim] tensors passes them
