@@ -62,9 +62,10 @@ struct TileSummaryJob {
   void* out;  // int4 [batch, cdiv(len, kTileRows), 2]
   int len;
 };
-// `zero` (optional): `batch` + kQueueCounters int32 counters the kernel clears: the arrival counters
-// of a following launch_tile_order() and the item queues of the dK/dV kernel (one per XCD).
-constexpr int kQueueCounters = 8;
+// `zero` (optional): `batch` + kQueueCounters + kOrderStats int32 counters the kernel clears: the arrival
+// counters of a following launch_tile_order(), the item queues of the dK/dV kernel (one per XCD) and the
+// ordering pass's sum and maximum of the items' work over all batch rows.
+constexpr int kQueueCounters = 8, kOrderStats = 2;
 int launch_tile_summaries(const TileSummaryJob* jobs, int num_jobs, int batch, hipStream_t stream,
                           int32_t* zero = nullptr);
 inline size_t tile_summary_bytes(int batch, int len) {
@@ -111,8 +112,8 @@ constexpr size_t kMaxTileListBytes = (size_t)KVAX_MAX_TILE_LIST_MB << 20;
 // work (ties: lower index first), so that the launch ends on short items; entries of items whose
 // work is zero carry the flag kDeadItem.  One launch; `ws` holds
 // the order (the result, int32 [batch, n_items], at the start), then the work counts, one
-// arrival counter per batch row and kQueueCounters item counters for the kernel that consumes the
-// order, all of which launch_tile_summaries() must have zeroed (pass it tile_order_counters(ws, ...)).
+// arrival counter per batch row, kQueueCounters item counters for the kernel that consumes the
+// order and the sum and the maximum of the work counts of all batch rows (kOrderStats), all of which launch_tile_summaries() must have zeroed (pass it tile_order_counters(ws, ...)).
 constexpr int kDeadItem = 1 << 30;  // flag on an entry of the order: the item's work count is zero
 struct TileOrderJob {
   const void* own;   // summaries of the items' sequence, int4 [batch, n_own, 2]
@@ -120,10 +121,11 @@ struct TileOrderJob {
   int32_t* ws;       // tile_order_bytes(batch, n_items)
   int n_own, n_opp, sub, n_items;
   int own_is_query;  // the items are query rows or key rows
+  int want_stats;    // also the sum and the maximum over all batch rows
 };
 int launch_tile_order(const TileOrderJob& job, int batch, hipStream_t stream);
 inline size_t tile_order_bytes(int batch, int n_items) {
-  return (((size_t)batch * (2 * n_items + 1) + kQueueCounters) * sizeof(int32_t) + 15) / 16 * 16;
+  return (((size_t)batch * (2 * n_items + 1) + kQueueCounters + kOrderStats) * sizeof(int32_t) + 15) / 16 * 16;
 }
 inline int32_t* tile_order_counters(int32_t* ws, int batch, int n_items) {
   return ws + (size_t)batch * 2 * n_items;

@@ -71,6 +71,12 @@ struct BwdParams {
   float scale, scale_log2;
   float scale_log2_abs;  // |scale| * log2(e) > 0, used with K negated when the scale is negative
   uint32_t k_sign;       // 0x80008000 when the scale is negative
+  // Where the device decides whether work items are shared (see kDecides): the ordering pass's sum and maximum of the
+  // items' work, and what dk, dv, their strides and dkdv_f32 are without parts; else null.
+  const int32_t* work_stats;
+  char *whole_dk, *whole_dv;
+  int64_t whole_dk_sb, whole_dk_ss, whole_dk_sh, whole_dv_sb, whole_dv_ss, whole_dv_sh;
+  int whole_f32;
   int dq_head_shift;     // log2 of the heads per dQ work-group (see heads_shift)
 };
 
@@ -174,8 +180,10 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_bwd_dq_kernel(const BwdParams
   const int qbs = p.bk, kbs = p.bq;  // the dQ mask swaps the backward block sizes
   const int64_t mbase = (int64_t)b * p.n_dq_blocks;
   // (the full ranges over TQ rows whatever the rows per head: see the forward)
-  const Range r = merged_range(p.dq_mask, mbase, q0 / TQ * TQ / qbs, min((q0 / TQ * TQ + TQ - 1) / qbs, p.n_dq_blocks - 1),
-                               kbs, p.kv_len, [&](int blk) { return blk >= q0 / qbs && blk <= (q0 + TR - 1) / qbs; });
+  const int blk0 = q0 / TQ * TQ / qbs, blk1 = min((q0 / TQ * TQ + TQ - 1) / qbs, p.n_dq_blocks - 1);
+  int own0 = blk0, own1 = blk1;
+  if (head_shift > 0) own0 = q0 / qbs, own1 = (q0 + TR - 1) / qbs;
+  const Range r = merged_range(p.dq_mask, mbase, blk0, blk1, kbs, p.kv_len, [&](int blk) { return blk >= own0 && blk <= own1; });
   const int t_lo = r.lo / kTile;
   const int t_hi = r.hi > r.lo ? (r.hi + kTile - 1) / kTile : t_lo;
   const int tf_lo = (r.flo + kTile - 1) / kTile, tf_hi = r.fhi / kTile;
@@ -500,6 +508,19 @@ struct DkdvCfg {
 };
 inline int dkdv_kv_rows(int head_dim) { return head_dim > 192 ? 64 : 128; }
 
+// At head_dim 256 items are 64 rows, and whether two work-groups should share each of 257 to 512 of them depends on the
+// documents, so the device decides, from the work the ordering pass has counted: where the longest item is 15 % longer
+// than a compute unit's share of the work.  dK/dV kernel and sum, us, items whole -> as decided: 8k tokens in documents of 2k,
+// heads 16/4 (longest item 232 steps, share 178) 789 -> 629; 16k in documents of 3k, 8/2, 1119 -> 732; 2 x 4k in documents
+// of 700, 16/4, 516 -> 400.  Left whole (whole / in two parts): one document of 8k, 16/4, 1278 / 1327; of 16k, 8/2, 2564 / 2633;
+// 4k bidirectional, 32/8, 1234 / 1300.  A sum kernel that finds nothing to add takes 3 us.
+template <int D>
+constexpr bool kDecides = D == 256;
+// stats: sum and maximum of the items' work (in tiles, the same for every kv head and query head)
+__device__ __forceinline__ bool shares_items(const int32_t* stats, int num_kv_heads) {
+  return (int64_t)stats[1] * kNumCus * 20 > (int64_t)stats[0] * num_kv_heads * 23;
+}
+
 template <int D, int DV>
 struct DkdvSmem {
   using Cfg = DkdvCfg<D>;
@@ -549,8 +570,11 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   // batch row and kv head) from the queues (see ItemQueue) until none is left.  The ticket for the
   // next item is drawn when the current one's step loop has ended, so that its latency hides behind
   // the final stores and an item is never held back by a long one.
-  const ItemMap items{p.batch * p.num_kv_heads, p.num_tiles, p.dkdv_parts};
-  ItemQueue work{p.dkdv_queue, p.total_items, (int)(blockIdx.x % 8)};  // thread 0's
+  const bool whole = kDecides<D> && p.work_stats && !shares_items(p.work_stats, p.num_kv_heads);
+  auto parts = [&] { return whole ? 1 : p.dkdv_parts; };
+  const ItemMap items{p.batch * p.num_kv_heads, p.num_tiles, parts()};
+  ItemQueue work{p.dkdv_queue, kDecides<D> ? items.grid() : p.total_items, (int)(blockIdx.x % 8)};  // thread 0's
+  auto dkdv_f32 = [&] { return whole ? p.whole_f32 : p.dkdv_f32; };
   int* next_item = reinterpret_cast<int*>(smem + Smem::kTotal) + 1;
   if (tid == 0) *next_item = work.resolve(work.draw());
   __syncthreads();
@@ -561,8 +585,8 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   // queries under a causal mask)
   int group, rank, member;  // member: which part of the item's steps
   if (items.decode(item, group, rank, member)) {
-  char* const dk_out = p.dk + member * p.dk_part;
-  char* const dv_out = p.dv + member * p.dv_part;
+  char* const dk_out = whole ? p.whole_dk : p.dk + member * p.dk_part;
+  char* const dv_out = whole ? p.whole_dv : p.dv + member * p.dv_part;
   const int kv_head = group % p.num_kv_heads;
   const int b = group / p.num_kv_heads;
   const int entry = p.dkdv_order ? p.dkdv_order[(int64_t)b * p.num_tiles + rank] : rank;
@@ -571,7 +595,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   if (entry & kDeadItem) {
     // no query tile can interact with these kv rows (known from the ordering pass): zeros, no bookkeeping
     if (tid == 0) ticket = work.draw();
-    const int esize = p.dkdv_f32 ? 4 : 2;
+    const int esize = dkdv_f32() ? 4 : 2;
     const int rows = min(TKV, p.kv_len - k0);
     auto zero_rows = [&](char* out, int64_t sb, int64_t sh, int64_t ss, int columns) {
       const int chunks = columns * esize / 16;
@@ -579,8 +603,13 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
         *reinterpret_cast<uint4*>(out + ((int64_t)b * sb + (int64_t)kv_head * sh + (int64_t)(k0 + i / chunks) * ss) * esize +
                                   (i % chunks) * 16) = make_uint4(0, 0, 0, 0);
     };
-    zero_rows(dk_out, p.dk_sb, p.dk_sh, p.dk_ss, D);
-    zero_rows(dv_out, p.dv_sb, p.dv_sh, p.dv_ss, DV);
+    if (whole) {
+      zero_rows(dk_out, p.whole_dk_sb, p.whole_dk_sh, p.whole_dk_ss, D);
+      zero_rows(dv_out, p.whole_dv_sb, p.whole_dv_sh, p.whole_dv_ss, DV);
+    } else {
+      zero_rows(dk_out, p.dk_sb, p.dk_sh, p.dk_ss, D);
+      zero_rows(dv_out, p.dv_sb, p.dv_sh, p.dv_ss, DV);
+    }
   } else {
 
   const int kbs = p.bk, qbs = p.bq;
@@ -646,9 +675,9 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   // every head of the group walks the same list; this part's share of the (head, list entry) pairs
   // (the divisions are a microsecond of an item: 16 rows of 1k tokens, 16 heads of 64, 184 -> 181 us without)
   int pair_lo = 0, pair_hi = n_live * p.group, first_head = 0;
-  if (p.dkdv_parts > 1) {
-    pair_lo = (int)((int64_t)(n_live * p.group) * member / p.dkdv_parts);
-    pair_hi = (int)((int64_t)(n_live * p.group) * (member + 1) / p.dkdv_parts);
+  if (parts() > 1) {
+    pair_lo = (int)((int64_t)(n_live * p.group) * member / parts());
+    pair_hi = (int)((int64_t)(n_live * p.group) * (member + 1) / parts());
     first_head = n_live ? pair_lo / n_live : 0;
   }
   const int steps = (pair_hi - pair_lo) * SUB;
@@ -986,10 +1015,15 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     // (padding keys, dead: exact zeros, see the dQ kernel's epilogue)
     const float mul = p_wave ? 1.f : p.scale;
     char* base = p_wave ? dv_out : dk_out;
-    const int64_t sb = p_wave ? p.dv_sb : p.dk_sb, sh = p_wave ? p.dv_sh : p.dk_sh, ss = p_wave ? p.dv_ss : p.dk_ss;
+    int64_t sb = p_wave ? p.dv_sb : p.dk_sb, sh = p_wave ? p.dv_sh : p.dk_sh, ss = p_wave ? p.dv_ss : p.dk_ss;
+    if (whole) {
+      sb = p_wave ? p.whole_dv_sb : p.whole_dk_sb;
+      sh = p_wave ? p.whole_dv_sh : p.whole_dk_sh;
+      ss = p_wave ? p.whole_dv_ss : p.whole_dk_ss;
+    }
     constexpr int PC = D % 128 == 0 && DV % 128 == 0 ? 128 : 64;  // columns per pass
     constexpr int kDtPerPass = PC / 32;
-    const int esize = p.dkdv_f32 ? 4 : 2;
+    const int esize = dkdv_f32() ? 4 : 2;
     const int row_bytes = PC * esize;             // 128, 256 or 512
     const int chunks = row_bytes / 16;            // 8, 16 or 32 per row
     char* stage = smem + wave * (32 * PC * 4);    // room for the fp32 case
@@ -999,7 +1033,7 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
     for (int pass = 0; pass < D / PC; pass++) {
       if (D != DV && p_wave && pass >= DV / PC) break;
       char* mine = stage + c * row_bytes;
-      if (p.dkdv_f32) {
+      if (dkdv_f32()) {
 #pragma unroll
         for (int d = 0; d < kDtPerPass; d++)
 #pragma unroll
@@ -1053,13 +1087,15 @@ struct DkdvSumParams {
   int pieces[2];          // and of one of its rows
   int num_parts, kv_len, num_kv_heads;
   int f32;
+  const int32_t* work_stats;  // null, or as in BwdParams: nothing to add where no items are shared
 };
 
 template <class Tr>
 __global__ __launch_bounds__(256) void dkdv_sum_kernel(const DkdvSumParams p) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int which = blockIdx.y;
-  if (i >= p.total[which]) return;
+  if (p.work_stats && !shares_items(p.work_stats, p.num_kv_heads)) return;
+  // (one round, but for launches that may have nothing to do)
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.total[which]; i += (int64_t)gridDim.x * 256) {
   const float4* src = reinterpret_cast<const float4*>(p.parts[which]) + i;
   float4 sum = src[0];
 #pragma unroll 4
@@ -1076,6 +1112,7 @@ __global__ __launch_bounds__(256) void dkdv_sum_kernel(const DkdvSumParams p) {
     *reinterpret_cast<float4*>(p.dst[which] + at * 4) = sum;
   else
     *reinterpret_cast<uint2*>(p.dst[which] + at * 2) = make_uint2(Tr::pack2(sum.x, sum.y), Tr::pack2(sum.z, sum.w));
+  }
 }
 
 // How many work-groups share the steps of a dK/dV work item.  A launch with fewer items than compute
@@ -1102,6 +1139,14 @@ int plan_dkdv_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_
   const int64_t one_round = min(kNumCus / items, steps / 8), two_rounds = min(2 * kNumCus / items, steps / 24),
                 three_rounds = min(3 * kNumCus / items, steps / 128);
   return (int)max(min(max(max(one_round, two_rounds), three_rounds), (int64_t)16), (int64_t)1);
+}
+
+// Whether the device decides between one part and two (see kDecides): the order is computed for such launches.
+bool device_decides_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int head_dim) {
+  if (!kDecides<256> || head_dim != 256 || plan_dkdv_parts(batch, q_len, kv_len, num_heads, num_kv_heads, head_dim) > 1) return false;
+  const int tiles = cdiv(kv_len, dkdv_kv_rows(head_dim));
+  const int64_t items = (int64_t)batch * num_kv_heads * tiles;
+  return items > kNumCus && items <= 2 * kNumCus && tiles >= kMinOrderedItems && tiles <= kMaxOrderedItems;
 }
 
 template <class K>
@@ -1164,10 +1209,11 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
         (int64_t)items * p.batch * p.num_kv_heads * p.dkdv_parts > kNumCus &&
         (int64_t)items * (p.n_q_tiles + 2) < 0x7fffffff) {
       const TileOrderJob job{p.kv_tiles, p.q_tiles, p.order_ws, p.n_kv_tiles, p.n_q_tiles,
-                             Cfg::kKvRows / kTileRows, items, 0};
+                             Cfg::kKvRows / kTileRows, items, 0, p.work_stats != nullptr};
       if (int rc = launch_tile_order(job, p.batch, stream)) return rc;
       p.dkdv_order = p.order_ws;
     }
+    if (!p.dkdv_order) p.work_stats = nullptr;
   }
   if (run_dq) {
     if constexpr (D == 256) {
@@ -1210,6 +1256,14 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
     p.num_tiles = cdiv(p.kv_len, Cfg::kKvRows);
     p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, p.dkdv_parts}.grid();
     DkdvSumParams sum{};
+    if (p.work_stats) {
+      p.dkdv_parts = 2;
+      p.whole_dk = p.dk, p.whole_dk_sb = p.dk_sb, p.whole_dk_ss = p.dk_ss, p.whole_dk_sh = p.dk_sh;
+      p.whole_dv = p.dv, p.whole_dv_sb = p.dv_sb, p.whole_dv_ss = p.dv_ss, p.whole_dv_sh = p.dv_sh;
+      p.whole_f32 = p.dkdv_f32;
+      p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, 2}.grid();
+      sum.work_stats = p.work_stats;
+    }
     if (p.dkdv_parts > 1) {  // the kernel leaves fp32 parts, dkdv_sum_kernel adds them
       const int64_t rows = (int64_t)p.batch * p.kv_len * p.num_kv_heads;
       sum.dst[0] = p.dk, sum.sb[0] = p.dk_sb, sum.ss[0] = p.dk_ss, sum.sh[0] = p.dk_sh;
@@ -1228,7 +1282,9 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, dim3(min(p.total_items, kNumCus)), dim3(NW * 64), smem, stream, p);
     if (int rc = check_launch("fa_bwd_dkdv_kernel")) return rc;
     if (p.dkdv_parts > 1) {
-      hipLaunchKernelGGL(dkdv_sum_kernel<Tr>, dim3((unsigned)((sum.total[0] + 255) / 256), 2), dim3(256), 0, stream, sum);
+      unsigned grid = (unsigned)((sum.total[0] + 255) / 256);
+      if (p.work_stats) grid = grid < 4 * kNumCus ? grid : 4 * kNumCus;
+      hipLaunchKernelGGL(dkdv_sum_kernel<Tr>, dim3(grid, 2), dim3(256), 0, stream, sum);
       if (int rc = check_launch("dkdv_sum_kernel")) return rc;
     }
   }
@@ -1253,8 +1309,11 @@ static size_t parts_offset(const kvax_fa_args* a) {
 static int dkdv_parts(const kvax_fa_args* a) {
   return plan_dkdv_parts(a->batch, a->q_len, a->kv_len, a->num_heads, a->num_kv_heads, a->head_dim);
 }
+static bool dkdv_device_decides(const kvax_fa_args* a) {
+  return device_decides_parts(a->batch, a->q_len, a->kv_len, a->num_heads, a->num_kv_heads, a->head_dim);
+}
 static size_t dkdv_parts_bytes(const kvax_fa_args* a) {
-  const int parts = dkdv_parts(a);
+  const int parts = dkdv_device_decides(a) ? 2 : dkdv_parts(a);
   return parts == 1 ? 0 : (size_t)parts * a->batch * a->kv_len * a->num_kv_heads * (a->head_dim + value_head_dim(a)) * sizeof(float);
 }
 
@@ -1323,6 +1382,8 @@ extern "C" int kvax_fa_bwd(const kvax_fa_args* a, void* workspace, size_t worksp
   p.n_dq_blocks = cdiv(a->q_len, a->bwd_kv_block);
   p.n_kv_blocks = cdiv(a->kv_len, a->bwd_kv_block);
   p.dkdv_parts = dkdv_parts(a);
+  if (dkdv_device_decides(a))
+    p.work_stats = tile_order_counters(p.order_ws, a->batch, cdiv(a->kv_len, dkdv_kv_rows(a->head_dim))) + a->batch + kQueueCounters;
   p.parts_ws = (float*)((char*)workspace + parts_offset(a));
   p.num_shards = shards;
   p.shard_rows = a->q_len / shards;

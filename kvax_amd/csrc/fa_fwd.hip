@@ -167,15 +167,16 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   {
     // The full ranges are intersected over TQ rows whatever the rows per head: ids that come back after another id (which
     // the entry point excludes) make the mask claim too much, and what used to be right there stays right.
-    const int first = SPLIT ? q0 / p.group : q0, last = SPLIT ? (q0 + TQ - 1) / p.group : q0 + TR - 1;
-    const int window = SPLIT ? first : q0 / TQ * TQ;
-    const int qb1 = min((SPLIT ? last : window + TQ - 1) / p.qbs, p.n_qblocks - 1);
-    for (int qb = window / p.qbs; qb <= qb1; qb++) {
+    const int first = SPLIT ? q0 / p.group : q0 / TQ * TQ;
+    const int qb0 = first / p.qbs, qb1 = min((SPLIT ? (q0 + TQ - 1) / p.group : first + TQ - 1) / p.qbs, p.n_qblocks - 1);
+    int own0 = qb0, own1 = qb1;
+    if (head_shift > 0) own0 = q0 / p.qbs, own1 = (q0 + TR - 1) / p.qbs;
+    for (int qb = qb0; qb <= qb1; qb++) {
       const int64_t mi = (int64_t)b * p.n_qblocks + qb;
       const int l_ = p.lower[mi] * p.kbs, u_ = p.upper[mi] * p.kbs;
       flo = max(flo, p.lower_full[mi] * p.kbs);
       fhi = min(fhi, p.upper_full[mi] * p.kbs);
-      if (u_ > l_ && qb >= first / p.qbs && qb <= last / p.qbs) {
+      if (u_ > l_ && qb >= own0 && qb <= own1) {
         lo = min(lo, l_);
         hi = max(hi, u_);
       }

@@ -16,7 +16,7 @@ namespace {
 
 struct Params {
   TileSummaryJob jobs[2];
-  int32_t* zero;  // counters to clear (one per batch row, then kQueueCounters more), or null
+  int32_t* zero;  // counters to clear (one per batch row, then kQueueCounters + kOrderStats more), or null
 };
 
 __global__ __launch_bounds__(256) void tile_summaries_kernel(Params p) {
@@ -24,7 +24,7 @@ __global__ __launch_bounds__(256) void tile_summaries_kernel(Params p) {
   const int lane = threadIdx.x % 64;
   if (p.zero && blockIdx.x == 0 && blockIdx.z == 0) {
     if (threadIdx.x == 0) p.zero[blockIdx.y] = 0;
-    if (blockIdx.y == 0 && threadIdx.x < kQueueCounters) p.zero[gridDim.y + threadIdx.x] = 0;
+    if (blockIdx.y == 0 && threadIdx.x < kQueueCounters + kOrderStats) p.zero[gridDim.y + threadIdx.x] = 0;
   }
   const int n_tiles = (job.len + kTileRows - 1) / kTileRows;
   const int tile = blockIdx.x * 4 + threadIdx.x / 64;
@@ -102,18 +102,30 @@ __global__ __launch_bounds__(256) void tile_order_kernel(TileOrderJob job, int b
   // Both rules in one sort key (unique per item): heavy items index, light items
   // n * (1 + max work - work) + index; the rank of an item is the number of smaller keys.
   extern __shared__ __attribute__((aligned(16))) int keys[];  // n_items values, padded to a multiple of 4
-  __shared__ int total;
-  if (threadIdx.x == 0) total = 0;
+  __shared__ int total, longest;
+  if (threadIdx.x == 0) total = longest = 0;
   __syncthreads();
-  int part = 0;
+  int part = 0, most = 0;
   for (int i = threadIdx.x; i < job.n_items; i += 256) {
     keys[i] = __hip_atomic_load(work + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     part += keys[i];
+    most = max(most, keys[i]);
   }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off);
-  if (lane == 0) atomicAdd(&total, part);
+  for (int off = 32; off > 0; off >>= 1) {
+    part += __shfl_xor(part, off);
+    most = max(most, __shfl_xor(most, off));
+  }
+  if (lane == 0) {
+    atomicAdd(&total, part);
+    atomicMax(&longest, most);
+  }
   __syncthreads();
+  if (job.want_stats && threadIdx.x == 0) {
+    int32_t* stats = job.ws + (size_t)batch * (2 * job.n_items + 1) + kQueueCounters;
+    atomicAdd(stats, total);
+    atomicMax(stats + 1, longest);
+  }
   const int light_max = total / job.n_items;  // work <= this: light
   const int padded = (job.n_items + 3) & ~3;
   for (int i = threadIdx.x; i < padded; i += 256) {
