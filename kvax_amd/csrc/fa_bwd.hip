@@ -71,7 +71,7 @@ struct BwdParams {
   float scale, scale_log2;
   float scale_log2_abs;  // |scale| * log2(e) > 0, used with K negated when the scale is negative
   uint32_t k_sign;       // 0x80008000 when the scale is negative
-  // Where the device decides whether work items are shared (see kDecides): the ordering pass's sum and maximum of the
+  // Where the device decides whether work items are shared (see shares_items): the ordering pass's sum and maximum of the
   // items' work, and what dk, dv, their strides and dkdv_f32 are without parts; else null.
   const int32_t* work_stats;
   char *whole_dk, *whole_dv;
@@ -508,17 +508,18 @@ struct DkdvCfg {
 };
 inline int dkdv_kv_rows(int head_dim) { return head_dim > 192 ? 64 : 128; }
 
-// At head_dim 256 items are 64 rows, and whether two work-groups should share each of 257 to 512 of them depends on the
-// documents, so the device decides, from the work the ordering pass has counted: where the longest item is 15 % longer
-// than a compute unit's share of the work.  dK/dV kernel and sum, us, items whole -> as decided: 8k tokens in documents of 2k,
-// heads 16/4 (longest item 232 steps, share 178) 789 -> 629; 16k in documents of 3k, 8/2, 1119 -> 732; 2 x 4k in documents
-// of 700, 16/4, 516 -> 400.  Left whole (whole / in two parts): one document of 8k, 16/4, 1278 / 1327; of 16k, 8/2, 2564 / 2633;
-// 4k bidirectional, 32/8, 1234 / 1300.  A sum kernel that finds nothing to add takes 3 us.
-template <int D>
-constexpr bool kDecides = D == 256;
+// Whether two work-groups should share each of 257 to 512 items depends on the documents, so the device decides, from the
+// work the ordering pass has counted: where the longest item is 15 % and 40 steps longer than a compute unit's share of the
+// work.  us of the dK/dV kernel and sum, items whole -> as decided: 8k tokens in documents of 2k, heads 32/8 of 64 512 -> 333,
+// of 128 645 -> 545, of 192 with 128 740 -> 613, 16/4 of 256 (longest item 232 steps, share 178) 734 -> 549; 4 x 4k in documents
+// of 1k, 16/4 of 128, 400 -> 318; 16k in documents of 3k, 8/2 of 256, 1119 -> 737.  Left whole (whole / in two parts): one
+// document of 8k, 16/4 of 256, 1278 / 1327; of 16k, 8/2, 2564 / 2633; without the limit of 40 steps 4k in documents of 1k, 16/16 of
+// 192 with 128, 112 / 181, and 2 x 2k in documents of 300, 16/16 of 128, 75 / 134.  Deciding against it costs 6 us, mostly a sum
+// kernel that finds nothing to add: only where an item can have 160 steps.
 // stats: sum and maximum of the items' work (in tiles, the same for every kv head and query head)
-__device__ __forceinline__ bool shares_items(const int32_t* stats, int num_kv_heads) {
-  return (int64_t)stats[1] * kNumCus * 20 > (int64_t)stats[0] * num_kv_heads * 23;
+__device__ __forceinline__ bool shares_items(const int32_t* stats, int num_kv_heads, int group) {
+  const int64_t longest = (int64_t)stats[1] * group * kNumCus, share = (int64_t)stats[0] * num_kv_heads * group;
+  return longest * 20 > share * 23 && longest - share > 40 * kNumCus;
 }
 
 template <int D, int DV>
@@ -539,7 +540,9 @@ struct DkdvSmem {
   static constexpr int kTotal = kExchange + Cfg::kPairs * 2 * kSlotBytes;
 };
 
-template <class Tr, int D, int DV>
+// DECIDES: the device decides whether the items are shared (p.work_stats; a kernel of its own, because what it adds costs
+// the one at head_dim 128 two more spilled registers and 1.5 to 2 %).
+template <class Tr, int D, int DV, bool DECIDES>
 __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_bwd_dkdv_kernel(const BwdParams p) {
   using vec8 = typename Tr::vec8;
   using Smem = DkdvSmem<D, DV>;
@@ -570,10 +573,10 @@ __global__ __launch_bounds__(DkdvCfg<D>::kWaves * 64, DkdvCfg<D>::kWps) void fa_
   // batch row and kv head) from the queues (see ItemQueue) until none is left.  The ticket for the
   // next item is drawn when the current one's step loop has ended, so that its latency hides behind
   // the final stores and an item is never held back by a long one.
-  const bool whole = kDecides<D> && p.work_stats && !shares_items(p.work_stats, p.num_kv_heads);
+  const bool whole = DECIDES && !shares_items(p.work_stats, p.num_kv_heads, p.group);
   auto parts = [&] { return whole ? 1 : p.dkdv_parts; };
   const ItemMap items{p.batch * p.num_kv_heads, p.num_tiles, parts()};
-  ItemQueue work{p.dkdv_queue, kDecides<D> ? items.grid() : p.total_items, (int)(blockIdx.x % 8)};  // thread 0's
+  ItemQueue work{p.dkdv_queue, DECIDES ? items.grid() : p.total_items, (int)(blockIdx.x % 8)};  // thread 0's
   auto dkdv_f32 = [&] { return whole ? p.whole_f32 : p.dkdv_f32; };
   int* next_item = reinterpret_cast<int*>(smem + Smem::kTotal) + 1;
   if (tid == 0) *next_item = work.resolve(work.draw());
@@ -1085,7 +1088,7 @@ struct DkdvSumParams {
   int64_t sb[2], ss[2], sh[2];
   int64_t total[2];       // 4-element pieces of a tensor
   int pieces[2];          // and of one of its rows
-  int num_parts, kv_len, num_kv_heads;
+  int num_parts, kv_len, num_kv_heads, group;
   int f32;
   const int32_t* work_stats;  // null, or as in BwdParams: nothing to add where no items are shared
 };
@@ -1093,7 +1096,7 @@ struct DkdvSumParams {
 template <class Tr>
 __global__ __launch_bounds__(256) void dkdv_sum_kernel(const DkdvSumParams p) {
   const int which = blockIdx.y;
-  if (p.work_stats && !shares_items(p.work_stats, p.num_kv_heads)) return;
+  if (p.work_stats && !shares_items(p.work_stats, p.num_kv_heads, p.group)) return;
   // (one round, but for launches that may have nothing to do)
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.total[which]; i += (int64_t)gridDim.x * 256) {
   const float4* src = reinterpret_cast<const float4*>(p.parts[which]) + i;
@@ -1141,9 +1144,10 @@ int plan_dkdv_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_
   return (int)max(min(max(max(one_round, two_rounds), three_rounds), (int64_t)16), (int64_t)1);
 }
 
-// Whether the device decides between one part and two (see kDecides): the order is computed for such launches.
+// Whether the device decides between one part and two (see shares_items): the order is computed for such launches.
 bool device_decides_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int head_dim) {
-  if (!kDecides<256> || head_dim != 256 || plan_dkdv_parts(batch, q_len, kv_len, num_heads, num_kv_heads, head_dim) > 1) return false;
+  if (plan_dkdv_parts(batch, q_len, kv_len, num_heads, num_kv_heads, head_dim) > 1) return false;
+  if (num_kv_heads <= 0 || (int64_t)cdiv(q_len, kTile) * (num_heads / num_kv_heads) < 160) return false;
   const int tiles = cdiv(kv_len, dkdv_kv_rows(head_dim));
   const int64_t items = (int64_t)batch * num_kv_heads * tiles;
   return items > kNumCus && items <= 2 * kNumCus && tiles >= kMinOrderedItems && tiles <= kMaxOrderedItems;
@@ -1244,15 +1248,16 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
   // dK/dV: wavefronts in role pairs (see DkdvCfg)
   if (run_dkdv) {
     constexpr int NW = Cfg::kWaves;
-    auto kernel = fa_bwd_dkdv_kernel<Tr, D, DV>;
-    static LdsReservation done;
+    static LdsReservation done, done_deciding;
+    const bool deciding = p.work_stats != nullptr;
+    auto kernel = deciding ? fa_bwd_dkdv_kernel<Tr, D, DV, true> : fa_bwd_dkdv_kernel<Tr, D, DV, false>;
     // live-tile bookkeeping for as many query tiles as the remaining LDS holds (a multiple of 64)
     constexpr int kLdsLimit = kLdsPerCu;
     int chunk = 64;
     while (chunk < p.n_q_tiles && DkdvSmem<D, DV>::kTotal + live_tiles_bytes(NW, chunk * 2) <= kLdsLimit) chunk *= 2;
     p.list_tiles = min(chunk, max(p.n_q_tiles, 1));
     const int smem = DkdvSmem<D, DV>::kTotal + live_tiles_bytes(NW, p.list_tiles);
-    if (int rc = reserve_lds(kernel, smem, kLdsLimit, &done, "the dK/dV kernel")) return rc;
+    if (int rc = reserve_lds(kernel, smem, kLdsLimit, deciding ? &done_deciding : &done, "the dK/dV kernel")) return rc;
     p.num_tiles = cdiv(p.kv_len, Cfg::kKvRows);
     p.total_items = ItemMap{p.batch * p.num_kv_heads, p.num_tiles, p.dkdv_parts}.grid();
     DkdvSumParams sum{};
@@ -1271,7 +1276,7 @@ int launch_bwd(BwdParams p, hipStream_t stream) {
       sum.pieces[0] = D / 4, sum.pieces[1] = DV / 4;
       sum.total[0] = rows * (D / 4), sum.total[1] = rows * (DV / 4);
       sum.parts[0] = p.parts_ws, sum.parts[1] = p.parts_ws + rows * D * p.dkdv_parts;
-      sum.num_parts = p.dkdv_parts, sum.kv_len = p.kv_len, sum.num_kv_heads = p.num_kv_heads;
+      sum.num_parts = p.dkdv_parts, sum.kv_len = p.kv_len, sum.num_kv_heads = p.num_kv_heads, sum.group = p.group;
       sum.f32 = p.dkdv_f32;
       p.dk = (char*)sum.parts[0], p.dk_sh = D, p.dk_ss = (int64_t)p.num_kv_heads * D, p.dk_sb = p.dk_ss * p.kv_len;
       p.dv = (char*)sum.parts[1], p.dv_sh = DV, p.dv_ss = (int64_t)p.num_kv_heads * DV, p.dv_sb = p.dv_ss * p.kv_len;

@@ -180,8 +180,8 @@ def flash_attention_forward(query, key, value, q_pos, q_seg, kv_pos, kv_seg, fwd
 
 def backward_workspace_bytes(query, key, value=None) -> int:
     """Size of the scratch buffer ``kvax_fa_bwd`` needs for these shapes: delta, tile summaries, the
-    dispatch order and, where several work-groups share a dK/dV work item, their fp32 results (up to 101 MB
-    at head_dim 128, 134 MB at 256, 151 MB at 192).  Without ``value`` its head_dim is taken to be the key's, which is
+    dispatch order and, where several work-groups share a dK/dV work item, their fp32 results (up to 134 MB
+    at head_dim 128 and 256, 201 MB at 192).  Without ``value`` its head_dim is taken to be the key's, which is
     enough for any."""
     a = _native.FaArgs()
     a.batch, a.q_len, a.num_heads = query.shape[0], query.shape[1], query.shape[2]
