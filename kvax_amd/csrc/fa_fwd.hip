@@ -53,7 +53,7 @@ struct FwdParams {
   bool split_mode;
   int qbs, kbs, n_qblocks;
   int num_q_tiles, total_items;
-  const int4* kv_tiles;  // tile summaries [batch, n_kv_tiles]
+  const int4* kv_tiles;  // tile summaries [batch, n_kv_tiles]; null where nobody reads them or work-groups make their own
   int n_kv_tiles;
   const uint32_t* lists;  // wide kernel: live-tile lists of its query tiles (see TileListJob)
   int list_stride;        // words between two lists
@@ -69,6 +69,11 @@ struct FwdParams {
   float* part_ml;             // [items, num_parts, part_rows, 2] running max (base 2) and sum
   int head_shift;             // log2 of the heads per work-group (see heads_shift), not in split mode
 };
+
+// Split mode: windows of up to this many tiles are summarised by the work-groups themselves, which is one launch less (3.5 to
+// 4.4 us and the gap before the next).  Kernel with the launch / without: windows of 4 tiles (777 tokens, heads 8/2 of 64)
+// 13.9 / 14.9 us, mask and forward 28.9 -> 24.6 a pass; of 8, two per wavefront (2k tokens) 23.5 / 26.8, so 12 would be no gain.
+constexpr int kOwnSummaries = 8;
 
 template <int D, int DV, int STAGES>
 struct FwdSmem {
@@ -248,8 +253,21 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   }
   const int4* kv_summaries = p.kv_tiles + 2 * (int64_t)b * p.n_kv_tiles;
   // (narrow mode walks every tile of its window: see below)
+  const bool own_summaries = SPLIT && !NARROW && !p.kv_tiles;
   const WordSummaries first_word =
-      load_word_summaries(kv_summaries, t_lo >> 6, t_lo, NARROW ? t_lo : t_hi, lane);
+      load_word_summaries(kv_summaries, t_lo >> 6, t_lo, NARROW || own_summaries ? t_lo : t_hi, lane);
+  // Short windows: the wavefronts summarise the window's tiles themselves, one after the other, instead of a launch that
+  // does so for the whole sequence.
+  TileParts window[kOwnSummaries / NW];
+  if (own_summaries) {
+#pragma unroll
+    for (int i = 0; i < kOwnSummaries / NW; i++) {
+      const int t = t_lo + i * NW + wave, key = t * kTK + lane;
+      const bool have = t < t_hi && key < p.kv_len;
+      const int seg = have ? kv_seg[key] : -1, pos = have ? kv_pos[key] : 0;
+      if (t_lo + i * NW < t_hi) window[i] = wave_parts(seg != -1, seg, pos);
+    }
+  }
 
 #pragma unroll
   for (int qt = 0; qt < MQ; qt++) {
@@ -279,7 +297,27 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   // tenth of such a work-group's time; every tile of the window is walked by all four wavefronts,
   // the element mask settles the rest, and the call needs no tile summaries at all.
   if (!NARROW) {
-    mark_live_tiles<true, MQ>(kv_summaries, mine, t_lo, t_hi, live_bits + wave * words, word0, lane, first_word);
+    if (own_summaries) {
+      // (in the first bytes of the tile space, which is not in use yet)
+      TileParts* parts = reinterpret_cast<TileParts*>(smem);
+#pragma unroll
+      for (int i = 0; i < kOwnSummaries / NW; i++)
+        if (lane == 0 && t_lo + i * NW + wave < t_hi) parts[i * NW + wave] = window[i];
+      __syncthreads();
+      for (int w = word0; w * 64 < t_hi; w++) {
+        const int t = w * 64 + lane;
+        bool live = false;
+        if (t >= t_lo && t < t_hi) {
+          const TileParts other = parts[t - t_lo];
+#pragma unroll
+          for (int qt = 0; qt < MQ; qt++) live |= !parts_cannot_attend(mine[qt], other);
+        }
+        const unsigned long long m = __ballot(live);
+        if (lane == 0) live_bits[wave * words + w - word0] = m;
+      }
+    } else {
+      mark_live_tiles<true, MQ>(kv_summaries, mine, t_lo, t_hi, live_bits + wave * words, word0, lane, first_word);
+    }
     __syncthreads();
     if (wave == 0)
       compact_live_tiles<NW>(live_bits, words, word0, const_cast<uint32_t*>(live_list), live_count, lane);
@@ -1062,6 +1100,7 @@ struct FwdPlan {
   bool narrow() const { return num_parts > num_splits; }
   bool wide = false;  // regular mode with fa_fwd_wide_kernel (on request): lists for items of 256 query rows
   size_t summary_bytes = 0, list_bytes = 0;
+  bool summaries = true;  // a launch makes the tile summaries
   size_t total_bytes() const { return summary_bytes + part_o_bytes + part_ml_bytes + list_bytes; }
 };
 // LDS of one stage of the K/V ring.
@@ -1109,6 +1148,8 @@ FwdPlan plan_forward(int batch, int q_len, int kv_len, int num_heads, int num_kv
     plan.part_ml_bytes = (slots * 2 * sizeof(float) + 15) / 16 * 16;
   }
   if (plan.narrow()) plan.summary_bytes = 0;
+  // (their room in the workspace stays: its size is part of the interface)
+  plan.summaries = !plan.narrow() && plan.split_tiles > kOwnSummaries;
   return plan;
 }
 
@@ -1328,10 +1369,10 @@ int fa_fwd_impl(const kvax_fa_args* a, void* workspace, kvax_stream_t stream_) {
   p.n_qblocks = cdiv(a->q_len, a->fwd_query_block);
   p.q_sign = a->scale < 0.f ? 0x80008000u : 0u;
   p.scale_log2 = fmaxf(fabsf(a->scale), 1e-30f) * 1.4426950408889634f;
-  p.kv_tiles = (const int4*)workspace;
   p.n_kv_tiles = cdiv(a->kv_len, kTileRows);
   const FwdPlan plan = plan_forward(a->batch, a->q_len, a->kv_len, a->num_heads, a->num_kv_heads, a->head_dim,
                                     value_head_dim(a), (a->flags & KVAX_FA_FWD_WIDE) != 0);
+  p.kv_tiles = plan.summaries ? (const int4*)workspace : nullptr;
   p.split_mode = plan.split_mode;
   p.num_splits = plan.num_splits;
   p.num_parts = plan.num_parts;
@@ -1350,7 +1391,7 @@ int fa_fwd_impl(const kvax_fa_args* a, void* workspace, kvax_stream_t stream_) {
       return fail(KVAX_EUNSUPPORTED, "kv_len %d needs %d bytes of LDS for tile bitmaps (limit %d)",
                   a->kv_len, need, kLdsPerCu);
   }
-  if (!plan.narrow()) {  // the narrow mode does not read them
+  if (plan.summaries) {
     TileSummaryJob job{a->kv_pos, a->kv_seg, workspace, a->kv_len};
     if (int rc = launch_tile_summaries(&job, 1, a->batch, stream)) return rc;
   }
