@@ -1148,6 +1148,7 @@ int plan_dkdv_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_
 bool device_decides_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int head_dim) {
   if (plan_dkdv_parts(batch, q_len, kv_len, num_heads, num_kv_heads, head_dim) > 1) return false;
   if (num_kv_heads <= 0 || (int64_t)cdiv(q_len, kTile) * (num_heads / num_kv_heads) < 160) return false;
+  if (cdiv(q_len, kTile) > 1 << 20) return false;  // the sum of 512 items' work stays below 2^31
   const int tiles = cdiv(kv_len, dkdv_kv_rows(head_dim));
   const int64_t items = (int64_t)batch * num_kv_heads * tiles;
   return items > kNumCus && items <= 2 * kNumCus && tiles >= kMinOrderedItems && tiles <= kMaxOrderedItems;
