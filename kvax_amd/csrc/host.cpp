@@ -3,7 +3,7 @@
 // argument structure, launch - as one C++ function each, without the interpreter and ctypes.
 //
 // These functions take the plain case only: strided tensors of the current GPU whose types, shapes and layouts need no
-// conversion and no error message.  For anything else they return None, before they have done anything, and the caller
+// conversion and no error message, and no Python rule (of a tensor subclass or a mode) that has to see the torch calls.  For anything else they return None, before they have done anything, and the caller
 // goes on with the Python code of the same name, which converts or raises.  The library's functions are
 // handed in as addresses (bind), so that this module serves whichever library the package has loaded.
 //
@@ -17,6 +17,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 
 #include "kvax_amd.h"
 
@@ -37,10 +38,29 @@ struct WithoutGil {
   ~WithoutGil() { PyEval_RestoreThread(state); }
 };
 
-// An ordinary tensor in the memory of GPU `device`: not a wrapper, a view with pending conjugation or negation, or one
-// that a transform or a Python dispatch rule stands in front of.
+// Whether a mode that overrides torch functions is active (TorchFunctionMode): it has to see the allocations of a call.
+// The one behind torch.set_default_device() and `with torch.device(...)` is passed over: it changes calls that name no
+// device, and those of the Python code name theirs.
+bool functions_overridden() {
+  if (!at::impl::torch_function_mode_enabled()) return false;
+  static PyObject* const device_context = [] {
+    PyObject* module = PyImport_ImportModule("torch.utils._device");
+    PyObject* type = module ? PyObject_GetAttrString(module, "DeviceContext") : nullptr;
+    Py_XDECREF(module);
+    PyErr_Clear();
+    return type;
+  }();
+  for (int64_t i = 0; i < at::impl::PythonTorchFunctionTLS::stack_len(); i++) {
+    const auto& mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i);
+    if ((PyObject*)Py_TYPE(mode->ptr(&mode->pyinterpreter())) != device_context) return true;
+  }
+  return false;
+}
+
+// An ordinary tensor in the memory of GPU `device`: a torch.Tensor or a Parameter and no other subclass, not a wrapper, a
+// view with pending conjugation or negation, or one that a transform or a Python dispatch rule stands in front of.
 const at::Tensor* plain(PyObject* o, int device) {
-  if (!THPVariable_Check(o)) return nullptr;
+  if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
   constexpr c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
                                          c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
@@ -153,7 +173,7 @@ PyObject* forward(PyObject*, PyObject* const* o, Py_ssize_t n) {
   int64_t ints[5];
   void* stream;
   Inputs in;
-  if (!PyFloat_Check(o[8]) || !integers(o + 9, 5, ints) || !stream_handle(o[14], &stream)) Py_RETURN_NONE;
+  if (functions_overridden() || !PyFloat_Check(o[8]) || !integers(o + 9, 5, ints) || !stream_handle(o[14], &stream)) Py_RETURN_NONE;
   if (!in.read(o, (int)ints[4], PyFloat_AS_DOUBLE(o[8]), ints)) Py_RETURN_NONE;
   kvax_fa_args& a = in.a;
   if (!plain_mask(o[7], (int)ints[4], a.batch, 1, a.q_len, a.fwd_query_block, a.fwd_mask)) Py_RETURN_NONE;
@@ -183,7 +203,7 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
   int64_t ints[6];
   void* stream;
   Inputs in;
-  if (!PyFloat_Check(o[12]) || !integers(o + 13, 6, ints) || !stream_handle(o[19], &stream)) Py_RETURN_NONE;
+  if (functions_overridden() || !PyFloat_Check(o[12]) || !integers(o + 13, 6, ints) || !stream_handle(o[19], &stream)) Py_RETURN_NONE;
   const int64_t shards = ints[4];
   const int device = (int)ints[5];
   if (shards < 1 || shards > INT16_MAX || !in.read(o, device, PyFloat_AS_DOUBLE(o[12]), ints)) Py_RETURN_NONE;
@@ -225,7 +245,7 @@ PyObject* masks(PyObject*, PyObject* const* o, Py_ssize_t n) {
   if (n != 9) return PyErr_Format(PyExc_TypeError, "masks takes 9 arguments");
   int64_t ints[3];
   void* stream;
-  if (!integers(o + 5, 3, ints) || !stream_handle(o[8], &stream) || !PyTuple_Check(o[4])) Py_RETURN_NONE;
+  if (functions_overridden() || !integers(o + 5, 3, ints) || !stream_handle(o[8], &stream) || !PyTuple_Check(o[4])) Py_RETURN_NONE;
   const int64_t skip_pad = ints[0], num_shards = ints[1];
   const int device = (int)ints[2];
   const at::Tensor *first = plain(o[0], device), *keys = plain(o[2], device);

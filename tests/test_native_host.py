@@ -106,3 +106,65 @@ def test_errors_of_the_library_reach_the_caller():
             flash_attention(q, q, q, ids, ids, ids, ids, mask, fwd_params=params, bwd_params=params)
 
 
+class _Tagged(torch.Tensor):
+    """A subclass whose torch functions are seen, and give tensors of the subclass, as torch.Tensor's default does."""
+    seen = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(getattr(func, "__name__", str(func)))
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+class _Watch(torch.overrides.TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(getattr(func, "__name__", str(func)))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.gpu
+def test_subclasses_and_function_modes_see_the_calls(monkeypatch):
+    """What overrides torch functions sees the allocations of a call, and a subclass's results are of the subclass; parameters
+    and the mode of a default device are plain."""
+    n, params = 128, FlashAttentionParamsConfig(query_block_size=64, kv_block_size=64)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    data = [torch.randn((1, n, h, 64), generator=g, device="cuda", dtype=torch.bfloat16) for h in (4, 2, 2, 4)]
+    pos = torch.arange(n, device="cuda", dtype=torch.int32).expand(1, n).contiguous()
+    ids = (pos, pos // 50, pos, pos // 50)
+    real = _native.host()
+
+    def run(wrap):
+        spy = _Spy(real, off=False)
+        monkeypatch.setattr(_native, "host", lambda: spy)
+        x = [wrap(t.clone()).requires_grad_(True) for t in data[:3]]
+        with attention_specs(*ONE):
+            masks = create_attention_mask(*ids, fwd_params=params, bwd_params=params, calc_bwd_mask=True)
+            out = flash_attention(*x, *ids, masks, scale=0.125, fwd_params=params, bwd_params=params)
+            grads = torch.autograd.grad(out, x, data[3])
+        return spy.taken, (out, *grads)
+
+    plain = lambda t: t
+    taken, want = run(plain)
+    assert taken == ["masks", "forward", "backward"]
+    as_bits = lambda ts: [t.detach().as_subclass(torch.Tensor).view(torch.int16) for t in ts]
+    same = lambda got: all(torch.equal(a, b) for a, b in zip(as_bits(got), as_bits(want)))
+
+    taken, got = run(torch.nn.Parameter)
+    assert taken == ["masks", "forward", "backward"] and same(got)
+    with torch.device("cuda"):
+        taken, got = run(plain)
+    assert taken == ["masks", "forward", "backward"] and same(got)
+
+    _Tagged.seen.clear()
+    taken, got = run(lambda t: t.as_subclass(_Tagged))
+    assert taken == ["masks"] and same(got)
+    assert type(got[0]) is _Tagged and "empty_like" in _Tagged.seen
+    with _Watch() as mode:
+        taken, got = run(plain)
+    # (the backward runs in autograd's thread of the device, where the mode is not active)
+    assert taken == ["backward"] and same(got)
+    assert {"empty", "empty_like"} <= set(mode.seen)
