@@ -1,12 +1,14 @@
 """ctypes binding of ``libkvax_amd.so`` (the C ABI declared in ``include/kvax_amd.h``).
 
 There is no fallback: if the shared library is missing, every op raises ``KvaxNativeError``
-telling the caller to build it (``python -m kvax_amd.csrc.build``).
+telling the caller to build it (``python -m kvax_amd.csrc.build``).  The extension module ``kvax_amd._host`` only shortens
+the host side of the calls: without it they go to the same library through ``ctypes``.
 """
 from __future__ import annotations
 
 import ctypes as C
 import os
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(os.environ.get("KVAX_AMD_LIB") or Path(__file__).resolve().parent / "libkvax_amd.so")
@@ -111,19 +113,32 @@ def lib() -> C.CDLL:
 _host = None
 
 
+class _NoHost:
+    """Stands in for the extension module where it cannot be used: takes no call, so that all go through the Python code."""
+
+    @staticmethod
+    def forward(*args):
+        return None
+
+    backward = masks = forward
+
+
 def host():
-    """The extension module with the host side of the calls, bound to the library's functions."""
+    """The extension module with the host side of the calls, bound to the library's functions.  It is tied to the torch
+    it was compiled against, the library is not: where it cannot be used, one warning."""
     global _host
     if _host is None:
         l = lib()
         try:
             from kvax_amd import _host as module
+
+            module.bind(*[C.cast(f, C.c_void_p).value for f in (
+                l.kvax_fa_fwd_workspace_bytes, l.kvax_fa_fwd, l.kvax_fa_bwd_workspace_bytes, l.kvax_fa_bwd,
+                l.kvax_mask_workspace_bytes, l.kvax_mask_build)])
         except ImportError as e:
-            raise KvaxNativeError(
-                f"kvax_amd._host cannot be imported ({e}): run `python -m kvax_amd.csrc.build`") from e
-        module.bind(*[C.cast(f, C.c_void_p).value for f in (
-            l.kvax_fa_fwd_workspace_bytes, l.kvax_fa_fwd, l.kvax_fa_bwd_workspace_bytes, l.kvax_fa_bwd,
-            l.kvax_mask_workspace_bytes, l.kvax_mask_build)])
+            warnings.warn(f"kvax_amd._host cannot be used ({e}): calls take about 20 us longer on the host; run "
+                          "`python -m kvax_amd.csrc.build`", RuntimeWarning, stacklevel=3)
+            module = _NoHost
         _host = module
     return _host
 

@@ -1,8 +1,12 @@
 """The host side of the calls in native code (kvax_amd/csrc/host.cpp): the plain case gives what the general path in Python
 gives, bit for bit, and everything else is left to that path."""
+import sys
+import warnings
+
 import pytest
 import torch
 
+import kvax_amd
 from kvax_amd import FlashAttentionParamsConfig, Mesh, _native, attention_specs, create_attention_mask, flash_attention
 
 ONE = (("data", None, "model", None), ("data", None, "model", None))
@@ -37,6 +41,21 @@ def test_what_is_not_on_the_gpu_is_left_alone():
         assert host.forward(bad, x, x, ids, ids, ids, ids, mask, 1.0, 64, 64, 64, 64, 0, 0) is None
     with pytest.raises(TypeError):
         host.forward(x)
+
+
+def test_without_the_extension_the_calls_go_through_python(monkeypatch):
+    """A torch that it was not built for, or no build of it: the library is still there."""
+    monkeypatch.setattr(_native, "_host", None)
+    monkeypatch.delattr(kvax_amd, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "kvax_amd._host", None)
+    with pytest.warns(RuntimeWarning, match="cannot be used"):
+        host = _native.host()
+    ids = torch.zeros((1, 64), dtype=torch.int32)
+    assert host.masks(ids, ids, ids, ids, ((64, 64, False),), 1, 1, 0, 0) is None
+    assert host.forward(*[None] * 15) is None and host.backward(*[None] * 20) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _native.host() is host
 
 
 # name -> (batch, q_len, kv_len, heads, kv heads, head_dim, value head_dim, shards, forward, backward in native code)
