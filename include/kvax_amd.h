@@ -31,7 +31,9 @@ enum {
 
 enum { KVAX_BF16 = 0, KVAX_F16 = 1 };
 
-/* Version of this ABI (bumped on any incompatible change) and last error text. */
+/* Version of this ABI (bumped on any incompatible change; kvax_abi_version() is the one a library was built with) and
+ * last error text. */
+#define KVAX_ABI_VERSION 1
 int kvax_abi_version(void);
 const char* kvax_last_error(void);
 

@@ -123,19 +123,27 @@ class _NoHost:
     backward = masks = forward
 
 
+def _host_key(l: C.CDLL):
+    """What the extension module has to have been compiled against."""
+    import torch
+
+    return l.kvax_abi_version(), C.sizeof(FaArgs), C.sizeof(MaskDesc), str(torch.__version__)
+
+
 def host():
-    """The extension module with the host side of the calls, bound to the library's functions.  It is tied to the torch
-    it was compiled against, the library is not: where it cannot be used, one warning."""
+    """The extension module with the host side of the calls, bound to the library's functions.  It is tied to the ABI of
+    the library and to the torch it was compiled against (a library from elsewhere, KVAX_AMD_LIB, may differ, and the
+    library itself does not depend on torch): where it cannot be used, one warning."""
     global _host
     if _host is None:
         l = lib()
         try:
             from kvax_amd import _host as module
 
-            module.bind(*[C.cast(f, C.c_void_p).value for f in (
+            module.bind(*_host_key(l), *[C.cast(f, C.c_void_p).value for f in (
                 l.kvax_fa_fwd_workspace_bytes, l.kvax_fa_fwd, l.kvax_fa_bwd_workspace_bytes, l.kvax_fa_bwd,
                 l.kvax_mask_workspace_bytes, l.kvax_mask_build)])
-        except ImportError as e:
+        except (ImportError, TypeError) as e:  # TypeError: built when bind() took other arguments
             warnings.warn(f"kvax_amd._host cannot be used ({e}): calls take about 20 us longer on the host; run "
                           "`python -m kvax_amd.csrc.build`", RuntimeWarning, stacklevel=3)
             module = _NoHost

@@ -15,5 +15,5 @@ int fail(int code, const char* fmt, ...) {
 }
 }  // namespace kvax
 
-extern "C" int kvax_abi_version(void) { return 1; }
+extern "C" int kvax_abi_version(void) { return KVAX_ABI_VERSION; }
 extern "C" const char* kvax_last_error(void) { return kvax::g_error; }

@@ -55,6 +55,7 @@ def _compile_host() -> Path:
 
     root = Path(torch.__file__).resolve().parent
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DKVAX_TORCH_VERSION="{torch.__version__}"',
            f"-I{ROOT / 'include'}", f"-isystem{root / 'include'}", f"-isystem{root / 'include/torch/csrc/api/include'}",
            f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host.cpp"), "-o", str(HOST),
            f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]

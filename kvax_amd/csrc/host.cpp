@@ -19,6 +19,8 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 
+#include <cstring>
+
 #include "kvax_amd.h"
 
 namespace {
@@ -155,11 +157,21 @@ bool stream_handle(PyObject* o, void** out) {
   return true;
 }
 
+// bind(ABI version, bytes of kvax_fa_args, bytes of kvax_mask_desc, torch version, 6 addresses): the functions behind the
+// addresses and the tensors read here are only what this module was compiled against if the first four are.
 PyObject* bind(PyObject*, PyObject* const* o, Py_ssize_t n) {
-  if (n != 6) return PyErr_Format(PyExc_TypeError, "bind takes 6 addresses");
+  if (n != 10) return PyErr_Format(PyExc_TypeError, "bind takes 10 arguments");
+  const long version = PyLong_AsLong(o[0]), args = PyLong_AsLong(o[1]), desc = PyLong_AsLong(o[2]);
+  const char* torch = PyUnicode_Check(o[3]) ? PyUnicode_AsUTF8(o[3]) : "";
+  if (!torch || PyErr_Occurred()) return nullptr;
+  if (version != KVAX_ABI_VERSION || args != (long)sizeof(kvax_fa_args) || desc != (long)sizeof(kvax_mask_desc))
+    return PyErr_Format(PyExc_ImportError, "built for version %d of the C ABI with structures of %d and %d bytes, not %ld, %ld and %ld",
+                        KVAX_ABI_VERSION, (int)sizeof(kvax_fa_args), (int)sizeof(kvax_mask_desc), version, args, desc);
+  if (strcmp(torch, KVAX_TORCH_VERSION) != 0)
+    return PyErr_Format(PyExc_ImportError, "built for torch " KVAX_TORCH_VERSION ", not %s", torch);
   void* p[6];
   for (int i = 0; i < 6; i++)
-    if (!(p[i] = PyLong_AsVoidPtr(o[i]))) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "null address");
+    if (!(p[i] = PyLong_AsVoidPtr(o[4 + i]))) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "null address");
   lib.fwd_bytes = (decltype(lib.fwd_bytes))p[0], lib.fwd = (decltype(lib.fwd))p[1];
   lib.bwd_bytes = (decltype(lib.bwd_bytes))p[2], lib.bwd = (decltype(lib.bwd))p[3];
   lib.mask_bytes = (decltype(lib.mask_bytes))p[4], lib.mask_build = (decltype(lib.mask_build))p[5];

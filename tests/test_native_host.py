@@ -1,5 +1,6 @@
 """The host side of the calls in native code (kvax_amd/csrc/host.cpp): the plain case gives what the general path in Python
 gives, bit for bit, and everything else is left to that path."""
+import re
 import sys
 import warnings
 
@@ -56,6 +57,19 @@ def test_without_the_extension_the_calls_go_through_python(monkeypatch):
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         assert _native.host() is host
+
+
+@pytest.mark.parametrize("which", range(4), ids=["abi_version", "fa_args", "mask_desc", "torch"])
+def test_an_extension_built_for_something_else_is_not_used(which, monkeypatch):
+    """It fills in structures for functions it gets as bare addresses and reads torch's tensors through inline code."""
+    real = _native.host()
+    key = list(_native._host_key(_native.lib()))
+    key[which] = key[which] + (1 if which < 3 else ".post1")
+    monkeypatch.setattr(_native, "_host_key", lambda l: tuple(key))
+    monkeypatch.setattr(_native, "_host", None)
+    with pytest.warns(RuntimeWarning, match=re.escape(str(key[which]))):
+        host = _native.host()
+    assert host is not real and host.forward(*[None] * 15) is None
 
 
 # name -> (batch, q_len, kv_len, heads, kv heads, head_dim, value head_dim, shards, forward, backward in native code)
