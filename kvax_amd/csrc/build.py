@@ -1,11 +1,13 @@
 """Compile the HIP sources in this directory into ``kvax_amd/libkvax_amd.so`` for gfx950.
 
-Usage: ``python -m kvax_amd.csrc.build`` (or ``build()`` from Python).  hipcc cross-compiles, so
-no GPU is needed.  The library is built in-tree next to the Python package.
+Usage: ``python -m kvax_amd.csrc.build`` (or ``build()`` from Python; ``python kvax_amd/csrc/build.py`` where there is no
+torch).  hipcc cross-compiles, so no GPU is needed.  The library is built in-tree next to the Python package, and with it,
+where torch and g++ are there, the extension module ``kvax_amd/_host.so``.
 """
 from __future__ import annotations
 
 import os
+import shutil
 import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
@@ -47,12 +49,18 @@ def _compile(src: str, extra: list[str]) -> Path:
     return out
 
 
-def _compile_host() -> Path:
-    """The extension module ``kvax_amd._host``: plain C++ against torch's headers and libraries."""
+def _compile_host() -> Path | None:
+    """The extension module ``kvax_amd._host``: plain C++ against torch's headers and libraries.  Nothing else needs them
+    or g++: without them it is left out."""
     import sysconfig
 
-    import torch
-
+    try:
+        import torch
+    except ImportError:
+        torch = None
+    if torch is None or not shutil.which("g++"):
+        print(f"{HOST.name} is left out: no {'torch' if torch is None else 'g++'}", file=sys.stderr)
+        return None
     root = Path(torch.__file__).resolve().parent
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f'-DKVAX_TORCH_VERSION="{torch.__version__}"',
@@ -77,12 +85,12 @@ def build(extra_flags: list[str] | None = None, jobs: int = 4, lib: Path | None 
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         host = ex.submit(_compile_host) if lib is None else None
         objs = list(ex.map(lambda s: _compile(s, extra), sources))
+        cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *map(str, objs)]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"link failed:\n{r.stderr}")
         if host is not None:
-            host.result()
-    cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *map(str, objs)]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"link failed:\n{r.stderr}")
+            host.result()  # raises once the library is there, which does not need it
     return LIB
 
 

@@ -1,6 +1,8 @@
 """The host side of the calls in native code (kvax_amd/csrc/host.cpp): the plain case gives what the general path in Python
 gives, bit for bit, and everything else is left to that path."""
 import re
+import shutil
+import subprocess
 import sys
 import warnings
 
@@ -70,6 +72,32 @@ def test_an_extension_built_for_something_else_is_not_used(which, monkeypatch):
     with pytest.warns(RuntimeWarning, match=re.escape(str(key[which]))):
         host = _native.host()
     assert host is not real and host.forward(*[None] * 15) is None
+
+
+@pytest.mark.parametrize("missing", ["torch", "g++", "headers"])
+def test_the_library_is_built_without_what_only_the_extension_needs(missing, monkeypatch, tmp_path, capsys):
+    from kvax_amd.csrc import build
+
+    commands = []
+
+    def run(cmd, **kwargs):
+        commands.append(cmd)
+        broken = cmd[0] == "g++" and missing == "headers"
+        return subprocess.CompletedProcess(cmd, int(broken), "", "no headers" if broken else "")
+
+    monkeypatch.setattr(build, "LIB", tmp_path / "lib.so")
+    monkeypatch.setattr(build, "OBJ", tmp_path / "obj")
+    monkeypatch.setattr(build.subprocess, "run", run)
+    monkeypatch.setattr(shutil, "which", lambda name: None if name == missing else f"/usr/bin/{name}")
+    if missing == "torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+    if missing == "headers":
+        with pytest.raises(RuntimeError, match="no headers"):
+            build.build()
+    else:
+        assert build.build() == tmp_path / "lib.so"
+        assert not any(cmd[0] == "g++" for cmd in commands) and missing in capsys.readouterr().err
+    assert any("-o" in cmd and cmd[cmd.index("-o") + 1] == str(tmp_path / "lib.so") for cmd in commands), "not linked"
 
 
 # name -> (batch, q_len, kv_len, heads, kv heads, head_dim, value head_dim, shards, forward, backward in native code)
