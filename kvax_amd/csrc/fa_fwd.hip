@@ -73,6 +73,10 @@ struct FwdParams {
 // Split mode: windows of up to this many tiles are summarised by the work-groups themselves, which is one launch less (3.5 to
 // 4.4 us and the gap before the next).  Kernel with the launch / without: windows of 4 tiles (777 tokens, heads 8/2 of 64)
 // 13.9 / 14.9 us, mask and forward 28.9 -> 24.6 a pass; of 8, two per wavefront (2k tokens) 23.5 / 26.8, so 12 would be no gain.
+// Only where all work-groups are resident at once: each summarises its window again and every further round pays for it.  Forward,
+// us, with the launch / without, rounds of 128 rows in brackets: 40 queries x 500 keys, heads 32/8 of 128, 32 batch rows (1) 38.3 /
+// 38.2, 64 (2) 69.7 / 74.0; 100 x 500, 256 rows (16) 451 / 477; 64 x 64, 512 rows (16) 114 / 118; 100 x 256 in documents of 50, 128
+// rows (8) 114 / 123; the best of several rounds, 40 x 200, 64 rows (2) 38.9 / 37.8.
 constexpr int kOwnSummaries = 8;
 
 template <int D, int DV, int STAGES>
@@ -1149,7 +1153,7 @@ FwdPlan plan_forward(int batch, int q_len, int kv_len, int num_heads, int num_kv
   }
   if (plan.narrow()) plan.summary_bytes = 0;
   // (their room in the workspace stays: its size is part of the interface)
-  plan.summaries = !plan.narrow() && plan.split_tiles > kOwnSummaries;
+  plan.summaries = !plan.narrow() && (plan.split_tiles > kOwnSummaries || items > resident);
   return plan;
 }
 

@@ -1,17 +1,27 @@
 """Split forward with windows of up to eight tiles, whose tiles the work-groups summarise themselves, and the first longer
 one: against the dense CPU oracle, with windows that lie across the words of the live-tile bitmap, documents, padding and
 NaN in keys of tiles that nothing attends to."""
+import ctypes
+import sys
+
 import numpy as np
 import pytest
 import torch
 
-from kvax_amd import create_attention_mask
+from kvax_amd import _native, create_attention_mask
 from kvax_amd.ops.flash_attention import flash_attention_forward
 from kvax_amd.utils import FlashAttentionParamsConfig, attention_specs
 from oracle import attention_oracle as ao
 from tests.tolerances import check_close
 
 pytestmark = pytest.mark.gpu
+flash_attention_module = sys.modules["kvax_amd.ops.flash_attention"]  # (the package exports a function of that name)
+
+
+def check_lse(got, ref):
+    """Base 2 against natural.  fp32 sums: a logit is off by at most (D + 1) 2^-24 sum |q k| scale = 1.6e-4 at D = 256 and normal
+    inputs, the sum over 500 keys by 500 x 2^-24, v_exp_f32 and v_log_f32 by an ulp."""
+    assert np.abs(got.cpu().numpy() * np.log(2.0) - ref).max() <= 1e-3
 
 
 @pytest.mark.parametrize("d, dv", [(64, 64), (128, 128), (192, 128), (256, 256)])
@@ -46,3 +56,37 @@ def test_short_windows(device, sq, sk, hq, hkv, d, dv):
     out, _ = flash_attention_forward(q, k, v, *ids, mask[0], d ** -0.5, p, p)
     check_close("out", out, ref)
     assert not out[ids[1] == -1].any()
+
+
+# One resident set of work-groups (512, or 256 above head_dim 128) summarises its windows itself, with more a launch does:
+# the summaries at the start of the workspace are left alone or written.
+@pytest.mark.parametrize("d, dv, resident", [(64, 64, 512), (128, 128, 512), (192, 128, 256), (256, 256, 256)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_more_work_groups_than_resident_take_summaries_from_a_launch(device, d, dv, resident, more):
+    hkv, sq, sk = 8, 40, 130
+    b = resident // hkv + more
+    seg = (np.arange(sk) >= 70).astype(np.int32)
+    seg[-9:] = -1
+    kv = [np.broadcast_to(x, (b, sk)).copy() for x in (np.arange(sk, dtype=np.int32), seg)]
+    ids = [x[:, 45:45 + sq].copy() for x in kv] + kv
+    on_gpu = [torch.from_numpy(x).to(device) for x in ids]
+    g = torch.Generator(device=device).manual_seed(7)
+    q, k, v = (torch.randn(s, generator=g, device=device, dtype=torch.bfloat16) for s in ((b, sq, hkv, d), (b, sk, hkv, d), (b, sk, hkv, dv)))
+    p = FlashAttentionParamsConfig(64, 64)
+    spec = ("data", None, "model", None)
+    with attention_specs(spec, spec):
+        mask = create_attention_mask(*on_gpu, fwd_params=p)[0]
+    a = flash_attention_module._base_args(q, k, v, *on_gpu, d ** -0.5, p, p)
+    out, lse = q.new_empty((b, sq, hkv, dv)), torch.empty((b, hkv, sq), device=device)
+    a.out, a.lse, a.o_strides = out.data_ptr(), lse.data_ptr(), flash_attention_module._strides3(out)
+    a.fwd_mask = flash_attention_module._mask_ptrs(mask)
+    lib = _native.lib()
+    ws = torch.full((lib.kvax_fa_fwd_workspace_bytes(ctypes.byref(a)),), 0x5A, dtype=torch.uint8, device=device)
+    assert ws.numel() >= 32 * b * 3
+    rc = lib.kvax_fa_fwd(ctypes.byref(a), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+    _native.check(rc, "kvax_fa_fwd")
+    assert bool((ws[:32 * b * 3] != 0x5A).any()) == bool(more)
+    rows = [0, b - 1]
+    ref, ref_lse = ao.attention_forward(*(t[rows].float().cpu().numpy() for t in (q, k, v)), *(x[rows] for x in ids), d ** -0.5)
+    check_close("out", out[rows], ref)
+    check_lse(lse[rows], ref_lse)
