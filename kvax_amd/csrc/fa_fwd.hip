@@ -266,8 +266,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void fa_fwd_kernel(const FwdParams p)
   if (own_summaries) {
 #pragma unroll
     for (int i = 0; i < kOwnSummaries / NW; i++) {
-      const int t = t_lo + i * NW + wave, key = t * kTK + lane;
-      const bool have = t < t_hi && key < p.kv_len;
+      // (without any key in the range t_lo is 2^25 - 1: the key index is formed for tiles of the window only)
+      const int t = t_lo + i * NW + wave, key = t < t_hi ? t * kTK + lane : p.kv_len;
+      const bool have = key < p.kv_len;
       const int seg = have ? kv_seg[key] : -1, pos = have ? kv_pos[key] : 0;
       if (t_lo + i * NW < t_hi) window[i] = wave_parts(seg != -1, seg, pos);
     }

@@ -90,3 +90,26 @@ def test_more_work_groups_than_resident_take_summaries_from_a_launch(device, d, 
     ref, ref_lse = ao.attention_forward(*(t[rows].float().cpu().numpy() for t in (q, k, v)), *(x[rows] for x in ids), d ** -0.5)
     check_close("out", out[rows], ref)
     check_lse(lse[rows], ref_lse)
+
+
+@pytest.mark.parametrize("d, dv", [(64, 64), (128, 128), (192, 128), (256, 256)])
+def test_short_windows_of_rows_without_any_key(device, d, dv):
+    """Work-groups whose block mask names no key at all (queries of padding, keys of padding) beside ones with keys."""
+    b, sq, sk, hq, hkv = 3, 130, 300, 4, 2
+    seg = np.zeros((b, sk), np.int32)
+    q_seg = np.zeros((b, sq), np.int32)
+    q_seg[0], seg[1] = -1, -1
+    pos = np.broadcast_to(np.arange(sk, dtype=np.int32), (b, sk)).copy()
+    ids = [pos[:, sk - sq:].copy(), q_seg, pos, seg]
+    on_gpu = [torch.from_numpy(x).to(device) for x in ids]
+    g = torch.Generator(device=device).manual_seed(9)
+    q, k, v = (torch.randn(s, generator=g, device=device, dtype=torch.bfloat16) for s in ((b, sq, hq, d), (b, sk, hkv, d), (b, sk, hkv, dv)))
+    p = FlashAttentionParamsConfig(64, 64)
+    spec = ("data", None, "model", None)
+    with attention_specs(spec, spec):
+        mask = create_attention_mask(*on_gpu, fwd_params=p)[0]
+    out, lse = flash_attention_forward(q, k, v, *on_gpu, mask, d ** -0.5, p, p)
+    ref, ref_lse = ao.attention_forward(*(t.float().cpu().numpy() for t in (q, k, v)), *ids, d ** -0.5)
+    check_close("out", out, ref)
+    check_lse(lse, ref_lse)
+    assert not out[:2].any() and not lse[:2].any()
