@@ -4,6 +4,7 @@ import re
 import shutil
 import subprocess
 import sys
+import threading
 import warnings
 
 import pytest
@@ -112,7 +113,11 @@ CASES = {
     "ids_not_contiguous": (2, 128, 128, 4, 2, 64, 64, 1, False, True),
     "mask_not_contiguous": (2, 128, 128, 4, 2, 64, 64, 1, False, False),
     "gradient_expanded": (1, 128, 128, 4, 2, 64, 64, 1, True, False),
+    "half": (2, 192, 192, 4, 2, 128, 128, 1, True, True),
+    "block_sizes": (3, 256, 384, 4, 2, 64, 64, 1, True, True),
+    "block_sizes_shards": (2, 512, 384, 4, 2, 64, 64, 2, True, True),
 }
+IDS_TO_CONVERT = ("int64_ids", "ids_not_contiguous")  # masks from the Python code, as the forward
 
 
 @pytest.mark.gpu
@@ -120,7 +125,8 @@ CASES = {
 def test_same_bits_as_the_general_path(name, monkeypatch):
     b, sq, sk, hq, hkv, d, dv, cp, fwd_native, bwd_native = CASES[name]
     g = torch.Generator(device="cuda").manual_seed(1)
-    draw = lambda *s: torch.randn(s, generator=g, device="cuda", dtype=torch.bfloat16)
+    dtype = torch.float16 if name == "half" else torch.bfloat16
+    draw = lambda *s: torch.randn(s, generator=g, device="cuda", dtype=dtype)
     q, k, v = draw(b, sq, hq, d), draw(b, sk, hkv, d), draw(b, sk, hkv, dv)
     if name == "transposed_views":
         q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
@@ -133,24 +139,28 @@ def test_same_bits_as_the_general_path(name, monkeypatch):
         ids = [x.long() for x in ids]
     if name == "ids_not_contiguous":
         ids = [torch.stack([x, x], 2)[..., 0] for x in ids]
-    params = FlashAttentionParamsConfig(query_block_size=64, kv_block_size=64)
+    # (apart: every size another, so that none can stand for another)
+    apart = name.startswith("block_sizes")
+    fwd_params = FlashAttentionParamsConfig(query_block_size=64 if not apart else 32, kv_block_size=64 if not apart else 16)
+    bwd_params = FlashAttentionParamsConfig(query_block_size=64, kv_block_size=64 if not apart else 128)
     mesh = Mesh({"data": 1, "context": cp, "model": 1}) if cp > 1 else None
     real = _native.host()
 
     def run(spy):
         monkeypatch.setattr(_native, "host", lambda: spy)
         with attention_specs(*(CP if cp > 1 else ONE)):
-            masks = create_attention_mask(*ids, fwd_params=params, bwd_params=params, calc_bwd_mask=True, mesh=mesh)
+            masks = create_attention_mask(*ids, fwd_params=fwd_params, bwd_params=bwd_params, calc_bwd_mask=True, mesh=mesh)
             arrays = [a for m in masks for a in m.flatten()]
             if name == "mask_not_contiguous":
                 masks = tuple(type(m)(*[torch.stack([a, a], -1)[..., 0] for a in m.flatten()]) for m in masks)
             x = [t.detach().requires_grad_(True) for t in (q, k, v)]
-            out = flash_attention(*x, *ids, masks, scale=d ** -0.5, fwd_params=params, bwd_params=params, mesh=mesh)
+            out = flash_attention(*x, *ids, masks, scale=d ** -0.5, fwd_params=fwd_params, bwd_params=bwd_params, mesh=mesh)
             grads = torch.autograd.grad(out, x, dout) if bwd_native is not None else []
         return arrays + [out.detach(), *grads]
 
     spy = _Spy(real, off=False)
     got, want = run(spy), run(_Spy(real, off=True))
+    assert ("masks" in spy.taken) == (name not in IDS_TO_CONVERT)
     assert ("forward" in spy.taken) == fwd_native and ("backward" in spy.taken) == bool(bwd_native)
     for a, e in zip(got, want):
         assert a.shape == e.shape and a.stride() == e.stride() and a.dtype == e.dtype and torch.equal(a, e)
@@ -229,3 +239,82 @@ def test_subclasses_and_function_modes_see_the_calls(monkeypatch):
     # (the backward runs in autograd's thread of the device, where the mode is not active)
     assert taken == ["backward"] and same(got)
     assert {"empty", "empty_like"} <= set(mode.seen)
+
+
+def _training_pass(seed, hq, hkv, d, n):
+    """(inputs, a function of them that builds the masks and runs forward and backward)"""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = [torch.randn((2, n, h, d), generator=g, device="cuda", dtype=torch.bfloat16) for h in (hq, hkv, hkv, hq)]
+    pos = torch.arange(n, device="cuda", dtype=torch.int32).expand(2, n).contiguous()
+    ids = (pos, pos // 300, pos, pos // 300)
+    params = FlashAttentionParamsConfig(query_block_size=64, kv_block_size=64)
+
+    def run(q, k, v, dout):
+        q, k, v = (t.detach().requires_grad_(True) for t in (q, k, v))
+        masks = create_attention_mask(*ids, fwd_params=params, bwd_params=params, calc_bwd_mask=True)
+        out = flash_attention(q, k, v, *ids, masks, scale=d ** -0.5, fwd_params=params, bwd_params=params)
+        return (*(a for m in masks for a in m.flatten()), out.detach(), *torch.autograd.grad(out, (q, k, v), dout))
+
+    return x, run
+
+
+@pytest.mark.gpu
+def test_two_threads_on_streams_of_their_own(monkeypatch):
+    """The interpreter lock is released in the launches, and memory and kernels are those of each thread's current stream."""
+    spy = _Spy(_native.host(), off=False)
+    monkeypatch.setattr(_native, "host", lambda: spy)
+    with attention_specs(*ONE):
+        passes = [_training_pass(1, 8, 2, 128, 1024), _training_pass(2, 4, 4, 64, 768)]
+        want = [run(*x) for x, run in passes]
+        torch.cuda.synchronize()
+        got, errors = [[], []], []
+
+        def worker(i):
+            try:
+                x, run = passes[i]
+                stream = torch.cuda.Stream()
+                with torch.cuda.stream(stream):
+                    for _ in range(20):
+                        # (what ran on the stream before may lie where the next pass allocates: all are kept and compared)
+                        got[i].append(run(*x))
+                stream.synchronize()
+            except Exception as e:  # surfaced below
+                errors.append(e)
+
+        threads = [threading.Thread(target=worker, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(60)
+    assert not errors and all(len(x) == 20 for x in got)
+    assert {name: spy.taken.count(name) for name in ("masks", "forward", "backward")} == dict.fromkeys(("masks", "forward", "backward"), 42)
+    for results, ref in zip(got, want):
+        assert all(torch.equal(a, b) for result in results for a, b in zip(result, ref))
+
+
+@pytest.mark.gpu
+def test_graph_replays_match_eager(monkeypatch):
+    """A step recorded into a graph through the native calls and replayed on new inputs, with eager work between the replays."""
+    spy = _Spy(_native.host(), off=False)
+    monkeypatch.setattr(_native, "host", lambda: spy)
+    with attention_specs(*ONE):
+        x, run = _training_pass(3, 8, 2, 128, 1024)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            run(*x)  # the kernels' LDS limits, autograd's thread
+        torch.cuda.current_stream().wait_stream(side)
+        static = [t.clone() for t in x]
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            results = run(*static)
+        assert spy.taken == ["masks", "forward", "backward"] * 2
+        for seed in (4, 5, 6):
+            g = torch.Generator(device="cuda").manual_seed(seed)
+            new = [torch.randn(t.shape, generator=g, device="cuda", dtype=t.dtype) for t in x]
+            for to, t in zip(static, new):
+                to.copy_(t)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(results, run(*new))), f"replay {seed}"
