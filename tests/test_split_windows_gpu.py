@@ -1,6 +1,6 @@
 """Split forward with windows of up to eight tiles, whose tiles the work-groups summarise themselves, and the first longer
-one: against the dense CPU oracle, with windows that lie across the words of the live-tile bitmap, documents, padding and
-NaN in keys of tiles that nothing attends to."""
+one: against the dense CPU oracle, with windows that lie across the words of the live-tile bitmap, documents, padding, and
+NaN in the keys of a document inside the windows that no row attends to."""
 import ctypes
 import sys
 
@@ -18,10 +18,10 @@ pytestmark = pytest.mark.gpu
 flash_attention_module = sys.modules["kvax_amd.ops.flash_attention"]  # (the package exports a function of that name)
 
 
-def check_lse(got, ref):
+def check_lse(got, ref, keys=500):
     """Base 2 against natural.  fp32 sums: a logit is off by at most (D + 1) 2^-24 sum |q k| scale = 1.6e-4 at D = 256 and normal
-    inputs, the sum over 500 keys by 500 x 2^-24, v_exp_f32 and v_log_f32 by an ulp."""
-    assert np.abs(got.cpu().numpy() * np.log(2.0) - ref).max() <= 1e-3
+    inputs, the sum over the keys by keys x 2^-24, v_exp_f32 and v_log_f32 by an ulp."""
+    assert np.abs(got.cpu().numpy() * np.log(2.0) - ref).max() <= 1e-3 + keys * 2.0 ** -24
 
 
 @pytest.mark.parametrize("d, dv", [(64, 64), (128, 128), (192, 128), (256, 256)])
@@ -49,12 +49,13 @@ def test_short_windows(device, sq, sk, hq, hkv, d, dv):
     spec = ("data", None, "model", None)
     with attention_specs(spec, spec):
         mask = create_attention_mask(*ids, fwd_params=p)
-    ref, _ = ao.attention_forward(*(x.float().cpu().numpy() for x in (q, k, v)), q_pos, q_seg, kv_pos, kv_seg, d ** -0.5)
-    if sk > 1000:  # whole tiles of padding: dead, whatever they hold
+    ref, ref_lse = ao.attention_forward(*(x.float().cpu().numpy() for x in (q, k, v)), q_pos, q_seg, kv_pos, kv_seg, d ** -0.5)
+    if sk > 1000:  # whole tiles of padding beyond the block mask: not in any window, whatever they hold
         first = -(-(sk - sk // 8) // 64) * 64
         k[:, first:], v[:, first:] = float("nan"), float("nan")
-    out, _ = flash_attention_forward(q, k, v, *ids, mask[0], d ** -0.5, p, p)
+    out, lse = flash_attention_forward(q, k, v, *ids, mask[0], d ** -0.5, p, p)
     check_close("out", out, ref)
+    check_lse(lse, ref_lse, sk)
     assert not out[ids[1] == -1].any()
 
 
@@ -113,3 +114,44 @@ def test_short_windows_of_rows_without_any_key(device, d, dv):
     check_close("out", out, ref)
     check_lse(lse, ref_lse)
     assert not out[:2].any() and not lse[:2].any()
+
+
+# The document in the middle of the keys has no queries: its tiles lie inside [lower, upper) of the block mask, whose blocks hold
+# queries of the documents on either side, and are passed over for what the work-groups know of them.  Its whole tiles hold
+# NaN, which would reach the results through 0 x NaN of any tile that is worked on.
+@pytest.mark.parametrize("d, dv, dtype", [(64, 64, torch.bfloat16), (128, 128, torch.float16), (192, 128, torch.bfloat16),
+                                          (256, 256, torch.float16)])
+@pytest.mark.parametrize("b, sq, sk, hq, hkv", [
+    (1, 40, 4480, 4, 1),     # windows of 4 tiles
+    (2, 40, 20500, 4, 1),    # of 6
+    (1, 40, 32700, 4, 1),    # of 8
+    (1, 40, 33000, 4, 1),    # of 9: a launch summarises the sequence
+    (2, 777, 777, 4, 2),
+])
+def test_dead_tiles_inside_the_windows(device, b, sq, sk, hq, hkv, d, dv, dtype):
+    first, last = sk * 3 // 10, sk * 7 // 10  # the document without queries
+    kv_pos = np.broadcast_to(np.arange(sk, dtype=np.int32), (b, sk)).copy()
+    kv_seg = ((kv_pos >= first).astype(np.int32) + (kv_pos >= last)).astype(np.int32)
+    kv_seg[:, sk - 20:] = -1
+    q_pos = np.maximum(kv_pos[:, sk - sq:], last + 64)  # every query sees the first document and some of the last
+    q_seg = np.where(np.arange(sq) < 16, 0, 2).astype(np.int32) * np.ones((b, 1), np.int32)
+    q_seg[:, -3:] = -1
+    if b > 1:
+        q_seg[1] = np.where(np.arange(sq) < 9, 0, 2)  # rows of the batch differ
+    host = (q_pos, q_seg, kv_pos, kv_seg)
+    ids = [torch.from_numpy(x).to(device) for x in host]
+    g = torch.Generator().manual_seed(sq + sk + d)
+    q, k, v = (torch.randn(s, generator=g).to(dtype).to(device) for s in ((b, sq, hq, d), (b, sk, hkv, d), (b, sk, hkv, dv)))
+    p = FlashAttentionParamsConfig(64, 64)
+    spec = ("data", None, "model", None)
+    with attention_specs(spec, spec):
+        mask = create_attention_mask(*ids, fwd_params=p)[0]
+    ref, ref_lse = ao.attention_forward(*(x.float().cpu().numpy() for x in (q, k, v)), *host, d ** -0.5)
+    dead = slice(-(-first // 64), last // 64)  # its whole tiles
+    lower, upper = (x[:, 0, 0].cpu().numpy() for x in (mask.lower_bounds, mask.upper_bounds))
+    assert dead.stop > dead.start and (lower <= dead.start).all() and (upper >= dead.stop).all()
+    k[:, dead.start * 64:dead.stop * 64], v[:, dead.start * 64:dead.stop * 64] = float("nan"), float("nan")
+    out, lse = flash_attention_forward(q, k, v, *ids, mask, d ** -0.5, p, p)
+    check_close("out", out, ref)
+    check_lse(lse, ref_lse, sk)
+    assert not out[ids[1] == -1].any() and not lse.transpose(1, 2)[ids[1] == -1].any()
