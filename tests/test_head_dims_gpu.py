@@ -190,3 +190,35 @@ def test_any_strides_at_192(device, d, dv, view_q, view_k, view_v, view_dout):
         given = [view(t) for view, t in zip((view_q, view_k, view_v, view_dout), (q, k, v, dout))]
         for got, want in zip(run(*given), run(*(t.contiguous().clone() for t in given))):
             assert torch.equal(got, want)
+
+
+# At head_dim 64 and 128 eight wavefronts run where the tile bitmaps of the keys leave no room for two work-groups on a compute
+# unit (more than 6929 and 2993 tiles of 64).  They take one, two, four or eight heads
+# of a group; the rows end inside a 32-row block, and the documents of the queries are spread over the keys.
+@pytest.mark.parametrize("group, hkv", [(1, 8), (2, 4), (4, 2), (8, 1), (12, 1)])
+@pytest.mark.parametrize("d, sk", [(64, 460_000), (128, 200_000)])
+def test_heads_of_a_group_share_a_work_group_of_eight_wavefronts(device, group, hkv, d, sk):
+    sq, hq = 300, group * hkv
+    seg = torch.arange(sk, device=device, dtype=torch.int32) * 7 // sk
+    kv_pos = torch.arange(sk, device=device, dtype=torch.int32)
+    at = torch.arange(sq, device=device) * 97 % 29 + torch.arange(sq, device=device) * (sk // sq)  # keys the queries stand at
+    q_pos, q_seg = at.int(), seg[at]
+    seg[sk - 3 * 64:], q_seg[-11:] = -1, -1
+    ids = [x[None].contiguous() for x in (q_pos, q_seg, kv_pos, seg)]
+    g = torch.Generator(device=device).manual_seed(d + group)
+    shapes = [(1, sq, hq, d), (1, sk, hkv, d), (1, sk, hkv, d), (1, sq, hq, d)]
+    q, k, v, dout = (torch.randn(s, generator=g, device=device, dtype=torch.bfloat16) for s in shapes)
+    with attention_specs(SPEC, SPEC):
+        masks = create_attention_mask(*ids, fwd_params=P, bwd_params=P, calc_bwd_mask=True)
+    scale = d ** -0.5
+    out, lse = flash_attention_forward(q, k, v, *ids, masks[0], scale, P, P)
+    dq = flash_attention_backward(q, k, v, *ids, masks[1], masks[2], out, lse, dout, scale, P, P)[0]
+    allowed = (q_seg[:, None] == seg) & (q_seg != -1)[:, None] & (q_pos[:, None] >= kv_pos)
+    for h in {0, hq // 2, hq - 1}:  # float64
+        kt, vt = (t[0, :, h // group].double() for t in (k, v))
+        s = (q[0, :, h].double() @ kt.t().contiguous() * scale).masked_fill_(~allowed, float("-inf"))
+        w = torch.softmax(s, 1).nan_to_num_(0.0)
+        dp = dout[0, :, h].double() @ vt.t().contiguous()
+        check_close("out", out[0, :, h], (w @ vt).cpu().numpy())
+        check_close("dq", dq[0, :, h], (w * (dp - (w * dp).sum(1, keepdim=True)) @ kt * scale).cpu().numpy(), rel=OPERAND_ROUNDING)
+    assert not out[ids[1] == -1].any() and not dq[ids[1] == -1].any()
