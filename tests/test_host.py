@@ -194,7 +194,7 @@ def test_workspace_sizes_follow_the_shapes():
     """The workspace functions are pure functions of the shapes (no GPU needed): 32 bytes per
     64-row tile and batch row for the summaries; the forward adds room for partial results only
     where it runs in its split mode (short query sequences); the backward holds delta, both
-    summaries, the order of the dK/dV work items and the counters of their queues."""
+    summaries, the order of the dK/dV work items, the counters of their queues and the sum and maximum of their work."""
     lib = _native.lib()
     fwd = lambda *s: lib.kvax_fa_fwd_workspace_bytes(ctypes.byref(_fa_args(*s)))
     bwd = lambda *s: lib.kvax_fa_bwd_workspace_bytes(ctypes.byref(_fa_args(*s)))
@@ -221,7 +221,8 @@ def test_workspace_sizes_follow_the_shapes():
     assert lib.kvax_fa_fwd_workspace_bytes(ctypes.byref(wide)) == 32 * 512
     assert fwd(0, 1, 32768, 32, 8, 128) == 0
     delta = 1 * 32 * 32768 * 4
-    order = (2 * 256 + 1 + 8) * 4 + 12      # 256 kv work items, an arrival counter, 8 queue counters; padded to 16
+    # 256 kv work items, an arrival counter, 8 queue counters, the sum and maximum of the items' work; padded to 16
+    order = ((2 * 256 + 1 + 8 + 2) * 4 + 15) // 16 * 16
     assert bwd(1, 32768, 32768, 32, 8, 128) == delta + 2 * 32 * 512 + order
 
 
@@ -330,3 +331,30 @@ def test_backward_workspace_knows_the_value_head_dim():
     q, k, v = (torch.empty((1, n, h, d), device="meta") for n, h, d in ((2048, 8, 192), (128, 1, 192), (128, 1, 128)))
     sizes = [flash_attention_module.backward_workspace_bytes(q, k, *more) for more in ((), (k,), (v,))]
     assert sizes[0] == sizes[1] == sizes[2] + 16 * 128 * (192 - 128) * 4
+
+
+# batch, q_len, kv_len, heads, kv heads, head_dim -> parts of a dK/dV item that the workspace holds: one (none), what the shapes
+# give, or two where the device decides (257 to 512 items of 160 steps or more, a step being a 64-row query tile of a head, at
+# least 16 items a row, one part by the shapes)
+@pytest.mark.parametrize("shape, parts", [
+    ((1, 4096, 4096, 40, 8, 128), 2),          # 256 items of 320 steps: two parts by the shapes
+    ((1, 64 * 40, 128 * 257, 4, 1, 128), 2),   # 257 items of 160 steps
+    ((1, 64 * 159, 128 * 257, 1, 1, 128), 1),  # of 159
+    ((1, 64 * 159 + 1, 128 * 257, 1, 1, 128), 2),
+    ((1, 64 * 160, 128 * 512, 1, 1, 128), 2),  # 512 items
+    ((1, 64 * 160, 128 * 512 + 1, 1, 1, 128), 1),  # 513
+    ((1, 64 * 160, 64 * 512, 1, 1, 256), 2),   # of 64 keys
+    ((1, 64 * 160, 64 * 512 + 1, 1, 1, 256), 1),
+    ((2, 64 * 160, 128 * 16, 16, 16, 64), 2),  # 16 items a row
+    ((2, 64 * 160, 128 * 15, 16, 16, 64), 1),  # 15: no order, 480 items
+    ((1, 64 * 512, 128 * 257, 1, 1, 192), 2),  # of 512 steps: two parts by the shapes
+])
+def test_backward_workspace_of_launches_where_the_device_decides(shape, parts):
+    batch, q_len, kv_len, heads, kv_heads, head_dim = shape
+    items = -(-kv_len // (64 if head_dim > 192 else 128))
+    up = lambda n: -(-n // 16) * 16
+    expected = up(batch * heads * q_len * 4) + sum(32 * batch * -(-n // 64) for n in (q_len, kv_len))
+    expected += up((batch * (2 * items + 1) + 8 + 2) * 4)
+    if parts > 1:
+        expected += parts * batch * kv_len * kv_heads * 2 * head_dim * 4
+    assert _native.lib().kvax_fa_bwd_workspace_bytes(ctypes.byref(_fa_args(*shape))) == expected
