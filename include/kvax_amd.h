@@ -164,8 +164,8 @@ typedef struct kvax_fa_args {
  *   backward: delta [batch, num_heads, q_len] fp32, the tile summaries of the kv and the query
  *             sequence, the order in which the dK/dV kernel takes its work items and the counters of
  *             the queues it takes them from (cleared by the call itself), plus, for launches with few
- *             such items, the fp32 dK and dV of the work-groups that share one (a function of the
- *             shapes only). */
+ *             such items, and for up to 512 of them that may be long, the fp32 dK and dV of the
+ *             work-groups that share one (a function of the shapes only). */
 size_t kvax_fa_fwd_workspace_bytes(const kvax_fa_args* args);
 size_t kvax_fa_bwd_workspace_bytes(const kvax_fa_args* args);
 int kvax_fa_fwd(const kvax_fa_args* args, void* workspace, size_t workspace_bytes,

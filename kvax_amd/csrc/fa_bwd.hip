@@ -126,8 +126,8 @@ __device__ __forceinline__ Vec8 operand(uint4 u) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// dQ: one work-group = NW wavefronts x 32 query rows of one (batch, head); streams the live K/V
-// tiles through a ring of LDS stages filled by asynchronous copies.
+// dQ: one work-group = NW wavefronts x 32 query rows of one (batch, kv head), of one head or the same rows of several
+// heads of the group (see heads_shift); streams the live K/V tiles through a ring of LDS stages filled by asynchronous copies.
 // ---------------------------------------------------------------------------------------------
 template <int D, int DV, int STAGES>
 struct DqSmem {
@@ -510,12 +510,14 @@ inline int dkdv_kv_rows(int head_dim) { return head_dim > 192 ? 64 : 128; }
 
 // Whether two work-groups should share each of 257 to 512 items depends on the documents, so the device decides, from the
 // work the ordering pass has counted: where the longest item is 15 % and 40 steps longer than a compute unit's share of the
-// work.  us of the dK/dV kernel and sum, items whole -> as decided: 8k tokens in documents of 2k, heads 32/8 of 64 512 -> 333,
-// of 128 645 -> 545, of 192 with 128 740 -> 613, 16/4 of 256 (longest item 232 steps, share 178) 734 -> 549; 4 x 4k in documents
-// of 1k, 16/4 of 128, 400 -> 318; 16k in documents of 3k, 8/2 of 256, 1119 -> 737.  Left whole (whole / in two parts): one
-// document of 8k, 16/4 of 256, 1278 / 1327; of 16k, 8/2, 2564 / 2633; without the limit of 40 steps 4k in documents of 1k, 16/16 of
-// 192 with 128, 112 / 181, and 2 x 2k in documents of 300, 16/16 of 128, 75 / 134.  Deciding against it costs 6 us, mostly a sum
-// kernel that finds nothing to add: only where an item can have 160 steps.
+// work.  A step is a live 64-row query tile of one head here and in plan_dkdv_parts (the kernel takes it as two above
+// head_dim 128).  us of the dK/dV kernel and the sum in a training pass, items whole -> as decided: 8k tokens in documents of about 2k,
+// heads 32/8 of 64 531 -> 373, of 128 664 -> 570, of 192 with 128 806 -> 720, 16/4 of 256 (longest item 232 steps, share 178) 803 ->
+// 638; 4 x 4k in documents of 1k, 16/4 of 128, 452 -> 388; 16k in documents of 3k, 8/2 of 256, 1243 -> 878.  Left whole (whole / in
+// two parts, the kernel alone on a faster machine): one document of 8k, 16/4 of 256, 1278 / 1327; of 16k, 8/2, 2564 / 2633; without
+// the limit of 40 steps 4k in documents of 1k, 16/16 of 192 with 128, 112 / 181, and 2 x 2k in documents of 300, 16/16 of 128,
+// 75 / 134.  Deciding against it costs 5 to 6 us of backwards of 100 us (16k in documents of 64, 8/4 of 64) and more, mostly a sum kernel
+// that finds nothing to add: only where an item can have 160 steps.
 // stats: sum and maximum of the items' work (in tiles, the same for every kv head and query head)
 __device__ __forceinline__ bool shares_items(const int32_t* stats, int num_kv_heads, int group) {
   const int64_t longest = (int64_t)stats[1] * group * kNumCus, share = (int64_t)stats[0] * num_kv_heads * group;
@@ -1134,7 +1136,8 @@ __global__ __launch_bounds__(256) void dkdv_sum_kernel(const DkdvSumParams p) {
 //   384 x 384 (6k)                       741 -> 683 (2)
 //   128 x 1024 (16k, heads 4/1)          622 -> 333 (2), 192 (4), 172 (6), 193 (8)
 //   256 x 2048 (32k, heads 4/1)          1179 -> 631 (2), 452 (3)
-// A function of the shapes, so that the workspace can be sized up front (at most 768 parts of 128 rows).
+// A function of the shapes, so that the workspace can be sized up front (at most 768 parts of 128 rows;
+// up to 1024 where the device decides, see device_decides_parts).
 int plan_dkdv_parts(int batch, int q_len, int kv_len, int num_heads, int num_kv_heads, int head_dim) {
   if (batch <= 0 || q_len <= 0 || kv_len <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return 1;
   const int64_t items = (int64_t)batch * num_kv_heads * cdiv(kv_len, dkdv_kv_rows(head_dim));

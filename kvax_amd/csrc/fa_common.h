@@ -127,8 +127,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // Work distribution.  Work-groups are dealt round-robin to the 8 XCDs (work-group L runs on XCD
 // L % 8, each XCD has its own L2), so the map from L to a work item decides both L2 sharing and
 // balance.  Items are (group, tile rank, member): a group is one (batch, kv head) -- everything
-// that reads the same K/V -- with `tiles` tiles ranked heaviest first and `members` query heads
-// per tile.  With at least 8 groups each XCD owns whole groups (visited in an order that rotates
+// that reads the same K/V -- with `tiles` tiles ranked heaviest first and `members` work-groups
+// per tile (forward and dQ: the query heads of the group, or the sets of them that a work-group takes, see
+// heads_shift; dK/dV: the parts of an item).  With at least 8 groups each XCD owns whole groups (visited in an order that rotates
 // from rank to rank, see decode()); with fewer (and 8 divisible by
 // the count) the tiles of a group are dealt round-robin to the XCDs that share it, so that every
 // XCD gets the same mix of heavy and light tiles; otherwise items are cut into 8 contiguous runs.
@@ -181,9 +182,11 @@ struct ItemMap {
 // (2^shift of them, where they divide the group), and 32-row blocks of the same heads for the rest.  The heads share the
 // key tiles and the mask, so with a head per wavefront all of them have the same live tiles and none waits at the
 // barrier of a tile that is live for others only, as with 128 rows of one head (us, 128 rows of one head -> this): 4 x 16k tokens
-// in bidirectional documents of 512, heads 64/8, forward 2404 -> 2296, dQ 3168 -> 3032; 32k in causal ones of 2k, 32/8,
-// 1154 -> 1135, 1554 -> 1531; 2 x 8k in blocks of 64, documents of 300, 189 -> 174, 259 -> 235; 8 x 1k, 101 -> 95, 144 -> 131.
-// Nothing on one long document or with one head per group.
+// in bidirectional documents of 512, heads 64/8 of 128, forward 2433 -> 2304, dQ 3191 -> 3037; 32k in causal ones of 2k, 32/8,
+// 1210 -> 1179, 1613 -> 1573; forward of 2 x 8k in documents of 100, 300 and 512 136 -> 124, 157 -> 143, 160 -> 150, 32/4 of 192 with
+// 128 in ones of 200 203 -> 163, 64 x 160 tokens, 32/4, 96 -> 69.  (In a whole step less is left, 1.0 % of the 32k one and 2.8 % of
+// the 4 x 16k one: the dK/dV behind it, the same code, runs up to 2 % slower at the power limit.)
+// Nothing on one long document or with one head per group; one row of 8k in documents of exactly 128 is slower, 54.7 -> 57.4.
 // At head_dim 256 it does not pay: the forward spills 2 registers more (8k tokens, heads 16/4: 236 -> 253 us), dQ
 // is equal on documents and 1.4 % slower on one long one.
 template <int D>

@@ -87,8 +87,9 @@ struct FwdSmem {
   static constexpr int kTotal = STAGES * kStage;
 };
 
-// One work-group: NW wavefronts x (32 * MQ) query rows of one (batch, head); streams the live kv
-// tiles through a STAGES-deep ring of LDS stages filled by asynchronous copies.
+// One work-group: NW wavefronts x (32 * MQ) rows of one (batch, kv head) - query rows of one head, or the same query rows
+// of several heads of the group (see heads_shift); streams the live kv tiles through a STAGES-deep ring of LDS stages filled
+// by asynchronous copies.
 //
 // SPLIT (short query sequences, e.g. decoding one token against a long key sequence, where one
 // work-group per (batch, head) would leave most of the chip idle and read the keys serially): the
