@@ -40,18 +40,15 @@ struct WithoutGil {
   ~WithoutGil() { PyEval_RestoreThread(state); }
 };
 
+// The type of the mode behind torch.set_default_device(), looked up in bind(): an import may hand the interpreter lock to
+// another thread, which must not then wait here for the import to end.
+PyObject* device_context;
+
 // Whether a mode that overrides torch functions is active (TorchFunctionMode): it has to see the allocations of a call.
 // The one behind torch.set_default_device() and `with torch.device(...)` is passed over: it changes calls that name no
 // device, and those of the Python code name theirs.
 bool functions_overridden() {
   if (!at::impl::torch_function_mode_enabled()) return false;
-  static PyObject* const device_context = [] {
-    PyObject* module = PyImport_ImportModule("torch.utils._device");
-    PyObject* type = module ? PyObject_GetAttrString(module, "DeviceContext") : nullptr;
-    Py_XDECREF(module);
-    PyErr_Clear();
-    return type;
-  }();
   for (int64_t i = 0; i < at::impl::PythonTorchFunctionTLS::stack_len(); i++) {
     const auto& mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i);
     if ((PyObject*)Py_TYPE(mode->ptr(&mode->pyinterpreter())) != device_context) return true;
@@ -169,6 +166,10 @@ PyObject* bind(PyObject*, PyObject* const* o, Py_ssize_t n) {
                         KVAX_ABI_VERSION, (int)sizeof(kvax_fa_args), (int)sizeof(kvax_mask_desc), version, args, desc);
   if (strcmp(torch, KVAX_TORCH_VERSION) != 0)
     return PyErr_Format(PyExc_ImportError, "built for torch " KVAX_TORCH_VERSION ", not %s", torch);
+  PyObject* module = PyImport_ImportModule("torch.utils._device");
+  device_context = module ? PyObject_GetAttrString(module, "DeviceContext") : nullptr;
+  Py_XDECREF(module);
+  PyErr_Clear();
   void* p[6];
   for (int i = 0; i < 6; i++)
     if (!(p[i] = PyLong_AsVoidPtr(o[4 + i]))) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "null address");
